@@ -106,8 +106,6 @@ struct Dev {
   void* cross = nullptr;    // cross-term factors T
   void* snap = nullptr;     // 'fixed' values of the evolving fields
   double* dx[3] = {nullptr, nullptr, nullptr};
-  int* bc_e = nullptr;      // [ne][6]
-  int* bc_b = nullptr;      // [nbg][6]
   unsigned long long* red = nullptr;  // [kSlots+1][kRedSlots]
   bool red_valid[kSlots] = {false, false, false, false};
   std::vector<double> stage;  // host staging
@@ -183,12 +181,20 @@ void t_collect(Dev& d) {
   d.timed.clear();
 }
 
+// the boundary codes of a ghost fill as kernel arguments (4 bits each)
+void set_codes(sac::GhostArgs& a, const std::vector<int>& codes) {
+  for (size_t v = 0; v < codes.size() / 6; v++) {
+    a.bc[v] = 0;
+    for (int iB = 0; iB < 6; iB++) a.bc[v] |= (unsigned)codes[v * 6 + iB] << (4 * iB);
+  }
+}
+
 void ghost_fill_evolving(Dev& d, int slot) {
   sac::GhostArgs a{};
   a.g = d.g;
   a.prec = d.prec;
   a.f = d.reg[slot];
-  a.bc = d.bc_e;
+  set_codes(a, d.bce_h);
   a.nvar = d.ne;
   a.snap = d.initialized ? d.snap : nullptr;
   a.keep_fixed = (!d.initialized && d.fullgridini) ? 1 : 0;
@@ -609,11 +615,6 @@ int sac_dev_init(int ndim, int ndir, const int* nx, int nw, const int* iws, int 
         d->ext1_b |= x1;
       }
     }
-  if (hipMalloc((void**)&d->bc_e, sizeof(int) * bce.size()) != hipSuccess ||
-      hipMalloc((void**)&d->bc_b, sizeof(int) * bcb.size()) != hipSuccess)
-    return bail(fail(SAC_E_NOMEM, "bc alloc"));
-  hipMemcpy(d->bc_e, bce.data(), sizeof(int) * bce.size(), hipMemcpyHostToDevice);
-  hipMemcpy(d->bc_b, bcb.data(), sizeof(int) * bcb.size(), hipMemcpyHostToDevice);
   if (hipMalloc((void**)&d->red, sizeof(unsigned long long) * (kSlots + 1) * sac::kRedSlots) !=
       hipSuccess)
     return bail(fail(SAC_E_NOMEM, "reduction buffer"));
@@ -645,8 +646,6 @@ int sac_dev_free(sac_handle h) {
   hipFree(d->J);
   hipFree(d->snap);
   for (int k = 0; k < 3; k++) hipFree(d->dx[k]);
-  hipFree(d->bc_e);
-  hipFree(d->bc_b);
   hipFree(d->red);
   if (d->cl) {
     Closure* c = d->cl;
@@ -798,7 +797,7 @@ int sac_dev_getboundary(sac_handle h) {
     a.g = d.g;
     a.prec = sac::PREC_FP64;
     a.f = d.bg;
-    a.bc = d.bc_b;
+    set_codes(a, d.bcb_h);
     a.nvar = d.nbg;
     a.snap = nullptr;
     a.keep_fixed = d.fullgridini ? 1 : 0;
@@ -817,7 +816,7 @@ int sac_dev_getboundary(sac_handle h) {
       st.g = d.g;
       st.prec = d.prec;
       st.f = d.reg[SAC_SLOT_W];
-      st.bc = d.bc_e;
+      set_codes(st, d.bce_h);
       st.nvar = d.ne;
       sac::launch_ghost_store(st, d.snap, d.stream);
     }

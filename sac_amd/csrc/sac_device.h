@@ -915,6 +915,12 @@ __device__ __forceinline__ void final_cell(const FinalArgs& a, const GridDesc& g
 // the stored value of a 'fixed' region), which is what every thread does
 // here; no thread reads a ghost cell, so the kernel is race-free.
 
+// boundary code of variable var in region iB = 2*axis + side (the codes are
+// kernel arguments, so a fill waits for no table in memory)
+__device__ __forceinline__ int ghost_code(const GhostArgs& a, int var, int iB) {
+  return (int)((a.bc[var] >> (4 * iB)) & 15u);
+}
+
 // Value of ghost cell c of variable var after the reference's sequential
 // region fills (src/vacgrid.t:195-512): the region of the highest axis along
 // which c is a ghost writes last, and its sources lie in the mesh along that
@@ -935,7 +941,7 @@ __device__ double ghost_eval(const GhostArgs& a, int var, int c0, int c1, int c2
     const S* snap = (const S*)a.snap;
     const long long i = vo + lin(g, c[0], c[1], c[2]);
     const int side = (c[D] > g.Mhi[D]) ? 1 : 0;
-    const int code = a.bc[var * 6 + 2 * D + side];
+    const int code = ghost_code(a, var, 2 * D + side);
     const int N = g.Mhi[D] - g.Mlo[D] + 1;
     const int ixe = side ? g.Mhi[D] : g.Mlo[D];  // edge cell
     auto at = [&](int cd) {
@@ -996,7 +1002,7 @@ __device__ __forceinline__ S ghost_value(const GhostArgs& a, int var, int c0, in
     const long long i = vo + lin(g, c[0], c[1], c[2]);
     if (d < 0) break;
     const int side = (c[d] > g.Mhi[d]) ? 1 : 0;
-    const int code = a.bc[var * 6 + 2 * d + side];
+    const int code = ghost_code(a, var, 2 * d + side);
     const int N = g.Mhi[d] - g.Mlo[d] + 1;
     const int ixe = side ? g.Mhi[d] : g.Mlo[d];
     const bool stored = code == BC_FIXED || code == BC_FIXED1 || code == BC_GRAD1;
@@ -1045,7 +1051,7 @@ __device__ __forceinline__ S ghost_stored(const GhostArgs& a, int var, int c0, i
     if (d < 0 && dd < g.ndim && (c[dd] < g.Mlo[dd] || c[dd] > g.Mhi[dd])) d = dd;
   if (d < 0) return (S)0;
   const int side = (c[d] > g.Mhi[d]) ? 1 : 0;
-  const int code = a.bc[var * 6 + 2 * d + side];
+  const int code = ghost_code(a, var, 2 * d + side);
   const S v = f[vo + lin(g, c[0], c[1], c[2])];
   if (code == BC_FIXED || code == BC_FIXED1) return v;
   if (code == BC_GRAD1) {

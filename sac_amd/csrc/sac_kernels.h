@@ -65,7 +65,7 @@ struct GhostArgs {
   int prec;            // storage type of f and snap
   void* f;             // nvar fields to fill in place
   const void* snap;    // stored 'fixed' values (null before they exist)
-  const int* bc;       // [nvar][6] boundary codes
+  unsigned bc[kMaxEvolve];  // boundary codes per variable, 4 bits per region (ghost_code)
   int nvar;
   int keep_fixed;      // initial fill with fullgridini: keep file values
   int general;         // some fill has two sources (cont1; fixed1/grad1 before storage)
