@@ -285,7 +285,11 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
     sac::launch_plane(x, d.stream);
     t_end(d, SAC_K_PLANE, e0);
   }
-  for (int k = plane ? 2 : 0; k < d.ndim; k++) {
+  // 1-D FP64: the whole stage in one launch (below), unless the resistive
+  // sources have to join the rate first
+  const bool stage1 = d.ndim == 1 && d.prec == SAC_PREC_FP64 && !learned && !(d.eta > 0.0) &&
+                      sac::line_tiles_built();
+  for (int k = plane ? 2 : 0; k < d.ndim && !stage1; k++) {
     // axis 1 (rows of a plane): neighbour rows in one XCD's L2.  Axes 0 and 2
     // keep the hardware order, whose round-robin already places the
     // neighbour planes of a row in the same XCD.
@@ -348,7 +352,10 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   s.skip_xy = plane ? 1 : 0;
   hipEvent_t e0{};
   t_begin(d, SAC_K_FINAL, &e0);
-  sac::launch_final(s, d.stream);
+  if (stage1)
+    sac::launch_stage1(s, x.ctot_src, x.red_visc, d.stream);
+  else
+    sac::launch_final(s, d.stream);
   t_end(d, SAC_K_FINAL, e0);
   d.red_valid[out] = true;
   if (d.any_zero)

@@ -249,11 +249,12 @@ __global__ void __launch_bounds__(256) kb_final(Args a, int wct, int base, int o
 }
 
 // Tubes: one whole RK stage of a tile of LT cells in one kernel: the x work
-// as an LDS line tile (line1_tile, sac_device.h, also the x kernel of 1-D
-// FP64 grids), then the combining update of the tile's cells (final_cell;
-// the thread that stored R of its cell reads it back, so no other block is
-// waited for) with the 'cont' ghosts.  The reductions of `out` must have
-// been cleared by kb_zero_red.
+// as an LDS line tile (line1_tile, sac_device.h, also used by 1-D FP64
+// grids), then the update of the thread's cell from the rate in its
+// registers, with the 'cont' ghosts.  With R stored and read back a
+// stage of 4.5 M cells took 0.383 ms (0.478 ms RK4's last), now 0.314 (0.388);
+// 232 B per cell without R, 3.3 TB/s: latency of two waits per block.
+// The reductions of `out` must have been cleared by kb_zero_red.
 template <int LT, bool RK4L>
 __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, int out, double da) {
   __shared__ double L[line1::LV<NDIR> * (LT + 6)];
@@ -261,10 +262,6 @@ __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, i
   if (a.state[tl.tube] != RUNNING) return;  // uniform over the block
   const GridDesc g = tube_grid<1>(a, tl.tube);
   const long long o = a.start[tl.tube];
-  double numax = 0.0;
-  line1_tile<LT, NDIR>(g, a.reg[wct] + o, a.bg + o, a.dx + a.dxo[tl.tube], a.R + o, a.gamma,
-                       a.visc_on, red_get(red_of(a, tl.tube, wct), 0), tl.c0, L, numax);
-  __syncthreads();  // orders each thread's R stores before its loads below
   const double dt = a.dt[tl.tube];
   FinalArgs f{};
   f.g = g;
@@ -272,19 +269,17 @@ __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, i
   f.wct = a.reg[wct] + o;
   f.bg = a.bg + o;
   f.dx[0] = a.dx + a.dxo[tl.tube];
-  f.R = a.R + o;
   f.base = a.reg[base] + o;
   f.out = a.reg[out] + o;
   set_rk4<RK4L>(a, o, f);
   f.qa = dt / da;
   f.gamma = a.gamma;
   f.visc_on = a.visc_on;
-  double redv[2] = {0.0, 0.0};
-  int c[3] = {tl.c0 + (int)threadIdx.x, 0, 0};
-  if (c[0] <= g.Mhi[0]) {
-    final_cell<1, NDIR, double, double, RK4L>(f, g, c, redv);
+  double numax = 0.0, redv[2] = {0.0, 0.0};
+  const double ctk = red_get(red_of(a, tl.tube, wct), 0);
+  const int c[3] = {tl.c0 + (int)threadIdx.x, 0, 0};
+  if (line1_stage<LT, NDIR, RK4L>(f, g, ctk, tl.c0, L, numax, redv))
     cont_ghosts_of<1>(g, (double*)f.out, c);
-  }
   if (a.visc_on) {
     double r[1] = {numax};
     block_max_atomic<1>(r, a.visc + tl.tube);

@@ -562,8 +562,8 @@ __device__ __forceinline__ void axis_group(const AxisArgs& a, const GridDesc& g,
 // averages, and setnu's q for rho', the thermal energy and v_x.  Each
 // thread then assembles its cell from its neighbours' values with the
 // expressions of axis_group<1, NDIR, 0, 1> in the same order, but with each
-// stencil point evaluated once instead of up to seven times.  R is stored
-// for the mesh cells of the tile; numax gets the thread's largest nu.
+// stencil point evaluated once instead of up to seven times.  R gets the rate
+// of the thread's cell c0 + threadIdx.x; numax its largest nu.
 namespace line1 {
 // values per point: F[NE], v, pTb, bg, rho_t, m, q[3]
 template <int NDIR>
@@ -574,7 +574,7 @@ template <int LT, int NDIR>
 __device__ __forceinline__ void line1_tile(const GridDesc& g, const double* __restrict__ W,
                                            const double* __restrict__ B,
                                            const double* __restrict__ dx,
-                                           double* __restrict__ Rout, double gamma, int visc_on,
+                                           double (&R)[2 + 2 * NDIR], double gamma, int visc_on,
                                            double ctk, int c0, double* __restrict__ L,
                                            double& numax) {
   constexpr int NE = 2 + 2 * NDIR, LP = LT + 6;
@@ -619,7 +619,6 @@ __device__ __forceinline__ void line1_tile(const GridDesc& g, const double* __re
   const bool z1 = (c == MloK && !g.per_lo[0]) || (c == MhiK && !g.per_hi[0]);
   const double dxd = dx[valid ? c : MhiK];
   const double dxk = dxd, idx = 1.0 / dxd;
-  double R[NE];
   {
     const double pTb0 = at(NE + 1, k), bgk = at(NE + 2, k), bgl = bgk;
     const double inv12 = idx / 12.0;
@@ -674,10 +673,6 @@ __device__ __forceinline__ void line1_tile(const GridDesc& g, const double* __re
       }
     }
   }
-  if (valid) {
-#pragma unroll
-    for (int n = 0; n < NE; n++) Rout[n * fs + c] = R[n];
-  }
 }
 
 // ---------------------------------------------------------------------
@@ -698,23 +693,16 @@ __device__ __forceinline__ void line1_tile(const GridDesc& g, const double* __re
 // of neighbouring cells (FP32 storage: 4 bytes apart) can be issued as one
 // wider load; the arithmetic of every cell is that of V = 1.  RK4L: RK4's
 // last stage (a.w1, a.w2 set; w3 is the stage input a.wct).
-template <int NDIM, int NDIR, typename S, typename C, int V, bool RK4L>
-__device__ __forceinline__ void final_cells(const FinalArgs& a, const GridDesc& g,
-                                            const int (&c)[3], int nv,
-                                            double (&redv)[2 * NDIM]) {
-  constexpr int NE = 2 + 2 * NDIR;
+// The parts take the rate R in registers: the combining kernel reads it from
+// memory (final_cells), the kernels that hold a cell's whole rate pass it on.
+
+// gravity on the perturbed density (addsource_grav, src/vacusr.gravity.t:46-78)
+template <int NDIM, int NDIR, typename S, typename C, int V>
+__device__ __forceinline__ void gravity_cells(const FinalArgs& a, const GridDesc& g, long long ic0,
+                                              C (&R)[V][2 + 2 * NDIR]) {
   const long long fs = g.fs;
   const S* __restrict__ W = (const S*)a.wct;
-  const S* __restrict__ RR = (const S*)a.R;
-  const S* __restrict__ TT = (const S*)a.T;
   const double* __restrict__ B = a.bg;
-  const long long ic0 = lin(g, c[0], c[1], c[2]);
-  C R[V][NE];
-#pragma unroll
-  for (int n = 0; n < NE; n++)
-#pragma unroll
-    for (int j = 0; j < V; j++) R[j][n] = (C)RR[n * fs + ic0 + j];
-  // gravity on the perturbed density (addsource_grav, src/vacusr.gravity.t:46-78)
   {
     // loads first, then selects (no branch between the loads)
     C rho[V], inv[V], md[V][NDIM];
@@ -739,6 +727,17 @@ __device__ __forceinline__ void final_cells(const FinalArgs& a, const GridDesc& 
       R[j][1 + NDIR] += rg;
     }
   }
+}
+
+// the cross-term derivatives along the axes that the line kernels left out
+template <int NDIM, int NDIR, typename S, typename C, int V>
+__device__ __forceinline__ void cross_cells(const FinalArgs& a, const GridDesc& g,
+                                            const int (&c)[3], long long ic0,
+                                            C (&R)[V][2 + 2 * NDIR]) {
+  const long long fs = g.fs;
+  const S* __restrict__ W = (const S*)a.wct;
+  const S* __restrict__ TT = (const S*)a.T;
+  const double* __restrict__ B = a.bg;
   if (a.visc_on && NDIM > 1) {
     // Branch-free, so that every load of the cell can be issued at once: the
     // neighbours c +- e_l of a mesh cell are in the grid; T outside the mesh
@@ -803,9 +802,21 @@ __device__ __forceinline__ void final_cells(const FinalArgs& a, const GridDesc& 
       }
     }
   }
-  // register update and cmax of the (stored) result.  out may be base (the
-  // in-place stages): each element is read by the thread that writes it,
-  // before it writes it, so the two pointers carry no no-alias promise.
+}
+
+// register update and cmax of the (stored) result
+template <int NDIM, int NDIR, typename S, typename C, int V, bool RK4L>
+__device__ __forceinline__ void update_cells(const FinalArgs& a, const GridDesc& g,
+                                             const int (&c)[3], long long ic0, int nv,
+                                             const C (&R)[V][2 + 2 * NDIR],
+                                             double (&redv)[2 * NDIM]) {
+  constexpr int NE = 2 + 2 * NDIR;
+  const long long fs = g.fs;
+  const S* __restrict__ W = (const S*)a.wct;
+  const double* __restrict__ B = a.bg;
+  // out may be base (the in-place stages): each element is read by the thread
+  // that writes it, before it writes it, so the two pointers carry no no-alias
+  // promise.
   S* out = (S*)a.out;
   const S* base = (const S*)a.base;
   S o[V][NE];
@@ -898,12 +909,47 @@ __device__ __forceinline__ void final_cells(const FinalArgs& a, const GridDesc& 
   }
 }
 
+template <int NDIM, int NDIR, typename S, typename C, int V, bool RK4L>
+__device__ __forceinline__ void final_cells(const FinalArgs& a, const GridDesc& g,
+                                            const int (&c)[3], int nv,
+                                            double (&redv)[2 * NDIM]) {
+  constexpr int NE = 2 + 2 * NDIR;
+  const S* __restrict__ RR = (const S*)a.R;
+  const long long ic0 = lin(g, c[0], c[1], c[2]);
+  C R[V][NE];
+#pragma unroll
+  for (int n = 0; n < NE; n++)
+#pragma unroll
+    for (int j = 0; j < V; j++) R[j][n] = (C)RR[n * g.fs + ic0 + j];
+  gravity_cells<NDIM, NDIR, S, C, V>(a, g, ic0, R);
+  cross_cells<NDIM, NDIR, S, C, V>(a, g, c, ic0, R);
+  update_cells<NDIM, NDIR, S, C, V, RK4L>(a, g, c, ic0, nv, R, redv);
+}
+
 // One mesh cell c of the grid g; the cmax values of the result go to redv.
 // RK4L: RK4's last stage (a.w1, a.w2 set; w3 is the stage input a.wct).
 template <int NDIM, int NDIR, typename S, typename C, bool RK4L>
 __device__ __forceinline__ void final_cell(const FinalArgs& a, const GridDesc& g, const int (&c)[3],
                                            double (&redv)[2 * NDIM]) {
   final_cells<NDIM, NDIR, S, C, 1, RK4L>(a, g, c, 1, redv);
+}
+
+// 1-D grids in FP64: a whole RK stage of the tile of LT cells from c0 on: the
+// x work (line1_tile), then gravity and the update of the thread's cell from
+// the rate in registers (1-D has no cross terms, so nothing waits for other
+// blocks); true if the thread stored a cell.
+template <int LT, int NDIR, bool RK4L>
+__device__ __forceinline__ bool line1_stage(const FinalArgs& f, const GridDesc& g, double ctk,
+                                            int c0, double* __restrict__ L, double& numax,
+                                            double (&redv)[2]) {
+  double R[1][2 + 2 * NDIR];
+  line1_tile<LT, NDIR>(g, (const double*)f.wct, f.bg, f.dx[0], R[0], f.gamma, f.visc_on, ctk, c0, L,
+                       numax);
+  const int c[3] = {c0 + (int)threadIdx.x, 0, 0};
+  if (c[0] > g.Mhi[0]) return false;
+  gravity_cells<1, NDIR, double, double, 1>(f, g, c[0], R);
+  update_cells<1, NDIR, double, double, 1, RK4L>(f, g, c, c[0], 1, R, redv);
+  return true;
 }
 
 // ---------------------------------------------------------------------

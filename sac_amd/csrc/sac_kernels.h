@@ -113,6 +113,9 @@ int line_tiles_built();
 // the x-y cross terms included; R is written fresh
 void launch_plane(const AxisArgs& a, hipStream_t st);
 void launch_final(const FinalArgs& a, hipStream_t st);
+// a whole stage of a 1-D FP64 grid (x work and update) in one launch
+void launch_stage1(const FinalArgs& a, const unsigned long long* ctot_src,
+                   unsigned long long* red_visc, hipStream_t st);
 void launch_cmax(const CmaxArgs& a, hipStream_t st);
 void launch_ghost(const GhostArgs& a, hipStream_t st);
 // stored ghost values of the fixed/fixed1/grad1 boundaries of a.f (after a fill)

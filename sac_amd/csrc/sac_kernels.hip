@@ -96,18 +96,42 @@ __global__ void __launch_bounds__(plane::NT) k_plane(AxisArgs a) {
   }
 }
 
-// kernel 1, 1-D grids in FP64: LDS line tiles of 256 cells (line1_tile)
+// kernel 1, 1-D grids in FP64 whose rate gets further terms before the
+// update (resistivity): LDS line tiles of 256 cells (line1_tile), R to memory
 template <int NDIR>
 __global__ void __launch_bounds__(256) k_line1(AxisArgs a) {
   __shared__ double L[line1::LV<NDIR> * (256 + 6)];
   double numax = 0.0;
-  line1_tile<256, NDIR>(a.g, (const double*)a.wct, a.bg, a.dx[0], (double*)a.R, a.gamma, a.visc_on,
-                  a.visc_on ? red_get(a.ctot_src, 0) : 0.0, a.g.Mlo[0] + 256 * (int)blockIdx.x, L,
-                  numax);
+  double R[2 + 2 * NDIR];
+  const int c0 = a.g.Mlo[0] + 256 * (int)blockIdx.x, c = c0 + (int)threadIdx.x;
+  line1_tile<256, NDIR>(a.g, (const double*)a.wct, a.bg, a.dx[0], R, a.gamma, a.visc_on,
+                        a.visc_on ? red_get(a.ctot_src, 0) : 0.0, c0, L, numax);
+  if (c <= a.g.Mhi[0]) {
+#pragma unroll
+    for (int n = 0; n < 2 + 2 * NDIR; n++) ((double*)a.R)[n * a.g.fs + c] = R[n];
+  }
   if (a.visc_on) {
     double r2[1] = {numax};
     block_max_atomic<1>(r2, a.red_visc);
   }
+}
+
+// 1-D grids in FP64: a whole RK stage per launch, LT cells per block, the
+// rate in registers (line1_stage).  With R through
+// memory a stage was two launches: 5.2 + 5.2 us at 800 cells, 8.2 + 8.5 us at
+// 60001 cells of three components; now 6.6 and 10.8 us.
+template <int LT, int NDIR, bool RK4L>
+__global__ void __launch_bounds__(LT) k_stage1(FinalArgs a, const unsigned long long* ctot_src,
+                                               unsigned long long* red_visc) {
+  __shared__ double L[line1::LV<NDIR> * (LT + 6)];
+  double numax = 0.0, redv[2] = {0.0, 0.0};
+  line1_stage<LT, NDIR, RK4L>(a, a.g, a.visc_on ? red_get(ctot_src, 0) : 0.0,
+                              a.g.Mlo[0] + LT * (int)blockIdx.x, L, numax, redv);
+  if (a.visc_on) {
+    double r2[1] = {numax};
+    block_max_atomic<1>(r2, red_visc);
+  }
+  block_max_atomic<2>(redv, a.red_out);
 }
 
 // segment length along K: whole lines unless that leaves fewer than 2048
@@ -514,6 +538,32 @@ int launch_axis(const AxisArgs& a, int axis, hipStream_t st) {
   dispatch(a.prec, g.ndim, g.ndir, 0, axis, &a, st, n);
   const bool line = SAC_LINE_TILES && g.ndim > 1;
   return (line && a.cross_last && a.visc_on && axis == g.ndim - 1) ? 1 : 0;
+}
+
+// Tile length of k_stage1: 64 cells for short grids, which spread over four
+// times as many CUs then (6.6 us a stage at 800 cells), else 256: every block adds its
+// maxima to the same words, and 938 blocks of 64 cells queued there (18.5 us a
+// stage at 60001 cells).
+template <int NDIR>
+static void launch_stage1_nd(const FinalArgs& a, const unsigned long long* ctot_src,
+                             unsigned long long* red_visc, hipStream_t st) {
+  const int n = a.g.Mhi[0] - a.g.Mlo[0] + 1;
+  const int LT = n > 4096 ? 256 : 64;
+  const dim3 nb((unsigned)((n + LT - 1) / LT)), bs(LT);
+  if (LT == 256) {
+    if (a.w1) hipLaunchKernelGGL((k_stage1<256, NDIR, true>), nb, bs, 0, st, a, ctot_src, red_visc);
+    else hipLaunchKernelGGL((k_stage1<256, NDIR, false>), nb, bs, 0, st, a, ctot_src, red_visc);
+  } else {
+    if (a.w1) hipLaunchKernelGGL((k_stage1<64, NDIR, true>), nb, bs, 0, st, a, ctot_src, red_visc);
+    else hipLaunchKernelGGL((k_stage1<64, NDIR, false>), nb, bs, 0, st, a, ctot_src, red_visc);
+  }
+}
+
+void launch_stage1(const FinalArgs& a, const unsigned long long* ctot_src,
+                   unsigned long long* red_visc, hipStream_t st) {
+  if (a.g.ndir == 1) launch_stage1_nd<1>(a, ctot_src, red_visc, st);
+  else if (a.g.ndir == 2) launch_stage1_nd<2>(a, ctot_src, red_visc, st);
+  else launch_stage1_nd<3>(a, ctot_src, red_visc, st);
 }
 
 void launch_plane(const AxisArgs& a, hipStream_t st) {
