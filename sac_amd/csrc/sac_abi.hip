@@ -106,7 +106,15 @@ struct Dev {
   void* cross = nullptr;    // cross-term factors T
   void* snap = nullptr;     // 'fixed' values of the evolving fields
   double* dx[3] = {nullptr, nullptr, nullptr};
-  unsigned long long* red = nullptr;  // [kSlots+1][kRedSlots]
+  unsigned long long* red = nullptr;  // [kSlots+1][kRedSlots], then the reduction lines
+  // the words of W and maxviscoef in pinned host memory, written by the
+  // kernel that combines them at the end of a stage into W; posted: they are
+  // those of the device (once the stream is idle)
+  unsigned long long* red_host = nullptr;
+  bool posted = false;
+  // getdt_special took maxviscoef: it counts as 0 until the next stage, whose
+  // combine overwrites it
+  bool visc_taken = false;
   bool red_valid[kSlots] = {false, false, false, false};
   std::vector<double> stage;  // host staging
   long long bytes = 0;
@@ -149,6 +157,22 @@ int ealloc(Dev& d, void** p, long long nelem) { return balloc(d, p, d.esz * (siz
 
 unsigned long long* red_of(Dev& d, int slot) { return d.red + (size_t)slot * sac::kRedSlots; }
 unsigned long long* red_visc(Dev& d) { return d.red + (size_t)kSlots * sac::kRedSlots; }
+unsigned long long* red_acc(Dev& d) { return d.red + (size_t)(kSlots + 1) * sac::kRedSlots; }
+constexpr size_t kRedBytes = sizeof(unsigned long long) *
+                             ((kSlots + 1) * sac::kRedSlots + sac::kRedLines * sac::kRedWords);
+
+// the combine of a stage into register `out`
+sac::RedCombine stage_combine(Dev& d, int out) {
+  sac::RedCombine c{};
+  c.acc = red_acc(d);
+  c.red = red_of(d, out);
+  c.visc = red_visc(d);
+  c.visc_keep = d.visc_taken ? 0 : 1;
+  d.visc_taken = false;
+  c.host = (out == SAC_SLOT_W) ? d.red_host : nullptr;
+  d.posted = out == SAC_SLOT_W;
+  return c;
+}
 
 // event helpers
 void t_begin(Dev& d, int k, hipEvent_t* a) {
@@ -189,8 +213,9 @@ void set_codes(sac::GhostArgs& a, const std::vector<int>& codes) {
   }
 }
 
-void ghost_fill_evolving(Dev& d, int slot) {
+void ghost_fill_evolving(Dev& d, int slot, const sac::RedCombine& combine = sac::RedCombine{}) {
   sac::GhostArgs a{};
+  a.combine = combine;
   a.g = d.g;
   a.prec = d.prec;
   a.f = d.reg[slot];
@@ -234,10 +259,10 @@ void ghost_fill_sequential(Dev& d, int slot, bool fill_bg) {
     }
   }
   d.red_valid[slot] = false;
+  if (slot == SAC_SLOT_W) d.posted = false;
 }
 
 void cmax_reduce(Dev& d, int slot) {
-  sac::launch_zero_u64(red_of(d, slot), sac::kRedSlots, d.stream);
   sac::CmaxArgs a{};
   a.g = d.g;
   a.prec = d.prec;
@@ -245,11 +270,17 @@ void cmax_reduce(Dev& d, int slot) {
   a.bg = d.bg;
   for (int k = 0; k < 3; k++) a.dx[k] = d.dx[k];
   a.gamma = d.gamma;
-  a.red_out = red_of(d, slot);
+  a.red_out = red_acc(d);
+  a.lines = sac::kRedLines;
   hipEvent_t e0{};
   t_begin(d, SAC_K_CMAX, &e0);
   sac::launch_cmax(a, d.stream);
   t_end(d, SAC_K_CMAX, e0);
+  sac::RedCombine c{};
+  c.acc = red_acc(d);
+  c.red = red_of(d, slot);
+  sac::launch_combine(c, d.stream);
+  if (slot == SAC_SLOT_W) d.posted = false;
   d.red_valid[slot] = true;
 }
 
@@ -269,7 +300,7 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   x.gamma = d.gamma;
   x.visc_on = d.visc_on;
   x.ctot_src = red_of(d, wct);
-  x.red_visc = red_visc(d);
+  x.acc = red_acc(d);
   const bool learned = d.cl && d.cl->on;
   int skip_last = 0;
   // plane tiles: the x and y work (and their cross terms) in one launch,
@@ -324,7 +355,6 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
     ra.compact = d.compactres;
     sac::launch_resistive(ra, d.stream);
   }
-  sac::launch_zero_u64(red_of(d, out), sac::kRedSlots, d.stream);
   sac::FinalArgs s{};
   s.g = d.g;
   s.prec = d.prec;
@@ -346,22 +376,26 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
     s.grav_on[k] = d.grav_on[k];
   }
   s.visc_on = d.visc_on;
-  s.red_out = red_of(d, out);
+  s.acc = red_acc(d);
+  s.ctot_src = x.ctot_src;
   s.xcd = 1;
   s.skip_last = skip_last;
   s.skip_xy = plane ? 1 : 0;
   hipEvent_t e0{};
   t_begin(d, SAC_K_FINAL, &e0);
   if (stage1)
-    sac::launch_stage1(s, x.ctot_src, x.red_visc, d.stream);
+    sac::launch_stage1(s, d.stream);
   else
     sac::launch_final(s, d.stream);
   t_end(d, SAC_K_FINAL, e0);
   d.red_valid[out] = true;
-  if (d.any_zero)
+  const sac::RedCombine combine = stage_combine(d, out);
+  if (d.any_zero) {
+    sac::launch_combine(combine, d.stream);
     ghost_fill_sequential(d, out, false);
-  else
-    ghost_fill_evolving(d, out);
+  } else {
+    ghost_fill_evolving(d, out, combine);
+  }
 }
 
 int check_handle(sac_handle h) {
@@ -418,12 +452,15 @@ int copy_out(Dev& d, double* dst, const void* src, int nfield, size_t esz) {
   return 0;
 }
 
-// the reductions [k0, k0+n) of register `slot` on the host (one copy, one wait)
-void red_host(Dev& d, int slot, int k0, int n, double* x) {
+// `n` reduction words from p on, on the host (one copy, one wait), or as
+// posted in host memory at word `at` (one wait)
+int red_host(Dev& d, const unsigned long long* p, int at, int n, double* x) {
   unsigned long long v[sac::kRedSlots] = {};
-  hipMemcpyAsync(v, red_of(d, slot) + k0, sizeof(v[0]) * n, hipMemcpyDeviceToHost, d.stream);
-  hipStreamSynchronize(d.stream);
-  memcpy(x, v, sizeof(double) * n);
+  if (!d.posted)
+    HIPCHK(hipMemcpyAsync(v, p, sizeof(v[0]) * n, hipMemcpyDeviceToHost, d.stream));
+  HIPCHK(hipStreamSynchronize(d.stream));
+  memcpy(x, d.posted ? d.red_host + at : v, sizeof(double) * n);
+  return 0;
 }
 
 }  // namespace
@@ -622,10 +659,11 @@ int sac_dev_init(int ndim, int ndir, const int* nx, int nw, const int* iws, int 
         d->ext1_b |= x1;
       }
     }
-  if (hipMalloc((void**)&d->red, sizeof(unsigned long long) * (kSlots + 1) * sac::kRedSlots) !=
-      hipSuccess)
+  if (hipMalloc((void**)&d->red, kRedBytes) != hipSuccess ||
+      hipHostMalloc((void**)&d->red_host, sizeof(unsigned long long) * sac::kRedSlots,
+                    hipHostMallocDefault) != hipSuccess)
     return bail(fail(SAC_E_NOMEM, "reduction buffer"));
-  hipMemset(d->red, 0, sizeof(unsigned long long) * (kSlots + 1) * sac::kRedSlots);
+  hipMemset(d->red, 0, kRedBytes);
   // getdt_grav (src/vacusr.gravity.t:114-121): computed once, at it==itmin
   d->dtgrav = kBigDouble;
   for (int k = 0; k < ndim; k++) {
@@ -654,6 +692,7 @@ int sac_dev_free(sac_handle h) {
   hipFree(d->snap);
   for (int k = 0; k < 3; k++) hipFree(d->dx[k]);
   hipFree(d->red);
+  if (d->red_host) hipHostFree(d->red_host);
   if (d->cl) {
     Closure* c = d->cl;
     hipFree(c->P32);
@@ -843,7 +882,7 @@ int sac_dev_getdt_courant(sac_handle h, double courantpar, double* dt, double* c
   if (!d.red_valid[SAC_SLOT_W]) cmax_reduce(d, SAC_SLOT_W);
   HIPCHK(hipGetLastError());
   double cmd[3] = {0.0, 0.0, 0.0};
-  red_host(d, SAC_SLOT_W, d.ndim, d.ndim, cmd);  // cmax_k/dx_k
+  if (int rc = red_host(d, red_of(d, SAC_SLOT_W) + d.ndim, d.ndim, d.ndim, cmd)) return rc;  // cmax_k/dx_k
   double cm = 0.0;
   for (int k = 0; k < d.ndim; k++) cm = std::fmax(cm, cmd[k]);
   double v = kBigDouble;
@@ -866,11 +905,9 @@ int sac_dev_getdt_special(sac_handle h, double* dt) {
     v = std::fmin(v, d.dtdiffpar * mn * mn / d.eta);
   }
   if (d.visc_on) {
-    unsigned long long u = 0;
-    HIPCHK(hipMemcpyAsync(&u, red_visc(d), sizeof(u), hipMemcpyDeviceToHost, d.stream));
-    HIPCHK(hipStreamSynchronize(d.stream));
-    double mv;
-    memcpy(&mv, &u, sizeof(mv));
+    double mv = 0.0;
+    if (!d.visc_taken)
+      if (int rc = red_host(d, red_visc(d), sac::kRedVisc, 1, &mv)) return rc;
     // getdt_visc: dtdiffpar=0.25 (assigned to the common variable, which the
     // resistive limit of later steps uses); +Inf when maxviscoef==0
     d.dtdiffpar = 0.25;
@@ -879,7 +916,7 @@ int sac_dev_getdt_special(sac_handle h, double* dt) {
       double dtd = 0.25 / mx;
       v = std::fmin(v, dtd);
     }
-    sac::launch_zero_u64(red_visc(d), 1, d.stream);
+    d.visc_taken = true;  // reset to 0
   }
   v = std::fmin(v, d.dtgrav);
   *dt = v;
@@ -1011,11 +1048,8 @@ int sac_dev_get_maxviscoef(sac_handle h, double* v) {
   if (int rc = check_handle(h)) return rc;
   if (!v) return fail(SAC_E_ARG, "null");
   Dev& d = *(Dev*)h;
-  unsigned long long u = 0;
-  HIPCHK(hipMemcpyAsync(&u, red_visc(d), sizeof(u), hipMemcpyDeviceToHost, d.stream));
-  HIPCHK(hipStreamSynchronize(d.stream));
-  memcpy(v, &u, sizeof(double));
-  return 0;
+  *v = 0.0;
+  return d.visc_taken ? 0 : red_host(d, red_visc(d), sac::kRedVisc, 1, v);
 }
 
 int sac_dev_set_maxviscoef(sac_handle h, double v) {
@@ -1026,6 +1060,8 @@ int sac_dev_set_maxviscoef(sac_handle h, double v) {
   memcpy(&u, &v, sizeof(u));
   HIPCHK(hipMemcpyAsync(red_visc(d), &u, sizeof(u), hipMemcpyHostToDevice, d.stream));
   HIPCHK(hipStreamSynchronize(d.stream));
+  d.visc_taken = false;
+  d.posted = false;
   return 0;
 }
 

@@ -157,14 +157,13 @@ __global__ void __launch_bounds__((line::Tile<K, double>::T)) kb_pline(Args a, i
   x.gamma = a.gamma;
   x.visc_on = a.visc_on;
   x.ctot_src = red_of(a, tl.tube, wct);
-  x.red_visc = a.visc + tl.tube;
   x.xcd = 1;
   x.cross_last = (K == 1) ? 1 : 0;
   double numax = 0.0;
   line::line_tile<2, NDIR, K, double, double>(x, tl.c1, L, numax, tl.c0);
   if (a.visc_on) {
     double r[1] = {numax};
-    block_max_atomic<1>(r, x.red_visc);
+    block_max_atomic<1>(r, a.visc + tl.tube);
   }
 }
 

@@ -47,12 +47,31 @@ struct GridDesc {
   int per_hi[3];
 };
 
-// reduction slots (as uint64 bit patterns of non-negative doubles), per
-// register: [d] = max over the mesh of cmax_d (c_tot of setnu) and
-// [ndim+d] = max over the mesh of cmax_d/dx_d (getdt_courant), d<ndim.
-// The maxviscoef accumulator is a separate buffer (slot 0).
-struct RedBuf {
-  unsigned long long v[kRedSlots];
+// Reductions (as uint64 bit patterns of non-negative doubles), per register:
+// [d] = max over the mesh of cmax_d (c_tot of setnu) and [ndim+d] = max over
+// the mesh of cmax_d/dx_d (getdt_courant), d<ndim; maxviscoef is a word of
+// its own.
+//
+// The blocks of a stage add their maxima to kRedLines lines of 128 bytes
+// (block b to line b % kRedLines; words as above, maxviscoef in word
+// kRedVisc), and the kernel after the stage takes the maximum over the lines
+// into the register's words and clears them (red_combine).  Maxima of one
+// word are served one after another, about 3-4 ns each: the 65536 blocks x 6
+// words of an update of 256^3 cells queued for longer than its memory
+// traffic takes.
+constexpr int kRedLines = 16;
+constexpr int kRedWords = 16;  // words per line
+constexpr int kRedVisc = 6;
+
+// What red_combine does with the lines: red[k] = max over the lines of word
+// k (k < kRedVisc); *visc = that of word kRedVisc, or the larger of it and
+// *visc (visc_keep); both also to host memory if given.
+struct RedCombine {
+  unsigned long long* acc;   // null: nothing to combine
+  unsigned long long* red;
+  unsigned long long* visc;  // null: leave maxviscoef
+  unsigned long long* host;  // pinned, kRedSlots words
+  int visc_keep;
 };
 
 }  // namespace sac

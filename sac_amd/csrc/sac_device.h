@@ -216,6 +216,43 @@ __device__ __forceinline__ void block_max_atomic(double (&v)[NV], unsigned long 
   }
 }
 
+// the block's reduction line
+__device__ __forceinline__ unsigned long long* red_line(unsigned long long* acc,
+                                                        int lines = kRedLines) {
+  return acc + (blockIdx.x % (unsigned)lines) * kRedWords;
+}
+
+// Combine and clear the reduction lines (RedCombine), by the first wavefront
+// of a block: lane (j, k) takes word k of lines j and j + 8.
+__device__ __forceinline__ void red_combine(const RedCombine& a) {
+  static_assert(kRedLines == 16 && kRedVisc < 8, "64 lanes take two lines of 8 words each");
+  const int t = (int)threadIdx.x;
+  if (t >= 64) return;
+  const int k = t & 7;
+  unsigned long long* p = a.acc + (t >> 3) * kRedWords + k;
+  unsigned long long x = p[0];
+  const unsigned long long y = p[8 * kRedWords];
+  p[0] = 0ull;
+  p[8 * kRedWords] = 0ull;
+  x = x > y ? x : y;
+#pragma unroll
+  for (int off = 8; off < 64; off <<= 1) {
+    const unsigned long long o = __shfl_xor(x, off, 64);
+    x = x > o ? x : o;
+  }
+  if (t < kRedVisc) {
+    a.red[t] = x;
+    if (a.host) a.host[t] = x;
+  } else if (t == kRedVisc && a.visc) {
+    if (a.visc_keep) {
+      const unsigned long long o = *a.visc;
+      x = x > o ? x : o;
+    }
+    *a.visc = x;
+    if (a.host) a.host[t] = x;
+  }
+}
+
 __device__ __forceinline__ double red_get(const unsigned long long* p, int k) {
   return __longlong_as_double((long long)p[k]);
 }

@@ -18,7 +18,7 @@ struct AxisArgs {
   double gamma;
   int visc_on;
   const unsigned long long* ctot_src;  // c_tot per direction of wct
-  unsigned long long* red_visc;        // maxviscoef accumulator
+  unsigned long long* acc;             // reduction lines (maxviscoef)
   int xcd;                             // XCD count for block renumbering (1 = off)
   const float* RF;                     // learned face ratios of axis K, or null (exact)
   int cross_last;                      // last axis: add the cross-term derivatives along it
@@ -44,7 +44,8 @@ struct FinalArgs {
   double grav[3];
   int grav_on[3];
   int visc_on;
-  unsigned long long* red_out;  // cmax reductions of out
+  unsigned long long* acc;      // reduction lines (cmax of out; maxviscoef of a fused stage)
+  const unsigned long long* ctot_src;  // c_tot per direction of wct (fused stages)
   int xcd;
   int skip_last;                // cross-term derivatives along the last axis already in R
   int skip_xy;                  // the x-y cross-term derivatives already in R (plane tiles)
@@ -57,7 +58,8 @@ struct CmaxArgs {
   const double* bg;
   const double* dx[3];
   double gamma;
-  unsigned long long* red_out;
+  unsigned long long* red_out;  // reduction lines, or one line (lines = 1)
+  int lines;
 };
 
 struct GhostArgs {
@@ -69,6 +71,7 @@ struct GhostArgs {
   int nvar;
   int keep_fixed;      // initial fill with fullgridini: keep file values
   int general;         // some fill has two sources (cont1; fixed1/grad1 before storage)
+  RedCombine combine;  // the stage's reductions, combined by one more block
 };
 
 // One region's fill of one field, in the reference's order (iB, then the
@@ -114,12 +117,13 @@ int line_tiles_built();
 void launch_plane(const AxisArgs& a, hipStream_t st);
 void launch_final(const FinalArgs& a, hipStream_t st);
 // a whole stage of a 1-D FP64 grid (x work and update) in one launch
-void launch_stage1(const FinalArgs& a, const unsigned long long* ctot_src,
-                   unsigned long long* red_visc, hipStream_t st);
+void launch_stage1(const FinalArgs& a, hipStream_t st);
 void launch_cmax(const CmaxArgs& a, hipStream_t st);
 void launch_ghost(const GhostArgs& a, hipStream_t st);
 // stored ghost values of the fixed/fixed1/grad1 boundaries of a.f (after a fill)
 void launch_ghost_store(const GhostArgs& a, void* store, hipStream_t st);
+// red_combine by itself, where no ghost fill follows
+void launch_combine(const RedCombine& a, hipStream_t st);
 void launch_zero_u64(unsigned long long* p, int n, hipStream_t st);
 void launch_axpy4(int prec, long long n, void* out, const void* a0, double c0, const void* a1,
                   double c1, const void* a2, double c2, const void* a3, double c3,

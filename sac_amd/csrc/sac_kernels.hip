@@ -67,7 +67,7 @@ __global__ void __launch_bounds__(256) k_axis(AxisArgs a) {
   }
   if (a.visc_on) {
     double r2[1] = {(double)numax};
-    block_max_atomic<1>(r2, a.red_visc);
+    block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
   }
 }
 
@@ -80,7 +80,7 @@ __global__ void __launch_bounds__((line::Tile<K, C>::T)) k_line(AxisArgs a, int 
   line::line_tile<NDIM, NDIR, K, S, C, LEARNED, DIVB>(a, seg, L, numax);
   if (a.visc_on) {
     double r2[1] = {(double)numax};
-    block_max_atomic<1>(r2, a.red_visc);
+    block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
   }
 }
 
@@ -92,7 +92,7 @@ __global__ void __launch_bounds__(plane::NT) k_plane(AxisArgs a) {
   plane::plane_tile<S, C>(a, sm, numax);
   if (a.visc_on) {
     double r2[1] = {(double)numax};
-    block_max_atomic<1>(r2, a.red_visc);
+    block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
   }
 }
 
@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(256) k_line1(AxisArgs a) {
   }
   if (a.visc_on) {
     double r2[1] = {numax};
-    block_max_atomic<1>(r2, a.red_visc);
+    block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
   }
 }
 
@@ -121,17 +121,16 @@ __global__ void __launch_bounds__(256) k_line1(AxisArgs a) {
 // memory a stage was two launches: 5.2 + 5.2 us at 800 cells, 8.2 + 8.5 us at
 // 60001 cells of three components; now 6.6 and 10.8 us.
 template <int LT, int NDIR, bool RK4L>
-__global__ void __launch_bounds__(LT) k_stage1(FinalArgs a, const unsigned long long* ctot_src,
-                                               unsigned long long* red_visc) {
+__global__ void __launch_bounds__(LT) k_stage1(FinalArgs a) {
   __shared__ double L[line1::LV<NDIR> * (LT + 6)];
   double numax = 0.0, redv[2] = {0.0, 0.0};
-  line1_stage<LT, NDIR, RK4L>(a, a.g, a.visc_on ? red_get(ctot_src, 0) : 0.0,
+  line1_stage<LT, NDIR, RK4L>(a, a.g, a.visc_on ? red_get(a.ctot_src, 0) : 0.0,
                               a.g.Mlo[0] + LT * (int)blockIdx.x, L, numax, redv);
   if (a.visc_on) {
     double r2[1] = {numax};
-    block_max_atomic<1>(r2, red_visc);
+    block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
   }
-  block_max_atomic<2>(redv, a.red_out);
+  block_max_atomic<2>(redv, red_line(a.acc));
 }
 
 // segment length along K: whole lines unless that leaves fewer than 2048
@@ -192,7 +191,7 @@ __global__ void __launch_bounds__(256) k_final(FinalArgs a) {
     const int nv = (V == 1) ? 1 : min(V, g.Mhi[0] - c[0] + 1);
     final_cells<NDIM, NDIR, S, C, V, RK4L>(a, g, c, nv, redv);
   }
-  block_max_atomic<2 * NDIM>(redv, a.red_out);
+  block_max_atomic<2 * NDIM>(redv, red_line(a.acc));
 }
 
 // ---------------------------------------------------------------------
@@ -224,7 +223,7 @@ __global__ void __launch_bounds__(256) k_cmax(CmaxArgs a) {
       r[NDIM + d] = cm[d] / a.dx[d][c[d]];
     }
   }
-  block_max_atomic<2 * NDIM>(r, a.red_out);
+  block_max_atomic<2 * NDIM>(r, red_line(a.red_out, a.lines));
 }
 
 // kernel 4: ghost-cell fill (see ghost_value), one ghost cell of one variable
@@ -280,6 +279,11 @@ __device__ __forceinline__ bool shell_cell(const GridDesc& g, unsigned t, int (&
 template <typename S, bool GENERAL>
 __global__ void __launch_bounds__(256) k_ghost(GhostArgs a) {
   const GridDesc& g = a.g;
+  // one block more than the shell takes: the stage's reductions
+  if (a.combine.acc && blockIdx.x == gridDim.x - 1) {
+    if (blockIdx.y == 0) red_combine(a.combine);
+    return;
+  }
   int c[3];
   if (!shell_cell(g, blockIdx.x * 256u + threadIdx.x, c)) return;
   const int v = (int)blockIdx.y;
@@ -409,6 +413,8 @@ __global__ void __launch_bounds__(256) k_prim_cons(GridDesc g, S* w, const doubl
 
 // ---------------------------------------------------------------------
 // small helpers
+
+__global__ void __launch_bounds__(64) k_combine(RedCombine a) { red_combine(a); }
 
 __global__ void k_zero_u64(unsigned long long* p, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -540,30 +546,28 @@ int launch_axis(const AxisArgs& a, int axis, hipStream_t st) {
   return (line && a.cross_last && a.visc_on && axis == g.ndim - 1) ? 1 : 0;
 }
 
-// Tile length of k_stage1: 64 cells for short grids, which spread over four
-// times as many CUs then (6.6 us a stage at 800 cells), else 256: every block adds its
-// maxima to the same words, and 938 blocks of 64 cells queued there (18.5 us a
-// stage at 60001 cells).
+// Tile length of k_stage1: 64 cells while that gives at most two blocks per
+// CU (800 cells: 9.3 us a stage with events against 10.0 for 256; 16000: 9.7
+// against 10.3), 256 above, where the 6 halo points of a tile count (60001:
+// 11.0 against 11.5; 262144: 19.2 against 23.1; 10^6: 61 against 72).
 template <int NDIR>
-static void launch_stage1_nd(const FinalArgs& a, const unsigned long long* ctot_src,
-                             unsigned long long* red_visc, hipStream_t st) {
+static void launch_stage1_nd(const FinalArgs& a, hipStream_t st) {
   const int n = a.g.Mhi[0] - a.g.Mlo[0] + 1;
-  const int LT = n > 4096 ? 256 : 64;
+  const int LT = n > 512 * 64 ? 256 : 64;
   const dim3 nb((unsigned)((n + LT - 1) / LT)), bs(LT);
   if (LT == 256) {
-    if (a.w1) hipLaunchKernelGGL((k_stage1<256, NDIR, true>), nb, bs, 0, st, a, ctot_src, red_visc);
-    else hipLaunchKernelGGL((k_stage1<256, NDIR, false>), nb, bs, 0, st, a, ctot_src, red_visc);
+    if (a.w1) hipLaunchKernelGGL((k_stage1<256, NDIR, true>), nb, bs, 0, st, a);
+    else hipLaunchKernelGGL((k_stage1<256, NDIR, false>), nb, bs, 0, st, a);
   } else {
-    if (a.w1) hipLaunchKernelGGL((k_stage1<64, NDIR, true>), nb, bs, 0, st, a, ctot_src, red_visc);
-    else hipLaunchKernelGGL((k_stage1<64, NDIR, false>), nb, bs, 0, st, a, ctot_src, red_visc);
+    if (a.w1) hipLaunchKernelGGL((k_stage1<64, NDIR, true>), nb, bs, 0, st, a);
+    else hipLaunchKernelGGL((k_stage1<64, NDIR, false>), nb, bs, 0, st, a);
   }
 }
 
-void launch_stage1(const FinalArgs& a, const unsigned long long* ctot_src,
-                   unsigned long long* red_visc, hipStream_t st) {
-  if (a.g.ndir == 1) launch_stage1_nd<1>(a, ctot_src, red_visc, st);
-  else if (a.g.ndir == 2) launch_stage1_nd<2>(a, ctot_src, red_visc, st);
-  else launch_stage1_nd<3>(a, ctot_src, red_visc, st);
+void launch_stage1(const FinalArgs& a, hipStream_t st) {
+  if (a.g.ndir == 1) launch_stage1_nd<1>(a, st);
+  else if (a.g.ndir == 2) launch_stage1_nd<2>(a, st);
+  else launch_stage1_nd<3>(a, st);
 }
 
 void launch_plane(const AxisArgs& a, hipStream_t st) {
@@ -596,7 +600,7 @@ void launch_ghost(const GhostArgs& a, hipStream_t st) {
   long long n = ncell - mesh_cells(g);
   if (n <= 0) return;
   const int bs = 256;
-  const dim3 grid((unsigned)((n + bs - 1) / bs), (unsigned)a.nvar);
+  const dim3 grid((unsigned)((n + bs - 1) / bs) + (a.combine.acc ? 1u : 0u), (unsigned)a.nvar);
   if (a.prec == PREC_MIXED) {
     if (a.general)
       hipLaunchKernelGGL((k_ghost<float, true>), grid, dim3(bs), 0, st, a);
@@ -655,6 +659,10 @@ void launch_ghost_store(const GhostArgs& a, void* store, hipStream_t st) {
     hipLaunchKernelGGL(k_ghost_store<float>, grid, dim3(bs), 0, st, a, (float*)store);
   else
     hipLaunchKernelGGL(k_ghost_store<double>, grid, dim3(bs), 0, st, a, (double*)store);
+}
+
+void launch_combine(const RedCombine& a, hipStream_t st) {
+  hipLaunchKernelGGL(k_combine, dim3(1), dim3(64), 0, st, a);
 }
 
 void launch_zero_u64(unsigned long long* p, int n, hipStream_t st) {

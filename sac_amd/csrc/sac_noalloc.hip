@@ -105,6 +105,7 @@ extern "C" int sac_getdt_courant_noalloc(int ndim, int ndir, const int* nx, int 
   a.dx[2] = (ndim > 2) ? dx + g.G[0] + g.G[1] : nullptr;
   a.gamma = gamma;
   a.red_out = red;
+  a.lines = 1;
   sac::launch_cmax(a, st);
   e = hipGetLastError();
   if (e != hipSuccess) return sac::set_error(SAC_E_HIP, "cmax launch: %s", hipGetErrorString(e));
