@@ -375,7 +375,7 @@ program sac_vac
   ! copied off the device while the next steps run and written once it has
   ! arrived, with the it, t and dt of the iteration that asked for it
   ! (SAC_SYNC_SAVES=1 in the environment downloads and writes at once)
-  logical :: asyncsave, savepending, savedue(nfile)
+  logical :: asyncsave, savepending, savedue(nfile), savesnap(nfile)
   integer :: itsnap
   real(dp) :: tsnap, dtsnap
   character(len=8) :: envval
@@ -505,6 +505,7 @@ program sac_vac
         call finish_save()
         call check(sac_dev_save_begin(h))
         savepending = .true.
+        savesnap = savedue
         itsnap = it
         tsnap = t
         dtsnap = dt
@@ -561,7 +562,8 @@ contains
     if (code /= 0) call die('libsac_amd: ' // trim(sac_error_message()))
   end subroutine check
 
-  ! write the files of the pending asynchronous save (waits for its copy)
+  ! write the files of the pending asynchronous save (waits for its copy):
+  ! those that were due when it began, not those due now
   subroutine finish_save()
     integer :: itnow
     real(dp) :: tnow, dtnow
@@ -575,7 +577,7 @@ contains
     t = tsnap
     dt = dtsnap
     do ifile = 1, nfile
-      if (savedue(ifile)) call savefile(ifile)
+      if (savesnap(ifile)) call savefile(ifile)
     end do
     it = itnow
     t = tnow
