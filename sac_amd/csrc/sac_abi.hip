@@ -320,7 +320,9 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   // sources have to join the rate first
   const bool stage1 = d.ndim == 1 && d.prec == SAC_PREC_FP64 && !learned && !(d.eta > 0.0) &&
                       sac::line_tiles_built();
-  for (int k = plane ? 2 : 0; k < d.ndim && !stage1; k++) {
+  // 2-D: the same, with the resistive sources handed over in R
+  const bool stage2 = d.plane && d.ndim == 2 && !learned && sac::stage_tiles_fit(d.g);
+  for (int k = plane ? 2 : 0; k < d.ndim && !stage1 && !stage2; k++) {
     // axis 1 (rows of a plane): neighbour rows in one XCD's L2.  Axes 0 and 2
     // keep the hardware order, whose round-robin already places the
     // neighbour planes of a row in the same XCD.
@@ -353,6 +355,7 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
     ra.R = d.rate;
     ra.eta = d.eta;
     ra.compact = d.compactres;
+    ra.fresh = stage2 ? 1 : 0;
     sac::launch_resistive(ra, d.stream);
   }
   sac::FinalArgs s{};
@@ -383,10 +386,15 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   s.skip_xy = plane ? 1 : 0;
   hipEvent_t e0{};
   t_begin(d, SAC_K_FINAL, &e0);
-  if (stage1)
+  if (stage1) {
     sac::launch_stage1(s, d.stream);
-  else
+  } else if (stage2) {
+    s.divbfix = d.divbfix;
+    if (!(d.eta > 0.0)) s.R = nullptr;
+    sac::launch_stage(s, d.stream);
+  } else {
     sac::launch_final(s, d.stream);
+  }
   t_end(d, SAC_K_FINAL, e0);
   d.red_valid[out] = true;
   const sac::RedCombine combine = stage_combine(d, out);

@@ -14,9 +14,8 @@
 // hipGraph holding several steps and replayed until every tube has reached
 // tmax; finished tubes skip their tiles.
 //
-// The line work and the combining update are the grid path's own device
-// functions (line1_tile for tubes, line_tile for patches, final_cell)
-// applied to a per-tube grid descriptor, so a tube or patch advanced here
+// A stage is the grid path's own device function (line1_stage for tubes,
+// stage_tile for patches) applied to a per-tube grid descriptor, so a tube or patch advanced here
 // follows the same arithmetic as the same tube or patch run alone through
 // sac_dev_*, bit for bit.
 #include <hip/hip_runtime.h>
@@ -32,7 +31,7 @@
 
 #include "../../include/sac_amd.h"
 #include "sac_device.h"
-#include "sac_line.h"
+#include "sac_tile.h"
 
 namespace sac {
 namespace batch {
@@ -40,7 +39,6 @@ namespace batch {
 constexpr int NDIR = 3;
 constexpr int NE = 2 + 2 * NDIR;  // evolving fields
 constexpr int NBG = 2 + NDIR;     // background fields
-constexpr int NT2 = 4;            // cross-term factor fields of a 2-D patch (2*ndim*(ndim-1))
 constexpr int kSlots = 4;         // W, S1, S2, S3
 constexpr int kRed = 4;           // per tube and register: max cmax_d, then max cmax_d/dx_d (d < ndim)
 
@@ -68,13 +66,11 @@ struct Args {
   int tbx;                   // tile width along x in cells (2-D)
   const int* active;         // tubes still running when the tiles were built
   int nactive;
-  const Tile* ltiles[2];     // patches: line tiles of x and y as (patch, logical block, segment)
-  int nltiles[2];
+  const Tile* stiles;        // patches: stage tiles (first cell at column c0 and row c1)
+  int nstiles;
   double* reg[kSlots];
   const double* bg;
   const double* dx;          // cell widths per tube: G_x values, then G_y values
-  double* R;
-  double* T;                 // cross-term factors (2-D), packed like NT2 fields
   unsigned long long* red;   // [tube][slot][kRed]
   unsigned long long* visc;  // [tube] maxviscoef since the last dt
   double* t;
@@ -132,41 +128,6 @@ __device__ __forceinline__ bool tile_cell(const Args& a, const Tile& tl, const G
   return c[0] <= g.Mhi[0] && c[1] <= g.Mhi[1];
 }
 
-// Patches: the work of axis K as the grid path's LDS line tiles (line_tile,
-// sac_line.h) on the patch's own grid; ltiles[K] holds (patch, logical
-// block, segment length along K).  The y kernel adds the y derivatives of
-// the x kernel's cross factors, as on a grid.  The x kernel's first block
-// of a patch also clears the patch's reductions of register `out`.
-template <int K>
-__global__ void __launch_bounds__((line::Tile<K, double>::T)) kb_pline(Args a, int wct, int out) {
-  __shared__ double L[line::lds_elems<2, NDIR, K, double, false>()];
-  const Tile tl = a.ltiles[K][blockIdx.x];
-  if (a.state[tl.tube] != RUNNING) return;  // uniform over the block
-  if (K == 0 && threadIdx.x < kRed && tl.c0 == 0) red_of(a, tl.tube, out)[threadIdx.x] = 0ull;
-  const GridDesc g = tube_grid<2>(a, tl.tube);
-  const long long o = a.start[tl.tube];
-  AxisArgs x{};
-  x.g = g;
-  x.prec = PREC_FP64;
-  x.wct = a.reg[wct] + o;
-  x.bg = a.bg + o;
-  x.dx[0] = a.dx + a.dxo[tl.tube];
-  x.dx[1] = x.dx[0] + g.G[0];
-  x.R = a.R + o;
-  x.T = a.T + o;
-  x.gamma = a.gamma;
-  x.visc_on = a.visc_on;
-  x.ctot_src = red_of(a, tl.tube, wct);
-  x.xcd = 1;
-  x.cross_last = (K == 1) ? 1 : 0;
-  double numax = 0.0;
-  line::line_tile<2, NDIR, K, double, double>(x, tl.c1, L, numax, tl.c0);
-  if (a.visc_on) {
-    double r[1] = {numax};
-    block_max_atomic<1>(r, a.visc + tl.tube);
-  }
-}
-
 // 'cont' ghost cells (getboundary, src/vacgrid.t:366-370) whose value is
 // that of mesh cell c of register f, written by the thread that stored c.
 // The reference fills the x regions over the whole grid along y, then the
@@ -204,47 +165,51 @@ __device__ __forceinline__ void set_rk4(const Args& a, long long o, FinalArgs& f
   }
 }
 
-// Patches: combining update of one tile: out = base + dt/da * R (see
-// set_rk4), with the x derivatives of the cross factors, then the 'cont'
-// ghosts of out
-template <int NDIM, int CK, bool RK4L>
-__global__ void __launch_bounds__(256) kb_final(Args a, int wct, int base, int out, double da) {
-  const Tile tl = a.tiles[blockIdx.x];
-  if (a.state[tl.tube] != RUNNING) return;
-  const GridDesc g = tube_grid<NDIM>(a, tl.tube);
+// The second stage's first tile of a tube clears the tube's reductions of W,
+// which the last stage fills: kb_dt and the first stage have read them, and
+// kb_dt has cleared those of the other registers.
+__device__ __forceinline__ void clear_red_w(const Args& a, int tube, bool first, int out) {
+  if (out == SAC_SLOT_S2 && first && threadIdx.x < kRed)
+    red_of(a, tube, SAC_SLOT_W)[threadIdx.x] = 0ull;
+}
+
+// Patches: a whole RK stage of one 16 x 16 tile (stage_tile, also used by 2-D
+// grids), with the 'cont' ghosts of its cells.  512 patches
+// of 32-160 cells (4.8 M): 0.706 ms a stage, RK4's last 0.769; the two line
+// kernels and the update before took 0.996 and 1.155.
+template <bool RK4L, typename Off>
+__global__ void __launch_bounds__(tile::NT) kb_patch_stage(Args a, int wct, int base, int out,
+                                                           double da) {
+  __shared__ tile::Smem<2, NDIR, double, false> sm;
+  // each XCD takes one contiguous range of tiles (shared halos in one L2)
+  const unsigned b = xcd_block8();
+  if (b >= (unsigned)a.nstiles) return;
+  const Tile tl = a.stiles[b];
+  if (a.state[tl.tube] != RUNNING) return;  // uniform over the block
+  const GridDesc g = tube_grid<2>(a, tl.tube);
+  clear_red_w(a, tl.tube, tl.c0 == 0 && tl.c1 == g.Mlo[1], out);
   const long long o = a.start[tl.tube];
-  const double dt = a.dt[tl.tube];
   FinalArgs f{};
   f.g = g;
   f.prec = PREC_FP64;
   f.wct = a.reg[wct] + o;
   f.bg = a.bg + o;
   f.dx[0] = a.dx + a.dxo[tl.tube];
-  if (NDIM == 2) f.dx[1] = f.dx[0] + g.G[0];
-  f.R = a.R + o;
-  f.T = (NDIM == 2) ? a.T + o : nullptr;
+  f.dx[1] = f.dx[0] + g.G[0];
   f.base = a.reg[base] + o;
   f.out = a.reg[out] + o;
   set_rk4<RK4L>(a, o, f);
-  f.qa = dt / da;
+  f.qa = a.dt[tl.tube] / da;
   f.gamma = a.gamma;
   f.visc_on = a.visc_on;
-  f.skip_last = (NDIM == 2) ? 1 : 0;  // the y line tiles added their cross terms
-  double redv[2 * NDIM];
-#pragma unroll
-  for (int k = 0; k < 2 * NDIM; k++) redv[k] = 0.0;
-#pragma unroll
-  for (int j = 0; j < CK; j++) {
-    int c[3];
-    if (tile_cell<NDIM, CK>(a, tl, g, j, c)) {
-      double r[2 * NDIM];
-      final_cell<NDIM, NDIR, double, double, RK4L>(f, g, c, r);
-      cont_ghosts_of<NDIM>(g, (double*)f.out, c);
-#pragma unroll
-      for (int k = 0; k < 2 * NDIM; k++) redv[k] = fmax(redv[k], r[k]);
-    }
-  }
-  block_max_atomic<2 * NDIM>(redv, red_of(a, tl.tube, out));
+  f.ctot_src = red_of(a, tl.tube, wct);
+  double numax = 0.0, redv[4] = {0.0, 0.0, 0.0, 0.0};
+  int c[3];
+  if (tile::stage_tile<2, NDIR, double, double, RK4L, false, Off>(f, g, tl.c0, tl.c1, 0, sm.v,
+                                                                  numax, redv, c))
+    cont_ghosts_of<2>(g, (double*)f.out, c);
+  double r[5] = {redv[0], redv[1], redv[2], redv[3], numax};
+  block_max_atomic<5>(r, red_of(a, tl.tube, out), a.visc + tl.tube);
 }
 
 // Tubes: one whole RK stage of a tile of LT cells in one kernel: the x work
@@ -253,13 +218,13 @@ __global__ void __launch_bounds__(256) kb_final(Args a, int wct, int base, int o
 // registers, with the 'cont' ghosts.  With R stored and read back a
 // stage of 4.5 M cells took 0.383 ms (0.478 ms RK4's last), now 0.314 (0.388);
 // 232 B per cell without R, 3.3 TB/s: latency of two waits per block.
-// The reductions of `out` must have been cleared by kb_zero_red.
 template <int LT, bool RK4L>
 __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, int out, double da) {
   __shared__ double L[line1::LV<NDIR> * (LT + 6)];
   const Tile tl = a.tiles[blockIdx.x];
   if (a.state[tl.tube] != RUNNING) return;  // uniform over the block
   const GridDesc g = tube_grid<1>(a, tl.tube);
+  clear_red_w(a, tl.tube, tl.c0 == g.Mlo[0], out);
   const long long o = a.start[tl.tube];
   const double dt = a.dt[tl.tube];
   FinalArgs f{};
@@ -279,11 +244,8 @@ __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, i
   const int c[3] = {tl.c0 + (int)threadIdx.x, 0, 0};
   if (line1_stage<LT, NDIR, RK4L>(f, g, ctk, tl.c0, L, numax, redv))
     cont_ghosts_of<1>(g, (double*)f.out, c);
-  if (a.visc_on) {
-    double r[1] = {numax};
-    block_max_atomic<1>(r, a.visc + tl.tube);
-  }
-  block_max_atomic<2>(redv, red_of(a, tl.tube, out));
+  double r[3] = {redv[0], redv[1], numax};
+  block_max_atomic<3>(r, red_of(a, tl.tube, out), a.visc + tl.tube);
 }
 
 // cmax reductions of register `slot` of every running tube
@@ -378,6 +340,7 @@ __device__ __forceinline__ double red_val(const unsigned long long* p) {
 // getdt_courant (src/vac.t:641-699), getdt_visc (src/vacusr.viscosity.t:509-541,
 // dtdiffpar 0.25, maxviscoef reset), then timetofinish (src/vac.t:585-605).
 // A tube whose dt is not a positive finite number is stopped as FAILED.
+// The reductions of the step's stage registers are cleared.
 __global__ void kb_dt(Args a) {
   const int tube = blockIdx.x * blockDim.x + threadIdx.x;
   if (tube >= a.ntubes || a.state[tube] != RUNNING) return;
@@ -394,6 +357,7 @@ __global__ void kb_dt(Args a) {
     }
     a.visc[tube] = 0ull;
   }
+  for (int k = SAC_SLOT_S1 * kRed; k < kSlots * kRed; k++) red_of(a, tube, 0)[k] = 0ull;
   if (a.it[tube] >= a.itmax || a.t[tube] >= a.tmax) {
     a.state[tube] = FINISHED;
   } else if (dt < a.dtmin) {
@@ -442,8 +406,10 @@ int bfail(int code, const char* fmt, ...) {
   } while (0)
 
 // launch shapes the autotuner chooses from.  Tubes: tiles of tb consecutive
-// cells of one tube, one cell per thread (kb_tube_stage<tb>).  Patches: one cell per thread, tiles of tbx x (tb/tbx)
-// cells.  Every shape gives the same result bit for bit.
+// cells of one tube, one cell per thread (kb_tube_stage<tb>).  Patches: a
+// stage has one tile, 16 x 16 cells; the shapes, tbx x (tb/tbx) cells, are
+// those of the first cmax sweep, and the autotuner times the steps only.
+// Every shape gives the same result bit for bit.
 struct Shape {
   int ck, tb, tbx;
 };
@@ -471,13 +437,12 @@ struct Batch {
   int* d_pitch = nullptr;
   long long* d_dxo = nullptr;
   Tile* d_tiles = nullptr;
-  Tile* d_ltiles[2] = {nullptr, nullptr};
+  Tile* d_stiles = nullptr;
+  bool rows_fit = true;          // 32-bit offsets in the stage tiles
   int* d_active = nullptr;
   double* d_reg[kSlots] = {nullptr, nullptr, nullptr, nullptr};
   double* d_bg = nullptr;
   double* d_dx = nullptr;
-  double* d_R = nullptr;
-  double* d_T = nullptr;
   double* d_save = nullptr;  // state kept aside while the autotuner runs
   unsigned long long* d_red = nullptr;
   unsigned long long* d_visc = nullptr;
@@ -509,9 +474,6 @@ int balloc(Batch& b, void** p, size_t bytes) {
   return 0;
 }
 
-// patch counts at or below which the line tiles use short segments
-constexpr size_t kFewPatches = 64;
-
 int set_shape(Batch& b, Shape s) {
   // the graph's kernel nodes hold the tile tables freed below: destroy the
   // executable graph first (the stream is idle here), so no graph ever
@@ -534,37 +496,20 @@ int set_shape(Batch& b, Shape s) {
   }
   if (tiles.empty()) tiles.push_back({b.active.empty() ? 0 : b.active[0], 2, 2});
   if (b.ndim == 2) {
-    // line tiles of each axis: every logical block of each running patch's
-    // grid.  Whole lines while many patches run; once few remain (their
-    // steps are latency-bound), segments of 32 cells give more, shorter
-    // blocks.  The result does not depend on the segment length.
-    const bool few = b.active.size() <= kFewPatches;
-    for (int K = 0; K < 2; K++) {
-      std::vector<Tile> lt;
-      for (int i : b.active) {
-        sac::GridDesc g{};
-        g.ndim = 2;
-        g.ndir = NDIR;
-        g.G[0] = b.gx(i);
-        g.G[1] = b.gy(i);
-        g.G[2] = 1;
-        g.Mlo[0] = g.Mlo[1] = 2;
-        g.Mhi[0] = g.G[0] - 3;
-        g.Mhi[1] = g.G[1] - 3;
-        const int ext = g.Mhi[K] - g.Mlo[K] + 1;
-        const int seg = few ? std::min(ext, 32) : ext;
-        const long long nb = (K == 0) ? sac::line::nblocks<2, 0, double>(g, seg)
-                                      : sac::line::nblocks<2, 1, double>(g, seg);
-        for (long long k = 0; k < nb; k++) lt.push_back({i, (int)k, seg});
-      }
-      if (lt.empty()) lt.push_back({b.active.empty() ? 0 : b.active[0], 1 << 30, 1});
-      if (b.d_ltiles[K]) hipFree(b.d_ltiles[K]);
-      b.d_ltiles[K] = nullptr;
-      BCHK(hipMalloc((void**)&b.d_ltiles[K], sizeof(Tile) * lt.size()));
-      BCHK(hipMemcpy(b.d_ltiles[K], lt.data(), sizeof(Tile) * lt.size(), hipMemcpyHostToDevice));
-      b.a.ltiles[K] = b.d_ltiles[K];
-      b.a.nltiles[K] = (int)lt.size();
-    }
+    // stage tiles of each running patch, along x from grid column 0
+    std::vector<Tile> st;
+    b.rows_fit = true;
+    for (int i : b.active) b.rows_fit = b.rows_fit && sac::tile::rows_fit(b.pitch[i]);
+    for (int i : b.active)
+      for (int c1 = 2; c1 < 2 + b.nxy[2 * i + 1]; c1 += sac::tile::TY)
+        for (int c0 = 0; c0 < 2 + b.nxy[2 * i]; c0 += sac::tile::TX) st.push_back({i, c0, c1});
+    if (st.empty()) st.push_back({b.active.empty() ? 0 : b.active[0], 0, 2});
+    b.a.nstiles = (int)st.size();
+    if (b.d_stiles) hipFree(b.d_stiles);
+    b.d_stiles = nullptr;
+    BCHK(hipMalloc((void**)&b.d_stiles, sizeof(Tile) * st.size()));
+    BCHK(hipMemcpy(b.d_stiles, st.data(), sizeof(Tile) * st.size(), hipMemcpyHostToDevice));
+    b.a.stiles = b.d_stiles;
   }
   if (b.d_tiles) hipFree(b.d_tiles);
   b.d_tiles = nullptr;
@@ -605,8 +550,16 @@ void launch_tube_stage(Batch& b, dim3 gt, dim3 bt, int wct, int base, int out, d
     hipLaunchKernelGGL((kb_tube_stage<256, RK4L>), gt, bt, 0, b.stream, a, wct, base, out, da);
 }
 
-template <int NDIM, int CK>
-void enqueue_step_ck(Batch& b) {
+template <typename Off>
+void launch_patch_stage(Batch& b, int wct, int base, int out, double da, int last) {
+  const dim3 gs((unsigned)((b.a.nstiles + 7) / 8 * 8)), bs(sac::tile::NT);  // for xcd_block8
+  if (last)
+    hipLaunchKernelGGL((kb_patch_stage<true, Off>), gs, bs, 0, b.stream, b.a, wct, base, out, da);
+  else
+    hipLaunchKernelGGL((kb_patch_stage<false, Off>), gs, bs, 0, b.stream, b.a, wct, base, out, da);
+}
+
+void enqueue_step(Batch& b) {
   const Args& a = b.a;
   hipStream_t st = b.stream;
   const dim3 gt(b.ntiles), bt(b.shape.tb);
@@ -626,31 +579,16 @@ void enqueue_step_ck(Batch& b) {
                         {S2, W, S3, 1.0, 0},
                         {S3, W, W, 6.0, 1}};
   for (const St& s : stages) {
-    if constexpr (NDIM == 1) {
-      hipLaunchKernelGGL(kb_zero_red, gn, bn, 0, st, a, s.out);
+    if (b.ndim == 1) {
       if (s.last) launch_tube_stage<true>(b, gt, bt, s.wct, s.base, s.out, s.da);
       else launch_tube_stage<false>(b, gt, bt, s.wct, s.base, s.out, s.da);
-      continue;
+    } else if (b.rows_fit) {
+      launch_patch_stage<unsigned>(b, s.wct, s.base, s.out, s.da, s.last);
     } else {
-      hipLaunchKernelGGL(kb_pline<0>, dim3(a.nltiles[0]), dim3(sac::line::Tile<0, double>::T), 0, st,
-                         a, s.wct, s.out);
-      hipLaunchKernelGGL(kb_pline<1>, dim3(a.nltiles[1]), dim3(sac::line::Tile<1, double>::T), 0, st,
-                         a, s.wct, s.out);
+      launch_patch_stage<unsigned long long>(b, s.wct, s.base, s.out, s.da, s.last);
     }
-    if (s.last)
-      hipLaunchKernelGGL((kb_final<NDIM, CK, true>), gt, bt, 0, st, a, s.wct, s.base, s.out, s.da);
-    else
-      hipLaunchKernelGGL((kb_final<NDIM, CK, false>), gt, bt, 0, st, a, s.wct, s.base, s.out,
-                         s.da);
   }
   hipLaunchKernelGGL(kb_tick, gn, bn, 0, st, a);
-}
-
-void enqueue_step(Batch& b) {
-  if (b.ndim == 2)
-    enqueue_step_ck<2, 1>(b);
-  else
-    enqueue_step_ck<1, 1>(b);
 }
 
 void enqueue_cmax(Batch& b, int slot) {
@@ -794,8 +732,6 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   for (int s = 0; s < kSlots; s++)
     if ((rc = balloc(*b, (void**)&b->d_reg[s], fb * NE))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_bg, fb * NBG))) return bail(rc);
-  if ((rc = balloc(*b, (void**)&b->d_R, fb * NE))) return bail(rc);
-  if (ndim == 2 && (rc = balloc(*b, (void**)&b->d_T, fb * NT2))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_dx, sizeof(double) * (size_t)doff))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_start, sizeof(long long) * ntubes))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_nxy, sizeof(int) * 2 * ntubes))) return bail(rc);
@@ -862,8 +798,6 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   for (int s = 0; s < kSlots; s++) a.reg[s] = b->d_reg[s];
   a.bg = b->d_bg;
   a.dx = b->d_dx;
-  a.R = b->d_R;
-  a.T = b->d_T;
   a.red = b->d_red;
   a.visc = b->d_visc;
   a.t = b->d_t;
@@ -905,16 +839,13 @@ int sac_batch_free(sac_batch_handle h) {
   for (int s = 0; s < kSlots; s++) hipFree(b->d_reg[s]);
   hipFree(b->d_bg);
   hipFree(b->d_dx);
-  hipFree(b->d_R);
-  hipFree(b->d_T);
   hipFree(b->d_save);
   hipFree(b->d_start);
   hipFree(b->d_nxy);
   hipFree(b->d_pitch);
   hipFree(b->d_dxo);
   hipFree(b->d_tiles);
-  hipFree(b->d_ltiles[0]);
-  hipFree(b->d_ltiles[1]);
+  hipFree(b->d_stiles);
   hipFree(b->d_active);
   hipFree(b->d_red);
   hipFree(b->d_visc);
@@ -947,11 +878,10 @@ int sac_batch_tune(sac_batch_handle h, int trial_steps, int* ck, int* tb, double
   if (int rc = save_state(b, r0)) return rc;
   double best = 1e300;
   Shape bs = b.shape;
-  const Shape* shapes = (b.ndim == 1) ? kShapes1 : kShapes2;
-  const int nshape = (b.ndim == 1) ? (int)(sizeof(kShapes1) / sizeof(Shape))
-                                   : (int)(sizeof(kShapes2) / sizeof(Shape));
+  const Shape* shapes = (b.ndim == 1) ? kShapes1 : &bs;
+  const int nshape = (b.ndim == 1) ? (int)(sizeof(kShapes1) / sizeof(Shape)) : 1;
   for (int k = 0; k < nshape; k++) {
-    const Shape& s = shapes[k];
+    const Shape s = shapes[k];
     if (int rc = set_shape(b, s)) return rc;
     if (int rc = build_graph(b, trial_steps)) return rc;
     BCHK(hipGraphLaunch(b.graph, b.stream));  // warm-up replay

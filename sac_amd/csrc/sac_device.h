@@ -195,24 +195,44 @@ __device__ __forceinline__ void cmax_all(const Pt<NDIR, double>& p, double gamma
 // ---------------------------------------------------------------------
 // block-wide max reduction into uint64 atomics (values are >= 0)
 
+// maximum over the wavefront, in lane 63: row shifts within 16 lanes, then
+// the rows' last lanes broadcast to the rows above them
+template <int CTRL>
+__device__ __forceinline__ double max_dpp(double x) {
+  const int lo = __double2loint(x), hi = __double2hiint(x);
+  // lanes without a source keep their own value
+  const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
+  const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
+  return fmax(x, __hiloint2double(h2, l2));
+}
+__device__ __forceinline__ double wave_max63(double x) {
+  x = max_dpp<0x111>(x);  // row_shr:1, 2, 4, 8
+  x = max_dpp<0x112>(x);
+  x = max_dpp<0x114>(x);
+  x = max_dpp<0x118>(x);
+  x = max_dpp<0x142>(x);  // row_bcast:15, 31
+  return max_dpp<0x143>(x);
+}
+
+// v[k] to dst[k], or the last one to *last
 template <int NV>
-__device__ __forceinline__ void block_max_atomic(double (&v)[NV], unsigned long long* dst) {
+__device__ __forceinline__ void block_max_atomic(double (&v)[NV], unsigned long long* dst,
+                                                 unsigned long long* last = nullptr) {
   __shared__ double red[NV][16];
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < NV; k++) {
-    double x = v[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off, 64));
-    if (lane == 0) red[k][wid] = x;
+    const double x = wave_max63(v[k]);
+    if (lane == 63) red[k][wid] = x;
   }
   __syncthreads();
   if (threadIdx.x < NV) {
     const int nwave = (blockDim.x + 63) >> 6;
     double x = 0.0;
     for (int j = 0; j < nwave; j++) x = fmax(x, red[threadIdx.x][j]);
-    atomicMax(dst + threadIdx.x, (unsigned long long)__double_as_longlong(x));
+    unsigned long long* p = (last && threadIdx.x == NV - 1) ? last : dst + threadIdx.x;
+    atomicMax(p, (unsigned long long)__double_as_longlong(x));
   }
 }
 
@@ -326,6 +346,13 @@ __device__ __forceinline__ long long xcd_block(int xcd) {
   if (xcd <= 1 || (nb % (unsigned)xcd) != 0) return blockIdx.x;
   const unsigned per = nb / (unsigned)xcd;
   return (long long)(blockIdx.x % (unsigned)xcd) * per + blockIdx.x / (unsigned)xcd;
+}
+
+// the same for a launch of a multiple of 8 blocks, in 32 bits (a 64-bit
+// division by a value that is no constant takes about a hundred scalar
+// instructions before a block's first load)
+__device__ __forceinline__ unsigned xcd_block8() {
+  return (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
 }
 
 // ---------------------------------------------------------------------
@@ -943,6 +970,57 @@ __device__ __forceinline__ void update_cells(const FinalArgs& a, const GridDesc&
         redv[NDIM + d] = fmax(redv[NDIM + d], r1);
       }
     }
+  }
+}
+
+// update_cells of one cell whose base register and background are at hand
+// (the loads of base precede the stores to out, which may be the same)
+template <int NDIM, int NDIR, typename S, typename C, bool RK4L>
+__device__ __forceinline__ void update_cell(const FinalArgs& a, const GridDesc& g,
+                                            const int (&c)[3], long long ic,
+                                            const S (&base)[2 + 2 * NDIR],
+                                            const Pt<NDIR, C>& own,
+                                            const C (&R)[2 + 2 * NDIR],
+                                            double (&redv)[2 * NDIM]) {
+  constexpr int NE = 2 + 2 * NDIR;
+  const long long fs = g.fs;
+  S o[NE];
+  if constexpr (RK4L) {
+    const S* __restrict__ r1 = (const S*)a.w1;
+    const S* __restrict__ r2 = (const S*)a.w2;
+    const S* __restrict__ r3 = (const S*)a.wct;
+#pragma unroll
+    for (int n = 0; n < NE; n++) {
+#pragma clang fp contract(off)
+      const long long i = n * fs + ic;
+      const double b = (double)base[n];
+      const double w = ((((double)r1[i] + 2.0 * (double)r2[i]) + (double)r3[i]) - 4.0 * b) / 3.0;
+      o[n] = (S)(fma(a.qa, (double)R[n], b) + w);
+    }
+  } else {
+#pragma unroll
+    for (int n = 0; n < NE; n++) o[n] = (S)((double)base[n] + a.qa * (double)R[n]);
+  }
+  S* out = (S*)a.out;
+#pragma unroll
+  for (int n = 0; n < NE; n++) out[n * fs + ic] = o[n];
+  Pt<NDIR, double> po;
+  po.rho = (double)o[0];
+  po.e = (double)o[1 + NDIR];
+  po.eb = own.eb;
+  po.rhob = own.rhob;
+#pragma unroll
+  for (int cd = 0; cd < NDIR; cd++) {
+    po.m[cd] = (double)o[1 + cd];
+    po.b[cd] = (double)o[2 + NDIR + cd];
+    po.bg[cd] = own.bg[cd];
+  }
+  double cm[NDIM];
+  cmax_all<NDIM, NDIR>(po, a.gamma, cm);
+#pragma unroll
+  for (int d = 0; d < NDIM; d++) {
+    redv[d] = cm[d];
+    redv[NDIM + d] = cm[d] / a.dx[d][c[d]];
   }
 }
 

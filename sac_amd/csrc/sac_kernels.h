@@ -49,6 +49,7 @@ struct FinalArgs {
   int xcd;
   int skip_last;                // cross-term derivatives along the last axis already in R
   int skip_xy;                  // the x-y cross-term derivatives already in R (plane tiles)
+  int divbfix;                  // Powell's sources (fused stages)
 };
 
 struct CmaxArgs {
@@ -104,6 +105,7 @@ struct ResistArgs {
   void* R;               // rate accumulator
   double eta;
   int compact;           // 1: addsource_res1, 0: addsource_res2
+  int fresh;             // R = the sources instead of R += them
 };
 void launch_resistive(const ResistArgs& a, hipStream_t st);
 
@@ -116,6 +118,11 @@ int line_tiles_built();
 // the x-y cross terms included; R is written fresh
 void launch_plane(const AxisArgs& a, hipStream_t st);
 void launch_final(const FinalArgs& a, hipStream_t st);
+// a whole stage of a 2-D grid in one launch; a.R, if given, is added to the
+// rate (k_resist)
+void launch_stage(const FinalArgs& a, hipStream_t st);
+// 1 if the tiles of launch_stage can address a plane of the grid
+int stage_tiles_fit(const GridDesc& g);
 // a whole stage of a 1-D FP64 grid (x work and update) in one launch
 void launch_stage1(const FinalArgs& a, hipStream_t st);
 void launch_cmax(const CmaxArgs& a, hipStream_t st);

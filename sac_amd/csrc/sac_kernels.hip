@@ -26,6 +26,7 @@
 #include "sac_device.h"
 #include "sac_line.h"
 #include "sac_plane.h"
+#include "sac_tile.h"
 
 // SAC_LINE_TILES=0 keeps the line-group kernel k_axis for every grid (the
 // default runs 2-D and 3-D grids through the LDS line tiles, k_line)
@@ -126,11 +127,33 @@ __global__ void __launch_bounds__(LT) k_stage1(FinalArgs a) {
   double numax = 0.0, redv[2] = {0.0, 0.0};
   line1_stage<LT, NDIR, RK4L>(a, a.g, a.visc_on ? red_get(a.ctot_src, 0) : 0.0,
                               a.g.Mlo[0] + LT * (int)blockIdx.x, L, numax, redv);
-  if (a.visc_on) {
-    double r2[1] = {numax};
-    block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
-  }
-  block_max_atomic<2>(redv, red_line(a.acc));
+  double m[3] = {redv[0], redv[1], numax};
+  block_max_atomic<3>(m, red_line(a.acc), red_line(a.acc) + kRedVisc);
+}
+
+// 2-D grids: a whole RK stage per launch (see stage_tile)
+template <int NDIM, int NDIR, typename S, typename C, bool RK4L, bool DIVB>
+__global__ void __launch_bounds__(tile::NT) k_stage(FinalArgs a) {
+  __shared__ tile::Smem<NDIM, NDIR, C, DIVB> sm;
+  // block -> tile: each XCD takes one contiguous range of tiles, so the halos
+  // a tile shares with its neighbours are fetched into one L2
+  const unsigned b = xcd_block8(), nx = tile::ntx(a.g), ny = tile::nty(a.g);
+  const unsigned r = b / nx, zt = r / ny;
+  if (zt > (unsigned)(a.g.Mhi[2] - a.g.Mlo[2])) return;
+  const int x0 = (int)(b - r * nx) * tile::TX;
+  const int y0 = a.g.Mlo[1] + (int)(r - zt * ny) * tile::TY;
+  const int z = a.g.Mlo[2] + (int)zt;
+  C numax = 0;
+  double redv[2 * NDIM];
+#pragma unroll
+  for (int k = 0; k < 2 * NDIM; k++) redv[k] = 0.0;
+  int c[3];
+  tile::stage_tile<NDIM, NDIR, S, C, RK4L, DIVB>(a, a.g, x0, y0, z, sm.v, numax, redv, c);
+  double m[2 * NDIM + 1];
+#pragma unroll
+  for (int k = 0; k < 2 * NDIM; k++) m[k] = redv[k];
+  m[2 * NDIM] = (double)numax;
+  block_max_atomic<2 * NDIM + 1>(m, red_line(a.acc), red_line(a.acc) + kRedVisc);
 }
 
 // segment length along K: whole lines unless that leaves fewer than 2048
@@ -568,6 +591,31 @@ void launch_stage1(const FinalArgs& a, hipStream_t st) {
   if (a.g.ndir == 1) launch_stage1_nd<1>(a, st);
   else if (a.g.ndir == 2) launch_stage1_nd<2>(a, st);
   else launch_stage1_nd<3>(a, st);
+}
+
+template <int NDIM, int NDIR, typename S, typename C>
+static void launch_stage_t(const FinalArgs& a, hipStream_t st) {
+  // xcd_block8 needs a multiple of 8 blocks
+  const dim3 nb((unsigned)((tile::nblocks(a.g) + 7) / 8 * 8)), bs(tile::NT);
+  if (a.divbfix) {
+    if (a.w1) hipLaunchKernelGGL((k_stage<NDIM, NDIR, S, C, true, true>), nb, bs, 0, st, a);
+    else hipLaunchKernelGGL((k_stage<NDIM, NDIR, S, C, false, true>), nb, bs, 0, st, a);
+  } else {
+    if (a.w1) hipLaunchKernelGGL((k_stage<NDIM, NDIR, S, C, true, false>), nb, bs, 0, st, a);
+    else hipLaunchKernelGGL((k_stage<NDIM, NDIR, S, C, false, false>), nb, bs, 0, st, a);
+  }
+}
+
+int stage_tiles_fit(const GridDesc& g) { return SAC_LINE_TILES && tile::rows_fit(g.st[1]) ? 1 : 0; }
+
+void launch_stage(const FinalArgs& a, hipStream_t st) {
+  if (a.prec == PREC_MIXED) {
+    if (a.g.ndir == 2) launch_stage_t<2, 2, float, float>(a, st);
+    else launch_stage_t<2, 3, float, float>(a, st);
+  } else {
+    if (a.g.ndir == 2) launch_stage_t<2, 2, double, double>(a, st);
+    else launch_stage_t<2, 3, double, double>(a, st);
+  }
 }
 
 void launch_plane(const AxisArgs& a, hipStream_t st) {

@@ -93,6 +93,12 @@ __global__ void __launch_bounds__(256) k_resist(ResistArgs a) {
   const double eta = a.eta;
   const int ib = 2 + NDIR, ie = 1 + NDIR;  // R index of b_1 and of e
   auto Jk = [&](int k, long long i) { return a.J[(long long)(k - 1) * fs + i]; };
+  // the rate so far; in a fresh R the sources are all there is
+  auto Rold = [&](long long i) { return a.fresh ? 0.0 : (double)R[i]; };
+  if (a.fresh) {
+#pragma unroll
+    for (int n = 0; n <= NDIR; n++) R[(long long)n * fs + ic] = (S)0;
+  }
   double de = 0.0;
   if (!a.compact) {
 #pragma unroll
@@ -110,7 +116,7 @@ __global__ void __launch_bounds__(256) k_resist(ResistArgs a) {
           acc = (l == 1) ? acc - gr : acc + gr;
         }
       const long long ir = (long long)(ib + i - 1) * fs + ic;
-      R[ir] = (S)((double)R[ir] + acc);
+      R[ir] = (S)(Rold(ir) + acc);
     }
 #pragma unroll
     for (int idir = 1; idir <= NDIM; idir++)
@@ -139,7 +145,7 @@ __global__ void __launch_bounds__(256) k_resist(ResistArgs a) {
       }
       lap = lap * eta;
       const long long ir = (long long)(ib + i - 1) * fs + ic;
-      R[ir] = (S)((double)R[ir] + lap);
+      R[ir] = (S)(Rold(ir) + lap);
       de += lap * q0;
     }
     double j2 = 0.0;
@@ -148,7 +154,7 @@ __global__ void __launch_bounds__(256) k_resist(ResistArgs a) {
     de += eta * j2;
   }
   const long long ir = (long long)ie * fs + ic;
-  R[ir] = (S)((double)R[ir] + de);
+  R[ir] = (S)(Rold(ir) + de);
 }
 
 template <int NDIM, int NDIR, typename S>

@@ -1,0 +1,552 @@
+// sac_tile.h -- an RK stage's x and y work and its register update on 16 x 16
+// tiles staged in LDS: whole stages of 2-D grids and patches, and the last
+// pass of 3-D stages.
+//
+// The work per mesh cell is that of the line tiles (sac_line.h) along x and
+// y with the same arithmetic per value -- 4th-order flux divergence with the
+// background energy terms (centdiff4, src/vaccd.t:35-70), Powell's sources,
+// setnu for the 2*ndim+1 variables of each axis (src/vacusr.viscosity.t:
+// 224-455), the hyperdiffusion line terms and the cross-term factors
+// (src/vacusr.viscosity.t:2-221) -- then the cross terms between x and y,
+//   m_1 += d_x(rho_t Tm_{1,0}), e += d_x(m_1 Tm_{1,0}), b_1 -= d_x(Tb_{1,0}), e -= d_x(b_1 Tb_{1,0})
+//   m_0 += d_y(rho_t Tm_{0,1}), e += d_y(m_0 Tm_{0,1}), b_0 -= d_y(Tb_{0,1}), e -= d_y(b_0 Tb_{0,1})
+// (central differences, zero at a non-periodic edge, T = 0 outside the
+// mesh), the rate of other kernels (f.R: the z work, resistivity), gravity,
+// and the update with the cmax of the result (update_cells).  Neither the
+// rate of x and y nor T_{0,1}, T_{1,0} leave the CU.
+//
+// Schedule.  A block of 512 threads owns a tile of one plane.  Each thread
+// loads and evaluates one point of the 22 x 22 around it (the corners that
+// nothing reads left out): 13 fields, coalesced along x, into setnu's q
+// values, rho_t, m and the x and y fluxes in LDS.  After one barrier the
+// lower four wavefronts do the x work of the 256 cells and the upper four
+// the y work at the same time; the y rates and the factors are handed over
+// through the space of the fluxes, and the lower four finish the cells.
+// What bounds such a tile is latency: its FP64 chains are long, and its LDS
+// (75 KB in 3-D) lets two blocks into a CU.  Two axes on twice the
+// wavefronts halve the chain and give four wavefronts per SIMD instead of
+// two.  A 2-D stage of 501 x 299 cells was an x and a y line kernel and an
+// update, 19.8 + 16.3 + 15.5 us; here 21.7.  Reading the cell's background,
+// c_tot and dx before the points, and the base register while the axes are
+// handed over, took that from 24.2 (512 patches: 0.83 -> 0.71 ms).  VALU issue
+// is 350 of the 706 us of 512 patches, the rest waits.
+//
+// Grid edges follow the line tiles: a point beyond the grid along x (y) is
+// the mirror cell 6 inward (src/vacusr.viscosity.t:378-400), read only by
+// the x (y) work of cells in the grid.
+#pragma once
+#include "sac_device.h"
+
+namespace sac {
+namespace tile {
+
+constexpr int TX = 16, TY = 16, HALO = 3;
+constexpr int PX = TX + 2 * HALO, PY = TY + 2 * HALO;  // 22 x 22 points
+constexpr int NC = TX * TY;  // cells, and threads of each axis
+constexpr int NT = 2 * NC;
+
+// LDS layout (elements).  q of rho', thermal energy, v_l (and b_2 in 3-D) on
+// all 22 x 22 points; b_0, which only the y work takes differences of, on
+// columns -1..16, b_1 on rows -1..16; rho_t and m_l on -1..16 both ways; the
+// x fluxes on columns -2..17 of the tile's rows, the y fluxes on rows -2..17
+// of its columns.  The flux of b_K along K is zero and has no slot; Powell's
+// sources keep b_K + bg_K in one (slot NE-1).
+//
+// In FP64, 16 lanes read one tile row of 16 doubles (128 bytes: every bank
+// once).  In FP32 a half-wave (32 lanes, served together) reads two tile
+// rows; they are rows r and r+8 (see cell_row), and every pitch is 2 (mod 4)
+// floats, so the two rows' reads fall 8 * pitch = 16 (mod 32) banks apart and
+// never share a bank.
+template <int NDIM, int NDIR, typename C, bool DIVB>
+struct Lay {
+  static constexpr bool F32 = sizeof(C) == 4;
+  static constexpr int NE = 2 + 2 * NDIR;
+  static constexpr int QP = PX;                      // pitch of the full planes
+  static constexpr int NFULL = 2 + NDIM + (NDIM == 3 ? 1 : 0);
+  static constexpr int SP = TX + 2;                  // pitch of the 18-wide planes
+  static constexpr int B0 = NFULL * PY * QP;         // [22][18]
+  static constexpr int B1 = B0 + PY * SP;            // [18][22]
+  static constexpr int RT = B1 + (TY + 2) * QP;      // [18][18]
+  static constexpr int M0 = RT + (TY + 2) * SP;      // [NDIM][18][18]
+  static constexpr int FXP = F32 ? TX + 6 : TX + 4;  // pitch of the x fluxes
+  static constexpr int FYP = F32 ? TX + 2 : TX;      // and of the y fluxes
+  static constexpr int NF = DIVB ? NE : NE - 1;
+  static constexpr int FX = M0 + NDIM * (TY + 2) * SP;  // [NF][16][FXP]
+  static constexpr int FY = FX + NF * TY * FXP;         // [NF][20][FYP]
+  static constexpr int END = FY + NF * (TY + 4) * FYP;
+  // after the fluxes are read, in their place
+  static constexpr int RY = FX;                     // y rates [NE][16][FYP]
+  static constexpr int T01 = RY + NE * TY * FYP;    // Tm_{0,1}, Tb_{0,1}: [2][18][FYP], rows -1..16
+  static constexpr int T10 = T01 + 2 * (TY + 2) * FYP;  // Tm_{1,0}, Tb_{1,0}: [2][16][18], cols -1..16
+  static_assert(T10 + 2 * TY * SP <= END, "the exchange fits the space of the fluxes");
+};
+
+template <int NDIM, int NDIR, typename C, bool DIVB>
+struct Smem {
+  C v[Lay<NDIM, NDIR, C, DIVB>::END];
+};
+
+// flux slot of field n along K
+__host__ __device__ constexpr int fslot(int ndir, int K, int n) {
+  return n > 2 + ndir + K ? n - 1 : n;
+}
+
+// tile row of thread t (0..255) of its axis: t / 16 in FP64; in FP32 lanes
+// 0-15, 16-31, 32-47, 48-63 of wave w take rows 2w, 2w+8, 2w+1, 2w+9
+template <typename C>
+__device__ __forceinline__ int cell_row(int t) {
+  if constexpr (sizeof(C) == 4)
+    return 2 * (t >> 6) + ((t >> 5) & 1) + 8 * ((t >> 4) & 1);
+  else
+    return t / TX;
+}
+
+// tiles of a plane along x (from grid column 0, so that a tile row fills
+// whole 128-byte lines) and y
+__host__ __device__ inline int ntx(const GridDesc& g) { return (g.Mhi[0] + 1 + TX - 1) / TX; }
+__host__ __device__ inline int nty(const GridDesc& g) {
+  return (g.Mhi[1] - g.Mlo[1] + 1 + TY - 1) / TY;
+}
+__host__ __device__ inline long long nblocks(const GridDesc& g) {
+  return (long long)ntx(g) * nty(g) * (g.Mhi[2] - g.Mlo[2] + 1);
+}
+// 32-bit byte offsets reach the 22 rows of a tile's points
+__host__ __device__ inline bool rows_fit(long long pitch) { return pitch < (1LL << 32) / (8 * PY); }
+
+// One cell's line terms along axis K (0 or 1) from the staged plane, as in
+// line_tile: flux divergence, background energy terms, Powell's sources,
+// setnu face ratios, hyperdiffusion line terms; returns the factors
+// T_{K,1-K} in Tm, Tb.  fget(s, d) is flux slot s at offset d along K,
+// qget(p, d) the q of setnu's variable p of axis K (rho', thermal energy,
+// v_0.., b_l (l != K)), rget(d) rho_t, mget(l, d) m_l.
+template <int NDIM, int NDIR, int K, typename S, typename C, bool DIVB, typename FG, typename QG,
+          typename RG, typename MG>
+__device__ __forceinline__ void cell_axis(const FinalArgs& f, const GridDesc& g, long long icell,
+                                          const Pt<NDIR, C>& pbg, C (&R)[2 + 2 * NDIR], int c,
+                                          double dxd, C ctk,
+                                          bool valid, C& numax, FG fget, QG qget, RG rget, MG mget,
+                                          C& Tm, C& Tb) {
+  constexpr int NE = 2 + 2 * NDIR, NP = 2 * NDIM + 1;
+  const long long fs = g.fs;
+  const double* __restrict__ Bg = f.bg;
+  const int MloK = g.Mlo[K], MhiK = g.Mhi[K];
+  const C dxk = (C)dxd, idx = (C)(1.0 / dxd);
+  {
+    const bool fluxc = c >= MloK + 2 && c <= MhiK - 2;
+    const C inv12 = idx / (C)12;
+#pragma unroll
+    for (int n = 0; n < NE; n++) {
+      if (n == 2 + NDIR + K) {
+        R[n] = 0;
+        continue;
+      }
+      const int s = fslot(NDIR, K, n);
+      C E1, e2;
+      const C D1 = two_diff(fget(s, 1), fget(s, -1), E1);
+      const C D2 = two_diff(fget(s, 2), fget(s, -2), e2);
+      R[n] = ((D2 - (C)8 * D1) + (e2 - (C)8 * E1)) * inv12;
+    }
+    const C pTb0 = (C)ptotal_bg<NDIR, C>(pbg, f.gamma);
+    const C bgk = (C)pbg.bg[K];
+    C re = 0;
+#pragma unroll
+    for (int l = 0; l < NDIM; l++) {
+      const C dv1 = qget(2 + l, 1) - qget(2 + l, -1);
+      const C dv2 = qget(2 + l, 2) - qget(2 + l, -2);
+      const C Dv = -(dv2 - (C)8 * dv1) * inv12;
+      if (l == K) re -= Dv * pTb0;
+      re += bgk * (C)pbg.bg[l] * Dv;
+    }
+    R[1 + NDIR] += re;
+#pragma unroll
+    for (int n = 0; n < NE; n++) R[n] = fluxc ? R[n] : (C)0;
+    // Powell's div B sources (see line_tile)
+    if (DIVB && fluxc && valid) {
+      const S* __restrict__ Wf = (const S*)f.wct;
+      const C D1b = fget(NE - 1, 1) - fget(NE - 1, -1);
+      const C D2b = fget(NE - 1, 2) - fget(NE - 1, -2);
+      const C gK = -((D2b - (C)8 * D1b) * inv12);
+      const double rt = (double)Wf[icell] + Bg[fs + icell];
+      double sm = 0.0;
+#pragma unroll
+      for (int cd = 0; cd < NDIR; cd++) {
+        const double m = (double)Wf[(1 + cd) * fs + icell];
+        const double bt = (double)Wf[(2 + NDIR + cd) * fs + icell] + Bg[(2 + cd) * fs + icell];
+        R[1 + cd] -= (C)bt * gK;
+        R[2 + NDIR + cd] -= (C)(m / rt) * gK;
+        sm = (cd == 0) ? m * bt : sm + m * bt;
+      }
+      R[1 + NDIR] -= (C)(sm / rt) * gK;
+    }
+  }
+  if (f.visc_on) {
+#pragma clang fp contract(off)
+    const bool z1 = (c == MloK && !g.per_lo[K]) || (c == MhiK && !g.per_hi[K]);
+    const C rtm = rget(-1), rt0 = rget(0), rtp = rget(1);
+    const C rhoL = (rt0 + rtm) * (C)0.5, rhoR = (rtp + rt0) * (C)0.5;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      C q[7];
+#pragma unroll
+      for (int s = 0; s < 7; s++) q[s] = qget(p, s - 3);
+      C ratL, ratR;
+      face_pair<C>(q, ratL, ratR);
+      const C ch = (p >= 2 && p < 2 + NDIM) ? (C)0.4 : (C)0.04;
+      const C Kc = ctk * ch;
+      const C nuL = Kc * ratL * dxk;
+      const C nuR = Kc * ratR * dxk;
+      numax = valid ? fmax(numax, fmax(nuR, nuL)) : numax;
+      const C qm = q[2], q0 = q[3], qp = q[4];
+      const C gL = z1 ? (C)0 : (q0 - qm) * idx;
+      const C gR = z1 ? (C)0 : (qp - q0) * idx;
+      const C tL = nuL * gL, tR = nuR * gR;
+      if (p == 0) {
+        R[0] += (tR - tL) * idx;
+      } else if (p == 1) {
+        R[1 + NDIR] += (tR - tL) * idx;
+      } else if (p < 2 + NDIM) {
+        const int l = p - 2;
+        const C m0 = mget(l, 0);
+        const C mL = (m0 + mget(l, -1)) * (C)0.5;
+        const C mR = (mget(l, 1) + m0) * (C)0.5;
+        const C mult = (l == K) ? (C)1 : (C)0.5;  // the i==k branch runs twice for l==k
+        R[1 + l] += mult * (rhoR * tR - rhoL * tL) * idx;
+        R[1 + NDIR] += mult * (mR * tR - mL * tL) * idx;
+        if (l == 1 - K) {
+          const C gC = z1 ? (C)0 : (qp - qm) * idx * (C)0.5;
+          Tm = gC * (nuL + nuR) * (C)0.25;
+        }
+      } else {
+        const int n = p - 2 - NDIM;
+        const int lb = (n < K) ? n : n + 1;
+        const C BL = (q0 + qm) * (C)0.5, BR = (qp + q0) * (C)0.5;
+        R[2 + NDIR + lb] += (tR - tL) * idx;
+        R[1 + NDIR] += (tR * BR - tL * BL) * idx;
+        if (lb == 1 - K) {
+          const C gC = z1 ? (C)0 : (qp - qm) * idx * (C)0.5;
+          Tb = gC * (nuL + nuR) * (C)0.5;
+        }
+      }
+    }
+  }
+}
+
+// The factor T_{K,1-K} of one halo cell for one of its two variables (which
+// 0: the velocity, 1: the field), from q[0..6] along K; the same arithmetic
+// as cell_axis.
+template <typename C>
+__device__ __forceinline__ C cross_factor(const C (&q)[7], int which, bool z1, double dxd, C ctk) {
+#pragma clang fp contract(off)
+  const C dxk = (C)dxd, idx = (C)(1.0 / dxd);
+  const C Kc = ctk * (which ? (C)0.04 : (C)0.4);
+  C ratL, ratR;
+  face_pair<C>(q, ratL, ratR);
+  const C nuL = Kc * ratL * dxk;
+  const C nuR = Kc * ratR * dxk;
+  const C gC = z1 ? (C)0 : (q[4] - q[2]) * idx * (C)0.5;
+  return gC * (nuL + nuR) * (which ? (C)0.5 : (C)0.25);
+}
+
+// The stage of the tile with its first cell at grid column x0 and row y0 of
+// plane z.  True for the threads that stored a cell (at c).  Off: the type of
+// the points' byte offsets (see rows_fit).
+template <int NDIM, int NDIR, typename S, typename C, bool RK4L, bool DIVB, typename Off = unsigned>
+__device__ __forceinline__ bool stage_tile(const FinalArgs& f, const GridDesc& g, int x0, int y0,
+                                           int z, C* __restrict__ sm, C& numax,
+                                           double (&redv)[2 * NDIM], int (&c)[3]) {
+  using L = Lay<NDIM, NDIR, C, DIVB>;
+  constexpr int NE = L::NE;
+  const long long fs = g.fs;
+  const long long zoff = (long long)z * g.st[2];
+  const int tid = (int)threadIdx.x;
+  const bool xgrp = tid < NC;  // uniform over a wavefront
+  const int t = tid & (NC - 1);
+  const int tx = t % TX, ty = cell_row<C>(t);
+
+  // ---- the thread's cell ----
+  const int cx = x0 + tx, cy = y0 + ty;
+  const bool valid = cx >= g.Mlo[0] && cx <= g.Mhi[0] && cy <= g.Mhi[1];
+  const int cxc = (cx > g.G[0] - 1) ? g.G[0] - 1 : cx;
+  const int cyc = (cy > g.G[1] - 1) ? g.G[1] - 1 : cy;
+  const long long icell = zoff + (long long)cyc * g.st[1] + cxc;
+  const double dxx = f.dx[0][cxc], dxy = f.dx[1][cyc];
+  const C ctk = f.visc_on ? (C)red_get(f.ctot_src, xgrp ? 0 : 1) : (C)0;
+  Pt<NDIR, C> own;  // the cell's background
+  own.eb = f.bg[icell];
+  own.rhob = f.bg[fs + icell];
+#pragma unroll
+  for (int cd = 0; cd < NDIR; cd++) own.bg[cd] = f.bg[(2 + cd) * fs + icell];
+  const bool xlo = !g.per_lo[0], xhi = !g.per_hi[0], ylo = !g.per_lo[1], yhi = !g.per_hi[1];
+
+  // ---- one point per thread: the tile's cells, then the halo ----
+  {
+    int ix, iy;
+    bool point = true, fx = true, fy = true;
+    if (xgrp) {
+      ix = tx + HALO;
+      iy = ty + HALO;
+    } else if (t < 96) {  // columns -3..-1 and 16..18 of the tile's rows
+      const int r = t / 6, k = t - 6 * r;
+      ix = k < 3 ? k : k + TX;
+      iy = r + HALO;
+      fy = false;
+      fx = ix >= 1 && ix <= PX - 2;
+    } else if (t < 192) {  // rows -3..-1 and 16..18 of its columns
+      const int k = (t - 96) / TX;
+      ix = (t - 96) % TX + HALO;
+      iy = k < 3 ? k : k + TY;
+      fx = false;
+      fy = iy >= 1 && iy <= PY - 2;
+    } else {  // of the corners what the factors of the halo rows and columns take
+      const int u = t - 192;
+      fx = fy = false;
+      point = u < 20;
+      if (u < 12) {
+        const int k = u % 6;
+        ix = k < 3 ? k : k + TX;
+        iy = u < 6 ? HALO - 1 : TY + HALO;
+      } else {
+        const int k = u & 3;
+        ix = u < 16 ? HALO - 1 : TX + HALO;
+        iy = k < 2 ? k : k + TY + 2;
+      }
+    }
+    if (point) {
+      int gx = x0 - HALO + ix, gy = y0 - HALO + iy;
+      // mirror layer beyond the grid (used only along its own axis)
+      if (gx < 0) gx = g.Mlo[0] + 3;
+      if (gx > g.G[0] - 1) gx = g.Mhi[0] - 3;
+      if (gy < 0) gy = g.Mlo[1] + 3;
+      if (gy > g.G[1] - 1) gy = g.Mhi[1] - 3;
+      // offsets from the tile's first row (a mirrored row lies in the tile too)
+      const int yb = y0 > HALO ? y0 - HALO : 0;
+      const long long ob0 = zoff + yb * g.st[1];
+      const Off i = (Off)(gy - yb) * (Off)g.st[1] + (Off)gx;
+      const char* __restrict__ Wp = (const char*)((const S*)f.wct + ob0);
+      const char* __restrict__ Bp = (const char*)(f.bg + ob0);
+      const Off ow = i * (Off)sizeof(S), ob = i * (Off)8;
+      auto wv = [&](int n) { return (C) * (const S*)(Wp + (size_t)n * fs * sizeof(S) + ow); };
+      auto bv = [&](int n) { return *(const double*)(Bp + (size_t)n * fs * 8 + ob); };
+      Pt<NDIR, C> p;
+      p.rho = wv(0);
+#pragma unroll
+      for (int cd = 0; cd < NDIR; cd++) p.m[cd] = wv(1 + cd);
+      p.e = wv(1 + NDIR);
+#pragma unroll
+      for (int cd = 0; cd < NDIR; cd++) p.b[cd] = wv(2 + NDIR + cd);
+      p.eb = bv(0);
+      p.rhob = bv(1);
+#pragma unroll
+      for (int cd = 0; cd < NDIR; cd++) p.bg[cd] = bv(2 + cd);
+      if (fx) {
+        C F[NE], v[1];
+        flux_pt<NDIR, 1, C>(p, 0, f.gamma, F, v);
+        C* o = sm + L::FX + (iy - HALO) * L::FXP + ix - 1;
+#pragma unroll
+        for (int n = 0; n < NE; n++)
+          if (n != 2 + NDIR) o[fslot(NDIR, 0, n) * TY * L::FXP] = F[n];
+        if constexpr (DIVB) o[(NE - 1) * TY * L::FXP] = (C)((double)p.b[0] + p.bg[0]);
+      }
+      if (fy) {
+        C F[NE], v[1];
+        flux_pt<NDIR, 1, C>(p, 1, f.gamma, F, v);
+        C* o = sm + L::FY + (iy - 1) * L::FYP + ix - HALO;
+#pragma unroll
+        for (int n = 0; n < NE; n++)
+          if (n != 3 + NDIR) o[fslot(NDIR, 1, n) * (TY + 4) * L::FYP] = F[n];
+        if constexpr (DIVB) o[(NE - 1) * (TY + 4) * L::FYP] = (C)((double)p.b[1] + p.bg[1]);
+      }
+      {
+#pragma clang fp contract(off)
+        const double rtd = (double)p.rho + p.rhob;
+        const double inv = recip<C>(rtd);
+        double sb = 0.0, smm = 0.0;
+#pragma unroll
+        for (int cd = 0; cd < NDIR; cd++) {
+          const double mc = (double)p.m[cd], bc = (double)p.b[cd];
+          sb += bc * bc;
+          smm += mc * mc;
+        }
+        C* q = sm + iy * L::QP + ix;
+        q[0] = p.rho;
+        q[PY * L::QP] = (C)((double)p.e - 0.5 * (sb + smm * inv));
+#pragma unroll
+        for (int l = 0; l < NDIM; l++) q[(2 + l) * PY * L::QP] = p.m[l] * (C)inv;
+        if constexpr (NDIM == 3) q[5 * PY * L::QP] = p.b[2];
+        const bool inx = ix >= HALO - 1 && ix <= TX + HALO, iny = iy >= HALO - 1 && iy <= TY + HALO;
+        if (inx) sm[L::B0 + iy * L::SP + ix - (HALO - 1)] = p.b[0];
+        if (iny) sm[L::B1 + (iy - (HALO - 1)) * L::QP + ix] = p.b[1];
+        if (inx && iny) {
+          C* r = sm + L::RT + (iy - (HALO - 1)) * L::SP + ix - (HALO - 1);
+          r[0] = (C)rtd;
+#pragma unroll
+          for (int l = 0; l < NDIM; l++) r[(1 + l) * (TY + 2) * L::SP] = p.m[l];
+        }
+      }
+    }
+  }
+
+  const C* qc = sm + (ty + HALO) * L::QP + tx + HALO;       // full planes
+  const C* rc = sm + L::RT + (ty + 1) * L::SP + tx + 1;     // 18 x 18 planes
+  const C* b0 = sm + L::B0 + (ty + HALO) * L::SP + tx + 1;  // b_0
+  const C* b1 = sm + L::B1 + (ty + 1) * L::QP + tx + HALO;  // b_1
+  constexpr int QA = PY * L::QP, RA = (TY + 2) * L::SP;     // array strides
+  __syncthreads();
+
+  C R[1][NE], Tm = 0, Tb = 0, Th = 0;
+  if (xgrp) {
+    const C* fc = sm + L::FX + ty * L::FXP + tx + 2;
+    cell_axis<NDIM, NDIR, 0, S, C, DIVB>(
+        f, g, icell, own, R[0], cx, dxx, ctk, valid, numax,
+        [&](int s, int d) { return fc[s * TY * L::FXP + d]; },
+        [&](int p, int d) {
+          return p < 2 + NDIM ? qc[p * QA + d] : (p == 2 + NDIM ? b1[d] : qc[5 * QA + d]);
+        },
+        [&](int d) { return rc[d]; }, [&](int l, int d) { return rc[(1 + l) * RA + d]; }, Tm, Tb);
+    // T_{0,1} of the rows below and above the tile, one variable per lane
+    if (f.visc_on && t >= NC - 64) {
+      const int hx = t & 15, hy = (t & 16) ? TY : -1, which = (t >> 5) & 1;
+      const int hcx = x0 + hx, hcxc = (hcx > g.G[0] - 1) ? g.G[0] - 1 : hcx;
+      const C* a = which ? sm + L::B1 + (hy + 1) * L::QP + hx + HALO
+                         : sm + 3 * QA + (hy + HALO) * L::QP + hx + HALO;
+      C q[7];
+#pragma unroll
+      for (int s = 0; s < 7; s++) q[s] = a[s - 3];
+      const bool z1 = (hcx == g.Mlo[0] && xlo) || (hcx == g.Mhi[0] && xhi);
+      Th = cross_factor<C>(q, which, z1, f.dx[0][hcxc], ctk);
+    }
+  } else {
+    const C* fc = sm + L::FY + (ty + 2) * L::FYP + tx;
+    cell_axis<NDIM, NDIR, 1, S, C, DIVB>(
+        f, g, icell, own, R[0], cy, dxy, ctk, valid, numax,
+        [&](int s, int d) { return fc[(s * (TY + 4) + d) * L::FYP]; },
+        [&](int p, int d) {
+          return p < 2 + NDIM ? qc[p * QA + d * L::QP]
+                              : (p == 2 + NDIM ? b0[d * L::SP] : qc[5 * QA + d * L::QP]);
+        },
+        [&](int d) { return rc[d * L::SP]; },
+        [&](int l, int d) { return rc[(1 + l) * RA + d * L::SP]; }, Tm, Tb);
+    // T_{1,0} of the columns left and right of the tile
+    if (f.visc_on && t >= NC - 64) {
+      const int hy = t & 15, hx = (t & 16) ? TX : -1, which = (t >> 5) & 1;
+      const int hcy = y0 + hy, hcyc = (hcy > g.G[1] - 1) ? g.G[1] - 1 : hcy;
+      const C* a = which ? sm + L::B0 + (hy + HALO) * L::SP + hx + 1
+                         : sm + 2 * QA + (hy + HALO) * L::QP + hx + HALO;
+      const int st = which ? L::SP : L::QP;
+      C q[7];
+#pragma unroll
+      for (int s = 0; s < 7; s++) q[s] = a[(s - 3) * st];
+      const bool z1 = (hcy == g.Mlo[1] && ylo) || (hcy == g.Mhi[1] && yhi);
+      Th = cross_factor<C>(q, which, z1, f.dx[1][hcyc], ctk);
+    }
+  }
+  // The rate of other kernels, the z factors of the cell's neighbours and the
+  // base register: on their way while the axes are handed over.
+  C Rin[NE], Tz[8];
+  S base[NE];
+  if (xgrp) {
+#pragma unroll
+    for (int n = 0; n < NE; n++) base[n] = ((const S*)f.base)[n * fs + icell];
+  }
+  if (xgrp && f.R) {
+#pragma unroll
+    for (int n = 0; n < NE; n++) Rin[n] = (C)((const S*)f.R)[n * fs + icell];
+  }
+  if constexpr (NDIM == 3) {
+    if (xgrp && f.visc_on) {
+      // in-grid indices: the neighbours of a mesh cell
+      const long long ex = valid ? 1 : 0, ey = valid ? g.st[1] : 0;
+      const S* __restrict__ T0 = (const S*)f.T + (long long)cross_index(NDIM, 2, 0) * fs + icell;
+      const S* __restrict__ T1 = (const S*)f.T + (long long)cross_index(NDIM, 2, 1) * fs + icell;
+      Tz[0] = (C)T0[ex], Tz[1] = (C)T0[-ex], Tz[2] = (C)T0[fs + ex], Tz[3] = (C)T0[fs - ex];
+      Tz[4] = (C)T1[ey], Tz[5] = (C)T1[-ey], Tz[6] = (C)T1[fs + ey], Tz[7] = (C)T1[fs - ey];
+    }
+  }
+  __syncthreads();  // the fluxes are read; their space takes the exchange
+  if (xgrp) {
+    sm[L::T01 + (ty + 1) * L::FYP + tx] = Tm;
+    sm[L::T01 + ((TY + 2) + ty + 1) * L::FYP + tx] = Tb;
+    if (t >= NC - 64)
+      sm[L::T01 + (((t >> 5) & 1) * (TY + 2) + ((t & 16) ? TY + 1 : 0)) * L::FYP + (t & 15)] = Th;
+  } else {
+#pragma unroll
+    for (int n = 0; n < NE; n++) sm[L::RY + (n * TY + ty) * L::FYP + tx] = R[0][n];
+    sm[L::T10 + ty * L::SP + tx + 1] = Tm;
+    sm[L::T10 + (TY + ty) * L::SP + tx + 1] = Tb;
+    if (t >= NC - 64)
+      sm[L::T10 + (((t >> 5) & 1) * TY + (t & 15)) * L::SP + ((t & 16) ? TX + 1 : 0)] = Th;
+  }
+  __syncthreads();
+  if (!xgrp || !valid) return false;
+
+#pragma unroll
+  for (int n = 0; n < NE; n++) R[0][n] = R[0][n] + sm[L::RY + (n * TY + ty) * L::FYP + tx];
+  if (f.R) {
+#pragma unroll
+    for (int n = 0; n < NE; n++) R[0][n] = R[0][n] + Rin[n];
+  }
+  if (f.visc_on) {
+    // cross terms with derivatives along l of the factors made along k
+    const C* t10 = sm + L::T10 + ty * L::SP + tx + 1;
+    const C* t01 = sm + L::T01 + (ty + 1) * L::FYP + tx;
+#pragma unroll
+    for (int l = 0; l < 2; l++) {
+      const int cl = (l == 0) ? cx : cy;
+      const bool edge = (l == 0) ? ((cx == g.Mlo[0] && xlo) || (cx == g.Mhi[0] && xhi))
+                                 : ((cy == g.Mlo[1] && ylo) || (cy == g.Mhi[1] && yhi));
+      const C h = (C)(0.5 / ((l == 0) ? dxx : dxy));
+      const bool inP = cl + 1 <= g.Mhi[l], inM = cl - 1 >= g.Mlo[l];
+      const int rs = (l == 0) ? 1 : L::SP;  // neighbour along l in the 18-wide planes
+      const int qs = (l == 0) ? 1 : L::QP;
+      const C rtp = rc[rs], rtm = rc[-rs];
+#pragma unroll
+      for (int k = 0; k < NDIM; k++) {
+        if (k == l) continue;
+        C Tmp0, Tmm0, Tbp0, Tbm0, bkp, bkm;
+        if (k == 2) {
+          Tmp0 = Tz[4 * l], Tmm0 = Tz[4 * l + 1], Tbp0 = Tz[4 * l + 2], Tbm0 = Tz[4 * l + 3];
+          bkp = qc[5 * QA + qs], bkm = qc[5 * QA - qs];
+        } else if (l == 0) {
+          Tmp0 = t10[1], Tmm0 = t10[-1], Tbp0 = t10[TY * L::SP + 1], Tbm0 = t10[TY * L::SP - 1];
+          bkp = b1[1], bkm = b1[-1];
+        } else {
+          Tmp0 = t01[L::FYP], Tmm0 = t01[-L::FYP];
+          Tbp0 = t01[(TY + 3) * L::FYP], Tbm0 = t01[(TY + 1) * L::FYP];
+          bkp = b0[L::SP], bkm = b0[-L::SP];
+        }
+        const C Tmp = inP ? Tmp0 : (C)0, Tmm = inM ? Tmm0 : (C)0;
+        const C Tbp = inP ? Tbp0 : (C)0, Tbm = inM ? Tbm0 : (C)0;
+        const C mkp = rc[(1 + k) * RA + rs], mkm = rc[(1 + k) * RA - rs];
+        const C dm = (rtp * Tmp - rtm * Tmm) * h;
+        const C de1 = (mkp * Tmp - mkm * Tmm) * h;
+        const C db = (Tbp - Tbm) * h;
+        const C de2 = (Tbp * bkp - Tbm * bkm) * h;
+        R[0][1 + k] += edge ? (C)0 : dm;
+        R[0][1 + NDIR] += edge ? (C)0 : de1;
+        R[0][2 + NDIR + k] -= edge ? (C)0 : db;
+        R[0][1 + NDIR] -= edge ? (C)0 : de2;
+      }
+    }
+  }
+  c[0] = cx;
+  c[1] = cy;
+  c[2] = z;
+  // gravity on rho' (gravity_cells), with m_d/rho_t from setnu's q of v_d
+  {
+    const C rho = qc[0];
+    C rg = 0;
+#pragma unroll
+    for (int d = 0; d < NDIM; d++) {
+      const bool on = f.grav_on[d] != 0;
+      const C gr = (C)f.grav[d] * rho;
+      R[0][1 + d] = on ? R[0][1 + d] + gr : R[0][1 + d];
+      rg = on ? rg + gr * qc[(2 + d) * QA] : rg;
+    }
+    R[0][1 + NDIR] += rg;
+  }
+  update_cell<NDIM, NDIR, S, C, RK4L>(f, g, c, icell, base, own, R[0], redv);
+  return true;
+}
+
+}  // namespace tile
+}  // namespace sac
