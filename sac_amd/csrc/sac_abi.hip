@@ -105,7 +105,9 @@ struct Dev {
   void* rate = nullptr;     // R accumulator
   void* cross = nullptr;    // cross-term factors T
   void* snap = nullptr;     // 'fixed' values of the evolving fields
-  double* dx[3] = {nullptr, nullptr, nullptr};
+  double* dx[3] = {nullptr, nullptr, nullptr};  // in dx_all: kDxTables tables of dxs values
+  double* dx_all = nullptr;
+  long long dxs = 0;
   unsigned long long* red = nullptr;  // [kSlots+1][kRedSlots], then the reduction lines
   // the words of W and maxviscoef in pinned host memory, written by the
   // kernel that combines them at the end of a stage into W; posted: they are
@@ -152,8 +154,16 @@ int balloc(Dev& d, void** p, size_t bytes) {
 int dalloc(Dev& d, double** p, long long nelem) {
   return balloc(d, (void**)p, sizeof(double) * (size_t)nelem);
 }
-// nelem elements of the storage precision
-int ealloc(Dev& d, void** p, long long nelem) { return balloc(d, p, d.esz * (size_t)nelem); }
+// `nfield` fields of the grid in elements of `esz` bytes (kFieldPad)
+int falloc(Dev& d, void** p, int nfield, size_t esz) {
+  const long long n = (long long)nfield * d.g.fs + sac::kFieldPad + sac::kFieldPadEnd;
+  if (int rc = balloc(d, p, esz * (size_t)n)) return rc;
+  *p = (char*)*p + esz * sac::kFieldPad;
+  return 0;
+}
+void ffree(void* p, size_t esz) {
+  if (p) hipFree((char*)p - esz * sac::kFieldPad);
+}
 
 unsigned long long* red_of(Dev& d, int slot) { return d.red + (size_t)slot * sac::kRedSlots; }
 unsigned long long* red_visc(Dev& d) { return d.red + (size_t)kSlots * sac::kRedSlots; }
@@ -295,6 +305,7 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   x.wct = d.reg[wct];
   x.bg = d.bg;
   for (int k = 0; k < 3; k++) x.dx[k] = d.dx[k];
+  x.dxs = d.dxs;
   x.R = d.rate;
   x.T = d.cross;
   x.gamma = d.gamma;
@@ -303,26 +314,24 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   x.acc = red_acc(d);
   const bool learned = d.cl && d.cl->on;
   int skip_last = 0;
-  // plane tiles: the x and y work (and their cross terms) in one launch,
-  // then the z line tiles (which add the z cross terms), then k_final
-  const bool plane = d.plane && d.ndim == 3 && !learned && !d.divbfix && sac::line_tiles_built();
-  if (plane) {
-    x.xcd = d.xcd;
-    x.RF = nullptr;
-    x.cross_last = 0;
-    x.divbfix = 0;
-    hipEvent_t e0{};
-    t_begin(d, SAC_K_PLANE, &e0);
-    sac::launch_plane(x, d.stream);
-    t_end(d, SAC_K_PLANE, e0);
-  }
   // 1-D FP64: the whole stage in one launch (below), unless the resistive
   // sources have to join the rate first
   const bool stage1 = d.ndim == 1 && d.prec == SAC_PREC_FP64 && !learned && !(d.eta > 0.0) &&
                       sac::line_tiles_built();
   // 2-D: the same, with the resistive sources handed over in R
-  const bool stage2 = d.plane && d.ndim == 2 && !learned && sac::stage_tiles_fit(d.g);
-  for (int k = plane ? 2 : 0; k < d.ndim && !stage1 && !stage2; k++) {
+  const bool tiles = d.plane && d.ndim > 1 && !learned && sac::stage_tiles_fit(d.g);
+  const bool stage2 = tiles && d.ndim == 2;
+  // 3-D: the factors for z, then the z line tiles (which add the z cross
+  // terms), then the x and y work and the update in one launch
+  const bool stage3 = tiles && d.ndim == 3;
+  if (stage3 && d.visc_on) {
+    hipEvent_t e0{};
+    t_begin(d, SAC_K_PLANE, &e0);
+    sac::launch_tz(x, d.stream);
+    t_end(d, SAC_K_PLANE, e0);
+  }
+  x.fresh = stage3 ? 1 : 0;
+  for (int k = stage3 ? 2 : 0; k < d.ndim && !stage1 && !stage2; k++) {
     // axis 1 (rows of a plane): neighbour rows in one XCD's L2.  Axes 0 and 2
     // keep the hardware order, whose round-robin already places the
     // neighbour planes of a row in the same XCD.
@@ -364,6 +373,7 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   s.wct = d.reg[wct];
   s.bg = d.bg;
   for (int k = 0; k < 3; k++) s.dx[k] = d.dx[k];
+  s.dxs = d.dxs;
   s.R = d.rate;
   s.T = d.cross;
   s.base = d.reg[base];
@@ -383,14 +393,13 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   s.ctot_src = x.ctot_src;
   s.xcd = 1;
   s.skip_last = skip_last;
-  s.skip_xy = plane ? 1 : 0;
   hipEvent_t e0{};
   t_begin(d, SAC_K_FINAL, &e0);
   if (stage1) {
     sac::launch_stage1(s, d.stream);
-  } else if (stage2) {
+  } else if (tiles) {
     s.divbfix = d.divbfix;
-    if (!(d.eta > 0.0)) s.R = nullptr;
+    if (stage2 && !(d.eta > 0.0)) s.R = nullptr;
     sac::launch_stage(s, d.stream);
   } else {
     sac::launch_final(s, d.stream);
@@ -585,7 +594,8 @@ int sac_dev_init(int ndim, int ndir, const int* nx, int nw, const int* iws, int 
     ncg *= g.G[k];
   }
   d->ncell_grid = ncg;
-  const int pitch = (g.G[0] + 15) / 16 * 16;  // 128-byte rows
+  const int ra = 128 / (int)d->esz;  // rows of whole 128-byte lines (in evolving elements)
+  const int pitch = (g.G[0] + ra - 1) / ra * ra;
   g.st[0] = 1;
   g.st[1] = pitch;
   g.st[2] = (long long)pitch * g.G[1];
@@ -617,36 +627,38 @@ int sac_dev_init(int ndim, int ndir, const int* nx, int nw, const int* iws, int 
   };
   if (hipStreamCreate(&d->stream) != hipSuccess) return bail(fail(SAC_E_HIP, "hipStreamCreate"));
   for (int s = 0; s < kSlots; s++)
-    if ((rc = ealloc(*d, &d->reg[s], (long long)ne * g.fs))) return bail(rc);
-  if ((rc = dalloc(*d, &d->bg, (long long)d->nbg * g.fs))) return bail(rc);
-  if ((rc = ealloc(*d, &d->rate, (long long)ne * g.fs))) return bail(rc);
-  if (d->eta > 0.0 && (rc = dalloc(*d, &d->J, 3LL * g.fs))) return bail(rc);
+    if ((rc = falloc(*d, &d->reg[s], ne, d->esz))) return bail(rc);
+  if ((rc = falloc(*d, (void**)&d->bg, d->nbg, sizeof(double)))) return bail(rc);
+  if ((rc = falloc(*d, &d->rate, ne, d->esz))) return bail(rc);
+  if (d->eta > 0.0 && (rc = falloc(*d, (void**)&d->J, 3, sizeof(double)))) return bail(rc);
   if (d->visc_on && ndim > 1 &&
-      (rc = ealloc(*d, &d->cross, (long long)2 * ndim * (ndim - 1) * g.fs)))
+      (rc = falloc(*d, &d->cross, 2 * ndim * (ndim - 1), d->esz)))
     return bail(rc);
   if (d->any_fixed) {
-    if ((rc = ealloc(*d, &d->snap, (long long)ne * g.fs))) return bail(rc);
+    if ((rc = falloc(*d, &d->snap, ne, d->esz))) return bail(rc);
   }
-  // dx per axis, dxmin per axis over the mesh
+  // dx per axis and its reciprocals (kDxTables), dxmin per axis over the mesh
   long long off = 0;
+  d->dxs = (long long)g.G[0] + g.G[1] + g.G[2];
+  std::vector<double> dxt((size_t)(sac::kDxTables * d->dxs), 1.0);
+  if ((rc = dalloc(*d, &d->dx_all, (long long)dxt.size()))) return bail(rc);
   for (int k = 0; k < 3; k++) {
     int n = g.G[k];
-    if ((rc = dalloc(*d, &d->dx[k], n))) return bail(rc);
+    d->dx[k] = d->dx_all + off;
     if (k < ndim) {
-      if (hipMemcpy(d->dx[k], dx + off, sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess)
-        return bail(fail(SAC_E_HIP, "dx upload"));
       double mn = kBigDouble;
       for (int i = g.Mlo[k]; i <= g.Mhi[k]; i++) {
         if (!(dx[off + i] > 0.0)) return bail(fail(SAC_E_ARG, "dx must be > 0 on the mesh"));
         mn = std::fmin(mn, dx[off + i]);
       }
       d->dxmin[k] = mn;
-      off += n;
-    } else {
-      double one = 1.0;
-      hipMemcpy(d->dx[k], &one, sizeof(double), hipMemcpyHostToDevice);
+      sac::fill_dx_tables(dxt.data() + off, d->dxs, dx + off, n);
     }
+    off += n;
   }
+  if (hipMemcpy(d->dx_all, dxt.data(), sizeof(double) * dxt.size(), hipMemcpyHostToDevice) !=
+      hipSuccess)
+    return bail(fail(SAC_E_HIP, "dx upload"));
   // boundary codes per register
   std::vector<int>& bce = d->bce_h;
   std::vector<int>& bcb = d->bcb_h;
@@ -692,13 +704,13 @@ int sac_dev_free(sac_handle h) {
   Dev* d = (Dev*)h;
   if (d->stream) hipStreamSynchronize(d->stream);
   t_collect(*d);
-  for (int s = 0; s < kSlots; s++) hipFree(d->reg[s]);
-  hipFree(d->bg);
-  hipFree(d->rate);
-  hipFree(d->cross);
-  hipFree(d->J);
-  hipFree(d->snap);
-  for (int k = 0; k < 3; k++) hipFree(d->dx[k]);
+  for (int s = 0; s < kSlots; s++) ffree(d->reg[s], d->esz);
+  ffree(d->bg, sizeof(double));
+  ffree(d->rate, d->esz);
+  ffree(d->cross, d->esz);
+  ffree(d->J, sizeof(double));
+  ffree(d->snap, d->esz);
+  hipFree(d->dx_all);
   hipFree(d->red);
   if (d->red_host) hipHostFree(d->red_host);
   if (d->cl) {

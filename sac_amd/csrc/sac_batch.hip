@@ -71,6 +71,7 @@ struct Args {
   double* reg[kSlots];
   const double* bg;
   const double* dx;          // cell widths per tube: G_x values, then G_y values
+  long long dxs;             // and their further tables (kDxInv ...)
   unsigned long long* red;   // [tube][slot][kRed]
   unsigned long long* visc;  // [tube] maxviscoef since the last dt
   double* t;
@@ -178,7 +179,7 @@ __device__ __forceinline__ void clear_red_w(const Args& a, int tube, bool first,
 // of 32-160 cells (4.8 M): 0.706 ms a stage, RK4's last 0.769; the two line
 // kernels and the update before took 0.996 and 1.155.
 template <bool RK4L, typename Off>
-__global__ void __launch_bounds__(tile::NT) kb_patch_stage(Args a, int wct, int base, int out,
+__global__ void __launch_bounds__(tile::NT, 4) kb_patch_stage(Args a, int wct, int base, int out,
                                                            double da) {
   __shared__ tile::Smem<2, NDIR, double, false> sm;
   // each XCD takes one contiguous range of tiles (shared halos in one L2)
@@ -187,7 +188,7 @@ __global__ void __launch_bounds__(tile::NT) kb_patch_stage(Args a, int wct, int 
   const Tile tl = a.stiles[b];
   if (a.state[tl.tube] != RUNNING) return;  // uniform over the block
   const GridDesc g = tube_grid<2>(a, tl.tube);
-  clear_red_w(a, tl.tube, tl.c0 == 0 && tl.c1 == g.Mlo[1], out);
+  clear_red_w(a, tl.tube, tl.c0 == g.Mlo[0] && tl.c1 == g.Mlo[1], out);
   const long long o = a.start[tl.tube];
   FinalArgs f{};
   f.g = g;
@@ -195,6 +196,7 @@ __global__ void __launch_bounds__(tile::NT) kb_patch_stage(Args a, int wct, int 
   f.wct = a.reg[wct] + o;
   f.bg = a.bg + o;
   f.dx[0] = a.dx + a.dxo[tl.tube];
+  f.dxs = a.dxs;
   f.dx[1] = f.dx[0] + g.G[0];
   f.base = a.reg[base] + o;
   f.out = a.reg[out] + o;
@@ -209,7 +211,7 @@ __global__ void __launch_bounds__(tile::NT) kb_patch_stage(Args a, int wct, int 
                                                                   numax, redv, c))
     cont_ghosts_of<2>(g, (double*)f.out, c);
   double r[5] = {redv[0], redv[1], redv[2], redv[3], numax};
-  block_max_atomic<5>(r, red_of(a, tl.tube, out), a.visc + tl.tube);
+  block_max_atomic<5>(r, red_of(a, tl.tube, out), a.visc + tl.tube, tile::NC / 64);
 }
 
 // Tubes: one whole RK stage of a tile of LT cells in one kernel: the x work
@@ -233,6 +235,7 @@ __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, i
   f.wct = a.reg[wct] + o;
   f.bg = a.bg + o;
   f.dx[0] = a.dx + a.dxo[tl.tube];
+  f.dxs = a.dxs;
   f.base = a.reg[base] + o;
   f.out = a.reg[out] + o;
   set_rk4<RK4L>(a, o, f);
@@ -496,14 +499,14 @@ int set_shape(Batch& b, Shape s) {
   }
   if (tiles.empty()) tiles.push_back({b.active.empty() ? 0 : b.active[0], 2, 2});
   if (b.ndim == 2) {
-    // stage tiles of each running patch, along x from grid column 0
+    // stage tiles of each running patch
     std::vector<Tile> st;
     b.rows_fit = true;
     for (int i : b.active) b.rows_fit = b.rows_fit && sac::tile::rows_fit(b.pitch[i]);
     for (int i : b.active)
       for (int c1 = 2; c1 < 2 + b.nxy[2 * i + 1]; c1 += sac::tile::TY)
-        for (int c0 = 0; c0 < 2 + b.nxy[2 * i]; c0 += sac::tile::TX) st.push_back({i, c0, c1});
-    if (st.empty()) st.push_back({b.active.empty() ? 0 : b.active[0], 0, 2});
+        for (int c0 = 2; c0 < 2 + b.nxy[2 * i]; c0 += sac::tile::TX) st.push_back({i, c0, c1});
+    if (st.empty()) st.push_back({b.active.empty() ? 0 : b.active[0], 2, 2});
     b.a.nstiles = (int)st.size();
     if (b.d_stiles) hipFree(b.d_stiles);
     b.d_stiles = nullptr;
@@ -718,9 +721,9 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   long long off = 0, doff = 0;
   for (int i = 0; i < ntubes; i++) {
     const int G0 = b->gx(i), G1 = b->gy(i);
-    b->start[i] = off;  // each tube starts on a 128-byte line
+    b->start[i] = off + sac::kFieldPad;  // each mesh row starts on a 128-byte line
     b->pitch[i] = (ndim == 1) ? G0 : (G0 + 15) / 16 * 16;
-    off += ((long long)b->pitch[i] * G1 + 15) / 16 * 16;
+    off += ((long long)b->pitch[i] * G1 + sac::kFieldPad + sac::kFieldPadEnd + 15) / 16 * 16;
     b->dxo[i] = doff;
     doff += G0 + (ndim == 2 ? G1 : 0);
     b->max_frame = std::max(b->max_frame, 4 * G0 + 4 * (G1 - 4));
@@ -732,7 +735,8 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   for (int s = 0; s < kSlots; s++)
     if ((rc = balloc(*b, (void**)&b->d_reg[s], fb * NE))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_bg, fb * NBG))) return bail(rc);
-  if ((rc = balloc(*b, (void**)&b->d_dx, sizeof(double) * (size_t)doff))) return bail(rc);
+  if ((rc = balloc(*b, (void**)&b->d_dx, sizeof(double) * (size_t)doff * sac::kDxTables)))
+    return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_start, sizeof(long long) * ntubes))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_nxy, sizeof(int) * 2 * ntubes))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_pitch, sizeof(int) * ntubes))) return bail(rc);
@@ -753,6 +757,8 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   // another; dx: G0 values (then G1 values) per tube
   std::vector<double> pk((size_t)b->fs * (NE + NBG), 0.0);
   std::vector<double> dxmin(2 * (size_t)ntubes, 1.0);
+  std::vector<double> dxt((size_t)doff * sac::kDxTables);
+  sac::fill_dx_tables(dxt.data(), doff, dx, doff);
   long long hoff = 0;
   for (int i = 0; i < ntubes; i++) {
     const int G0 = b->gx(i), G1 = b->gy(i);
@@ -775,7 +781,8 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   if (hipMemcpy(b->d_reg[SAC_SLOT_W], pk.data(), fb * NE, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(b->d_bg, pk.data() + (size_t)b->fs * NE, fb * NBG, hipMemcpyHostToDevice) !=
           hipSuccess ||
-      hipMemcpy(b->d_dx, dx, sizeof(double) * (size_t)doff, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(b->d_dx, dxt.data(), sizeof(double) * dxt.size(), hipMemcpyHostToDevice) !=
+          hipSuccess ||
       hipMemcpy(b->d_start, b->start.data(), sizeof(long long) * ntubes, hipMemcpyHostToDevice) !=
           hipSuccess ||
       hipMemcpy(b->d_nxy, b->nxy.data(), sizeof(int) * 2 * ntubes, hipMemcpyHostToDevice) !=
@@ -798,6 +805,7 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   for (int s = 0; s < kSlots; s++) a.reg[s] = b->d_reg[s];
   a.bg = b->d_bg;
   a.dx = b->d_dx;
+  a.dxs = doff;
   a.red = b->d_red;
   a.visc = b->d_visc;
   a.t = b->d_t;

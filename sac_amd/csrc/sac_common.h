@@ -18,6 +18,20 @@ constexpr int kMaxBg = 2 + kMaxDir;          // eb, rhob, bg(3)
 constexpr int kMaxPairs = 21;                // setnu (variable, direction) pairs
 constexpr int kRedSlots = 8;                 // reduction values per buffer
 
+// Cell widths come as four tables, dxs elements apart: dx, 1/dx, (1/dx)/12 and
+// 0.5/dx, so that a cell's work starts with a load instead of an FP64 division
+constexpr int kDxInv = 1, kDxInv12 = 2, kDxHalf = 3, kDxTables = 4;
+
+// the tables of n widths dx, at t, t + dxs, ...
+inline void fill_dx_tables(double* t, long long dxs, const double* dx, long long n) {
+  for (long long i = 0; i < n; i++) {
+    t[i] = dx[i];
+    t[kDxInv * dxs + i] = 1.0 / dx[i];
+    t[kDxInv12 * dxs + i] = (1.0 / dx[i]) / 12.0;
+    t[kDxHalf * dxs + i] = 0.5 / dx[i];
+  }
+}
+
 // storage precision of the evolving fields
 enum PrecCode : int { PREC_FP64 = 0, PREC_MIXED = 1 };
 
@@ -35,6 +49,14 @@ enum BcCode : int {
   BC_CONTCD4 = 10,
   BC_ZERO = 11
 };
+
+// Fields start kFieldPad elements into their allocation, so that the first
+// mesh cell of every row (grid index 2, rows padded to 16 elements, 32 where
+// elements are FP32) lies on a 128-byte line: tiles that start at the mesh
+// fill whole lines, or halves of one with their neighbour in FP32.  (Tiles
+// that start at the row start to be aligned cover two ghost columns: 9 tiles
+// for 128 cells, 3 for 31; the 128^3 stage took 8 % longer with them.)
+constexpr int kFieldPad = 30, kFieldPadEnd = 2;
 
 struct GridDesc {
   int ndim, ndir;

@@ -78,6 +78,17 @@ __device__ __forceinline__ float two_diff(float a, float b, float& err) {
   return s;
 }
 
+// a*b + c, rounded once.  Where a sum has two products, which of them a
+// compiler fuses is its choice, in each kernel anew; a tube or patch of an
+// ensemble equals the same one run as a grid bit for bit, so what both
+// evaluate (fluxes, pressure, cmax, cross terms) makes the choice itself.
+__device__ __forceinline__ double fma_(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
+__device__ __forceinline__ float fma_(float a, float b, float c) {
+  return __builtin_fmaf(a, b, c);
+}
+
 // ---------------------------------------------------------------------
 // point state: perturbation (evolving) in C, static background in FP64
 
@@ -106,59 +117,81 @@ __device__ __forceinline__ void load_pt(const S* __restrict__ W, const double* _
 // inv = 1/rho_t
 template <int NDIR, typename C>
 __device__ __forceinline__ double ptotal(const Pt<NDIR, C>& p, double gamma, double inv) {
+#pragma clang fp contract(off)
   double sbbg = 0.0, sb2 = 0.0, sm2 = 0.0;
 #pragma unroll
   for (int c = 0; c < NDIR; c++) {
     const double b = (double)p.b[c], m = (double)p.m[c];
-    sbbg += b * p.bg[c];
-    sb2 += b * b;
-    sm2 += m * m;
+    sbbg = fma_(b, p.bg[c], sbbg);
+    sb2 = fma_(b, b, sb2);
+    sm2 = fma_(m, m, sm2);
   }
-  return (gamma - 1.0) * ((double)p.e - 0.5 * sm2 * inv) - (gamma - 2.0) * (sbbg + 0.5 * sb2);
+  const double pth = fma_(-0.5 * sm2, inv, (double)p.e), pb = fma_(0.5, sb2, sbbg);
+  return fma_(gamma - 1.0, pth, -((gamma - 2.0) * pb));
 }
 
 // background total pressure (getptotal_bg, src/vacphys0.t.mhd:208-224)
 template <int NDIR, typename C>
 __device__ __forceinline__ double ptotal_bg(const Pt<NDIR, C>& p, double gamma) {
+#pragma clang fp contract(off)
   double s = 0.0;
 #pragma unroll
-  for (int c = 0; c < NDIR; c++) s += p.bg[c] * p.bg[c];
-  return (gamma - 1.0) * p.eb - 0.5 * (gamma - 2.0) * s;
+  for (int c = 0; c < NDIR; c++) s = fma_(p.bg[c], p.bg[c], s);
+  return fma_(gamma - 1.0, p.eb, -(0.5 * (gamma - 2.0) * s));
 }
 
-// full flux (non-transport part of getflux + transport v_d*w) along axis d;
-// also returns v_l = m_l/rho_t for l < NV
+// what the fluxes along every axis share; invd = 1/rho_t
+template <typename C>
+struct FluxPt {
+  C inv, pT, sbgm, sbm;
+};
+template <int NDIR, typename C>
+__device__ __forceinline__ FluxPt<C> flux_common(const Pt<NDIR, C>& p, double gamma, double invd) {
+  FluxPt<C> f;
+  f.inv = (C)invd;
+  f.pT = (C)ptotal<NDIR, C>(p, gamma, invd);
+  f.sbgm = 0;
+  f.sbm = 0;
+#pragma unroll
+  for (int c = 0; c < NDIR; c++) {
+    f.sbgm = fma_((C)p.bg[c], p.m[c], f.sbgm);
+    f.sbm = fma_(p.b[c], p.m[c], f.sbm);
+  }
+  return f;
+}
+
+// full flux (non-transport part of getflux + transport v_d*w) along axis d
+template <int NDIR, typename C>
+__device__ __forceinline__ void flux_axis(const Pt<NDIR, C>& p, const FluxPt<C>& f, int d,
+                                          C (&F)[2 + 2 * NDIR]) {
+#pragma clang fp contract(off)
+  const C inv = f.inv;
+  const C vd = p.m[d] * inv, bd = p.b[d], bgd = (C)p.bg[d];
+  F[0] = fma_((C)p.rhob * p.m[d], inv, vd * p.rho);
+#pragma unroll
+  for (int c = 0; c < NDIR; c++) {
+    // b_c bg_d + b_d bg_c + b_c b_d
+    const C t = fma_(p.b[c], bd, fma_(p.b[c], bgd, bd * (C)p.bg[c]));
+    F[1 + c] = fma_(vd, p.m[c], (c == d) ? f.pT - t : -t);
+  }
+  // (m_d p_T - b_d (bg.m) - bg_d (b.m) + eb m_d - b_d (b.m)) / rho_t + v_d e
+  const C w = fma_(-bgd, f.sbm, fma_(p.m[d], f.pT, -(bd * f.sbgm)));
+  F[1 + NDIR] = fma_(vd, p.e, fma_(-(bd * f.sbm), inv, fma_(w, inv, (C)p.eb * p.m[d] * inv)));
+#pragma unroll
+  for (int c = 0; c < NDIR; c++) {
+    F[2 + NDIR + c] =
+        (c == d) ? (C)0 : fma_(vd, p.b[c], fma_(-(p.m[c] * inv), bd + bgd, vd * (C)p.bg[c]));
+  }
+}
+
+// the same for one axis alone; also returns v_l = m_l/rho_t for l < NV
 template <int NDIR, int NV, typename C>
 __device__ __forceinline__ void flux_pt(const Pt<NDIR, C>& p, int d, double gamma,
                                         C (&F)[2 + 2 * NDIR], C (&v)[NV]) {
-  const double rt = (double)p.rho + p.rhob;
-  const double invd = recip<C>(rt);
-  const C inv = (C)invd;
-  const C vd = p.m[d] * inv;
-  F[0] = (C)p.rhob * p.m[d] * inv + vd * p.rho;
-  const C pT = (C)ptotal<NDIR, C>(p, gamma, invd);
-  C sbgm = 0, sbm = 0;
+  const FluxPt<C> f = flux_common<NDIR, C>(p, gamma, recip<C>((double)p.rho + p.rhob));
+  flux_axis<NDIR, C>(p, f, d, F);
 #pragma unroll
-  for (int c = 0; c < NDIR; c++) {
-    sbgm += (C)p.bg[c] * p.m[c];
-    sbm += p.b[c] * p.m[c];
-  }
-#pragma unroll
-  for (int c = 0; c < NDIR; c++) {
-    C f = -(p.b[c] * (C)p.bg[d] + p.b[d] * (C)p.bg[c]) - p.b[c] * p.b[d];
-    if (c == d) f = pT + f;
-    F[1 + c] = f + vd * p.m[c];
-  }
-  F[1 + NDIR] = (p.m[d] * pT - p.b[d] * sbgm - (C)p.bg[d] * sbm) * inv +
-                (C)p.eb * p.m[d] * inv - p.b[d] * sbm * inv + vd * p.e;
-#pragma unroll
-  for (int c = 0; c < NDIR; c++) {
-    F[2 + NDIR + c] = (c == d) ? (C)0
-                               : (-p.m[c] * inv * (p.b[d] + (C)p.bg[d]) +
-                                  p.m[d] * inv * (C)p.bg[c] + vd * p.b[c]);
-  }
-#pragma unroll
-  for (int l = 0; l < NV; l++) v[l] = p.m[l] * inv;
+  for (int l = 0; l < NV; l++) v[l] = p.m[l] * f.inv;
 }
 
 // fast-mode speed + |v_d| (getcmax, src/vacphys0.t.mhd:77-112) in FP64 for
@@ -167,28 +200,27 @@ __device__ __forceinline__ void flux_pt(const Pt<NDIR, C>& p, int d, double gamm
 template <int NDIM, int NDIR>
 __device__ __forceinline__ void cmax_all(const Pt<NDIR, double>& p, double gamma,
                                          double (&cm)[NDIM]) {
+#pragma clang fp contract(off)
   const double rt = p.rho + p.rhob;
   const double inv = 1.0 / rt;
   double sm2 = 0.0, sb2 = 0.0, sbbg = 0.0, sbg2 = 0.0, sbt2 = 0.0;
 #pragma unroll
   for (int c = 0; c < NDIR; c++) {
-    sm2 += p.m[c] * p.m[c];
-    sb2 += p.b[c] * p.b[c];
-    sbbg += p.b[c] * p.bg[c];
-    sbg2 += p.bg[c] * p.bg[c];
-    double bt = p.b[c] + p.bg[c];
-    sbt2 += bt * bt;
+    sm2 = fma_(p.m[c], p.m[c], sm2);
+    sb2 = fma_(p.b[c], p.b[c], sb2);
+    sbbg = fma_(p.b[c], p.bg[c], sbbg);
+    sbg2 = fma_(p.bg[c], p.bg[c], sbg2);
+    const double bt = p.b[c] + p.bg[c];
+    sbt2 = fma_(bt, bt, sbt2);
   }
-  double pth = 0.5 * sm2 * inv;
-  pth = pth + 0.5 * sb2 + sbbg;
-  pth = (gamma - 1.0) * (p.e - pth);
-  const double cs2 = gamma * (pth + (gamma - 1.0) * (p.eb - 0.5 * sbg2)) * inv;
-  const double cf2 = sbt2 * inv + cs2;
+  const double pth = (gamma - 1.0) * (p.e - (fma_(0.5 * sm2, inv, 0.5 * sb2) + sbbg));
+  const double cs2 = gamma * fma_(gamma - 1.0, fma_(-0.5, sbg2, p.eb), pth) * inv;
+  const double cf2 = fma_(sbt2, inv, cs2);
   const double cf4 = cf2 * cf2, cs4 = 4.0 * cs2 * inv;
 #pragma unroll
   for (int d = 0; d < NDIM; d++) {
     const double bd = p.b[d] + p.bg[d];
-    cm[d] = sqrt(0.5 * (cf2 + sqrt(cf4 - cs4 * (bd * bd)))) + fabs(p.m[d] * inv);
+    cm[d] = sqrt(0.5 * (cf2 + sqrt(fma_(-cs4, bd * bd, cf4)))) + fabs(p.m[d] * inv);
   }
 }
 
@@ -203,7 +235,10 @@ __device__ __forceinline__ double max_dpp(double x) {
   // lanes without a source keep their own value
   const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
   const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
-  return fmax(x, __hiloint2double(h2, l2));
+  const double y = __hiloint2double(h2, l2);
+  double r;  // fmax would first quiet a y whose origin it cannot see
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
 }
 __device__ __forceinline__ double wave_max63(double x) {
   x = max_dpp<0x111>(x);  // row_shr:1, 2, 4, 8
@@ -214,21 +249,30 @@ __device__ __forceinline__ double wave_max63(double x) {
   return max_dpp<0x143>(x);
 }
 
-// v[k] to dst[k], or the last one to *last
+// v[k] to dst[k], or the last one to *last.  Wavefronts from `only` on have
+// nothing but the last one.
 template <int NV>
 __device__ __forceinline__ void block_max_atomic(double (&v)[NV], unsigned long long* dst,
-                                                 unsigned long long* last = nullptr) {
+                                                 unsigned long long* last = nullptr,
+                                                 int only = 16) {
   __shared__ double red[NV][16];
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
+  {
+    const double x = wave_max63(v[NV - 1]);
+    if (lane == 63) red[NV - 1][wid] = x;
+  }
+  if (wid < only) {
 #pragma unroll
-  for (int k = 0; k < NV; k++) {
-    const double x = wave_max63(v[k]);
-    if (lane == 63) red[k][wid] = x;
+    for (int k = 0; k < NV - 1; k++) {
+      const double x = wave_max63(v[k]);
+      if (lane == 63) red[k][wid] = x;
+    }
   }
   __syncthreads();
   if (threadIdx.x < NV) {
-    const int nwave = (blockDim.x + 63) >> 6;
+    const int nw = (blockDim.x + 63) >> 6;
+    const int nwave = (threadIdx.x == NV - 1) ? nw : min(nw, only);
     double x = 0.0;
     for (int j = 0; j < nwave; j++) x = fmax(x, red[threadIdx.x][j]);
     unsigned long long* p = (last && threadIdx.x == NV - 1) ? last : dst + threadIdx.x;
@@ -317,6 +361,8 @@ __device__ __forceinline__ C face_ratio(const C* q) {
 // The two windows share four of their five first differences and two of
 // their three third differences; the maximum over the shared ones is taken
 // once (max is exact, so the grouping does not change the result).
+// The divisor is at least the smallest positive number, so that equal values
+// (md1 = md3 = 0) give 0 without a test.
 template <typename C>
 __device__ __forceinline__ void face_pair(const C* q, C& ratL, C& ratR) {
 #pragma clang fp contract(off)
@@ -325,12 +371,46 @@ __device__ __forceinline__ void face_pair(const C* q, C& ratL, C& ratR) {
   for (int j = 0; j < 6; j++) s[j] = q[j + 1] - q[j];
 #pragma unroll
   for (int j = 0; j < 4; j++) d3[j] = fabs((C)3 * s[j + 1] - (q[j + 3] - q[j]));
-  const C m1 = fmax(fmax(fabs(s[1]), fabs(s[2])), fmax(fabs(s[3]), fabs(s[4])));
+  const C tiny = sizeof(C) == 8 ? (C)4.9406564584124654e-324 : (C)1.4012984643e-45f;
+  const C m1 = fmax(fmax(fmax(fabs(s[1]), tiny), fabs(s[2])), fmax(fabs(s[3]), fabs(s[4])));
   const C m3 = fmax(d3[1], d3[2]);
   const C md1L = fmax(m1, fabs(s[0])), md1R = fmax(m1, fabs(s[5]));
   const C md3L = fmax(d3[0], m3), md3R = fmax(m3, d3[3]);
-  ratL = (md1L > (C)0) ? cdiv(md3L, md1L) : (C)0;
-  ratR = (md1R > (C)0) ? cdiv(md3R, md1R) : (C)0;
+  ratL = cdiv(md3L, md1L);
+  ratR = cdiv(md3R, md1R);
+}
+
+// Hyperdiffusion along an axis (setnu, addsource_visc) of one cell, shared by
+// the line and plane tiles.  For one variable, nu dq at the cell's two faces
+// from its q window; with nu = c_tot c_hyp dx ratio:
+//   t = nu dq,  terms = (a_R t_R - a_L t_L) / dx^2 with the face means a
+// (the factors 1/2 of the means and of the momentum terms are taken into the
+// power-of-two multiples of 1/dx^2, so nothing is rounded by them).
+template <typename C>
+struct HyperAxis {
+  C kv, ks;      // c_tot c_hyp dx of the velocities (c_hyp 0.4) and the others (0.04)
+  C i2, i2h, i2q;  // 1/dx^2 and its half and quarter
+  C it;          // 1/dx / 8
+  __device__ __forceinline__ HyperAxis(C ctk, C dxk, C idx) {
+    kv = ctk * (C)0.4 * dxk;
+    ks = ctk * (C)0.04 * dxk;
+    i2 = idx * idx;
+    i2h = (C)0.5 * i2;
+    i2q = (C)0.25 * i2;
+    it = (C)0.125 * idx;
+  }
+};
+// the two faces' t (zero: gradients replaced by zero, at a mesh end); returns
+// (q_+ - q_-) (nu_L + nu_R), the cross factor's product, and adds to numax
+template <typename C>
+__device__ __forceinline__ C hyper_faces(const C* q, C k, C ratL, C ratR, bool zero, C& tL, C& tR,
+                                         C& numax) {
+#pragma clang fp contract(off)
+  const C nuL = k * ratL, nuR = k * ratR;
+  numax = fmax(numax, fmax(nuR, nuL));
+  tL = zero ? (C)0 : nuL * (q[3] - q[2]);
+  tR = zero ? (C)0 : nuR * (q[4] - q[3]);
+  return zero ? (C)0 : (q[4] - q[2]) * (nuL + nuR);
 }
 
 __device__ __forceinline__ int cross_index(int ndim, int k, int l) {
@@ -637,7 +717,7 @@ constexpr int LV = 2 + 2 * NDIR + 8;
 template <int LT, int NDIR>
 __device__ __forceinline__ void line1_tile(const GridDesc& g, const double* __restrict__ W,
                                            const double* __restrict__ B,
-                                           const double* __restrict__ dx,
+                                           const double* __restrict__ dx, long long dxs,
                                            double (&R)[2 + 2 * NDIR], double gamma, int visc_on,
                                            double ctk, int c0, double* __restrict__ L,
                                            double& numax) {
@@ -681,11 +761,11 @@ __device__ __forceinline__ void line1_tile(const GridDesc& g, const double* __re
   const int k = t + 3;  // LDS index of the cell
   const bool fluxc = valid && c >= MloK + 2 && c <= MhiK - 2;
   const bool z1 = (c == MloK && !g.per_lo[0]) || (c == MhiK && !g.per_hi[0]);
-  const double dxd = dx[valid ? c : MhiK];
-  const double dxk = dxd, idx = 1.0 / dxd;
+  const double* dxc = dx + (valid ? c : MhiK);
+  const double dxk = dxc[0], idx = dxc[kDxInv * dxs];
   {
     const double pTb0 = at(NE + 1, k), bgk = at(NE + 2, k), bgl = bgk;
-    const double inv12 = idx / 12.0;
+    const double inv12 = dxc[kDxInv12 * dxs];
     double D1[NE], E1[NE];
 #pragma unroll
     for (int n = 0; n < NE; n++) D1[n] = two_diff(at(n, k + 1), at(n, k - 1), E1[n]);
@@ -831,7 +911,6 @@ __device__ __forceinline__ void cross_cells(const FinalArgs& a, const GridDesc& 
 #pragma unroll
       for (int k = 0; k < NDIM; k++) {
         if (k == l) continue;
-        if (a.skip_xy && k + l == 1) continue;  // added by the plane tiles
         const long long xi = (long long)cross_index(NDIM, k, l) * fs;
         C Tmp0[V], Tmm0[V], Tbp0[V], Tbm0[V], mkp[V], mkm[V], bkp[V], bkm[V];
 #pragma unroll
@@ -1058,7 +1137,7 @@ __device__ __forceinline__ bool line1_stage(const FinalArgs& f, const GridDesc& 
                                             int c0, double* __restrict__ L, double& numax,
                                             double (&redv)[2]) {
   double R[1][2 + 2 * NDIR];
-  line1_tile<LT, NDIR>(g, (const double*)f.wct, f.bg, f.dx[0], R[0], f.gamma, f.visc_on, ctk, c0, L,
+  line1_tile<LT, NDIR>(g, (const double*)f.wct, f.bg, f.dx[0], f.dxs, R[0], f.gamma, f.visc_on, ctk, c0, L,
                        numax);
   const int c[3] = {c0 + (int)threadIdx.x, 0, 0};
   if (c[0] > g.Mhi[0]) return false;

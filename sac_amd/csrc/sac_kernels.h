@@ -13,6 +13,7 @@ struct AxisArgs {
   const void* wct;       // stage input (time-centred state)
   const double* bg;      // background fields
   const double* dx[3];   // per-axis cell widths, indexed by grid index
+  long long dxs;         // their further tables (kDxInv ...)
   void* R;               // rate accumulator (n_evolve fields)
   void* T;               // cross-term factors (2*ndim*(ndim-1) fields)
   double gamma;
@@ -23,6 +24,7 @@ struct AxisArgs {
   const float* RF;                     // learned face ratios of axis K, or null (exact)
   int cross_last;                      // last axis: add the cross-term derivatives along it
   int divbfix;                         // Powell's div B sources (ndim > 1)
+  int fresh;                           // R is written, not added to (K = 0 always does)
 };
 
 struct FinalArgs {
@@ -31,6 +33,7 @@ struct FinalArgs {
   const void* wct;
   const double* bg;
   const double* dx[3];
+  long long dxs;
   const void* R;
   const void* T;
   const void* base;      // out = base + qa*R
@@ -48,7 +51,6 @@ struct FinalArgs {
   const unsigned long long* ctot_src;  // c_tot per direction of wct (fused stages)
   int xcd;
   int skip_last;                // cross-term derivatives along the last axis already in R
-  int skip_xy;                  // the x-y cross-term derivatives already in R (plane tiles)
   int divbfix;                  // Powell's sources (fused stages)
 };
 
@@ -114,12 +116,12 @@ void launch_resistive(const ResistArgs& a, hipStream_t st);
 int launch_axis(const AxisArgs& a, int axis, hipStream_t st);
 // 1 if the line-tile kernels (which carry the Powell sources) are built
 int line_tiles_built();
-// the x and y work of a 3-D grid in one pass over z-plane tiles (sac_plane.h),
-// the x-y cross terms included; R is written fresh
-void launch_plane(const AxisArgs& a, hipStream_t st);
+// 3-D grids: the cross-term factors T_{0,2} and T_{1,2} (sac_tile.h)
+void launch_tz(const AxisArgs& a, hipStream_t st);
 void launch_final(const FinalArgs& a, hipStream_t st);
-// a whole stage of a 2-D grid in one launch; a.R, if given, is added to the
-// rate (k_resist)
+// a whole stage of a 2-D grid in one launch, or the x and y work and the
+// update of a 3-D one after its z line tiles; a.R, if given, is added to the
+// rate (z work, k_resist)
 void launch_stage(const FinalArgs& a, hipStream_t st);
 // 1 if the tiles of launch_stage can address a plane of the grid
 int stage_tiles_fit(const GridDesc& g);

@@ -25,7 +25,6 @@
 //   getboundary        src/vacgrid.t:195-512
 #include "sac_device.h"
 #include "sac_line.h"
-#include "sac_plane.h"
 #include "sac_tile.h"
 
 // SAC_LINE_TILES=0 keeps the line-group kernel k_axis for every grid (the
@@ -85,18 +84,6 @@ __global__ void __launch_bounds__((line::Tile<K, C>::T)) k_line(AxisArgs a, int 
   }
 }
 
-// kernel 1, 3-D grids: the x and y work of z-plane tiles (see plane_tile)
-template <typename S, typename C>
-__global__ void __launch_bounds__(plane::NT) k_plane(AxisArgs a) {
-  __shared__ plane::Smem<C> sm;
-  C numax = 0;
-  plane::plane_tile<S, C>(a, sm, numax);
-  if (a.visc_on) {
-    double r2[1] = {(double)numax};
-    block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
-  }
-}
-
 // kernel 1, 1-D grids in FP64 whose rate gets further terms before the
 // update (resistivity): LDS line tiles of 256 cells (line1_tile), R to memory
 template <int NDIR>
@@ -105,7 +92,7 @@ __global__ void __launch_bounds__(256) k_line1(AxisArgs a) {
   double numax = 0.0;
   double R[2 + 2 * NDIR];
   const int c0 = a.g.Mlo[0] + 256 * (int)blockIdx.x, c = c0 + (int)threadIdx.x;
-  line1_tile<256, NDIR>(a.g, (const double*)a.wct, a.bg, a.dx[0], R, a.gamma, a.visc_on,
+  line1_tile<256, NDIR>(a.g, (const double*)a.wct, a.bg, a.dx[0], a.dxs, R, a.gamma, a.visc_on,
                         a.visc_on ? red_get(a.ctot_src, 0) : 0.0, c0, L, numax);
   if (c <= a.g.Mhi[0]) {
 #pragma unroll
@@ -131,18 +118,34 @@ __global__ void __launch_bounds__(LT) k_stage1(FinalArgs a) {
   block_max_atomic<3>(m, red_line(a.acc), red_line(a.acc) + kRedVisc);
 }
 
-// 2-D grids: a whole RK stage per launch (see stage_tile)
-template <int NDIM, int NDIR, typename S, typename C, bool RK4L, bool DIVB>
-__global__ void __launch_bounds__(tile::NT) k_stage(FinalArgs a) {
-  __shared__ tile::Smem<NDIM, NDIR, C, DIVB> sm;
-  // block -> tile: each XCD takes one contiguous range of tiles, so the halos
-  // a tile shares with its neighbours are fetched into one L2
-  const unsigned b = xcd_block8(), nx = tile::ntx(a.g), ny = tile::nty(a.g);
+// block -> tile (first cell at x0, y0 of plane z): each XCD takes one
+// contiguous range of tiles, so the halos a tile shares with its neighbours
+// are fetched into one L2; false for a block past the last tile
+__device__ __forceinline__ bool tile_of(const GridDesc& g, int& x0, int& y0, int& z) {
+  const unsigned b = xcd_block8(), nx = tile::ntx(g), ny = tile::nty(g);
   const unsigned r = b / nx, zt = r / ny;
-  if (zt > (unsigned)(a.g.Mhi[2] - a.g.Mlo[2])) return;
-  const int x0 = (int)(b - r * nx) * tile::TX;
-  const int y0 = a.g.Mlo[1] + (int)(r - zt * ny) * tile::TY;
-  const int z = a.g.Mlo[2] + (int)zt;
+  x0 = g.Mlo[0] + (int)(b - r * nx) * tile::TX;
+  y0 = g.Mlo[1] + (int)(r - zt * ny) * tile::TY;
+  z = g.Mlo[2] + (int)zt;
+  return z <= g.Mhi[2];
+}
+
+// 3-D grids: the factors the z line tiles differentiate (see tz_tile)
+template <typename S, typename C>
+__global__ void __launch_bounds__(tile::NC) k_tz(AxisArgs a) {
+  __shared__ tile::TzSmem<C> sm;
+  int x0, y0, z;
+  if (!tile_of(a.g, x0, y0, z)) return;
+  tile::tz_tile<S, C>(a, x0, y0, z, sm);
+}
+
+// 2-D grids: a whole RK stage per launch; 3-D grids: its last pass (see
+// stage_tile).  Four wavefronts per SIMD: the two blocks a CU's LDS holds.
+template <int NDIM, int NDIR, typename S, typename C, bool RK4L, bool DIVB>
+__global__ void __launch_bounds__(tile::NT, 4) k_stage(FinalArgs a) {
+  __shared__ tile::Smem<NDIM, NDIR, C, DIVB> sm;
+  int x0, y0, z;
+  if (!tile_of(a.g, x0, y0, z)) return;
   C numax = 0;
   double redv[2 * NDIM];
 #pragma unroll
@@ -153,7 +156,8 @@ __global__ void __launch_bounds__(tile::NT) k_stage(FinalArgs a) {
 #pragma unroll
   for (int k = 0; k < 2 * NDIM; k++) m[k] = redv[k];
   m[2 * NDIM] = (double)numax;
-  block_max_atomic<2 * NDIM + 1>(m, red_line(a.acc), red_line(a.acc) + kRedVisc);
+  // the y wavefronts have only their largest nu
+  block_max_atomic<2 * NDIM + 1>(m, red_line(a.acc), red_line(a.acc) + kRedVisc, tile::NC / 64);
 }
 
 // segment length along K: whole lines unless that leaves fewer than 2048
@@ -610,23 +614,22 @@ int stage_tiles_fit(const GridDesc& g) { return SAC_LINE_TILES && tile::rows_fit
 
 void launch_stage(const FinalArgs& a, hipStream_t st) {
   if (a.prec == PREC_MIXED) {
-    if (a.g.ndir == 2) launch_stage_t<2, 2, float, float>(a, st);
+    if (a.g.ndim == 3) launch_stage_t<3, 3, float, float>(a, st);
+    else if (a.g.ndir == 2) launch_stage_t<2, 2, float, float>(a, st);
     else launch_stage_t<2, 3, float, float>(a, st);
   } else {
-    if (a.g.ndir == 2) launch_stage_t<2, 2, double, double>(a, st);
+    if (a.g.ndim == 3) launch_stage_t<3, 3, double, double>(a, st);
+    else if (a.g.ndir == 2) launch_stage_t<2, 2, double, double>(a, st);
     else launch_stage_t<2, 3, double, double>(a, st);
   }
 }
 
-void launch_plane(const AxisArgs& a, hipStream_t st) {
-  long long nb = plane::nblocks(a.g);
-  const int xcd = a.xcd > 1 ? a.xcd : 1;
-  nb = (nb + xcd - 1) / xcd * xcd;  // xcd_block needs a multiple of the XCD count
-  if (nb <= 0) return;
+void launch_tz(const AxisArgs& a, hipStream_t st) {
+  const dim3 nb((unsigned)((tile::nblocks(a.g) + 7) / 8 * 8)), bs(tile::NC);
   if (a.prec == PREC_MIXED)
-    hipLaunchKernelGGL((k_plane<float, float>), dim3((unsigned)nb), dim3(plane::NT), 0, st, a);
+    hipLaunchKernelGGL((k_tz<float, float>), nb, bs, 0, st, a);
   else
-    hipLaunchKernelGGL((k_plane<double, double>), dim3((unsigned)nb), dim3(plane::NT), 0, st, a);
+    hipLaunchKernelGGL((k_tz<double, double>), nb, bs, 0, st, a);
 }
 
 void launch_final(const FinalArgs& a, hipStream_t st) {

@@ -93,13 +93,12 @@ struct Axes {
   static constexpr int B = (NDIM == 3) ? ((K == 2) ? 1 : 2) : -1;
 };
 
-// First grid index of the line tiles along A: tiles along x start at the
-// row start, so that a tile's 16 values of a row fill whole 128-byte lines
-// (rows are padded to a multiple of 16 elements) and no two tiles share a
-// line; the ghost columns of the first and last tile stay idle.
+// First grid index of the line tiles along A: the first mesh cell, which
+// along x lies on a 128-byte line (kFieldPad), so that a tile's 16 values of
+// a row fill whole lines and no two tiles share one.
 template <int A>
 __host__ __device__ inline int tile_origin(const GridDesc& g) {
-  return (A == 0) ? 0 : g.Mlo[A];
+  return g.Mlo[A];
 }
 
 // blocks of a launch for segments of `seg` cells along K
@@ -174,15 +173,15 @@ __device__ __forceinline__ void line_tile(const AxisArgs& a, int seg, C* __restr
   const int ce = (cs + seg - 1 < MhiK) ? cs + seg - 1 : MhiK;
   // first point of the ring: three before the first cell.  Along x it is
   // moved down so that the cells of every chunk (three behind its points)
-  // start on a multiple of 16 elements: each chunk then writes whole
+  // start on a multiple of 16 elements (index 2 does): each chunk then writes whole
   // 128-byte lines of R and T, and its loads, three elements earlier, share
   // their partial lines with the neighbouring chunk of the same block
   // (2 % faster than aligning the loads at 256^3).  The extra points only
   // feed cells before the segment, which are idle.
   int ps = cs - HALO;
   if (K == 0) {
-    const int q = cs - 2 * HALO;
-    ps = ((q >= 0) ? q / 16 * 16 : -((-q + 15) / 16) * 16) + HALO;
+    const int q = cs - 2 * HALO - 2;
+    ps = ((q >= 0) ? q / 16 * 16 : -((-q + 15) / 16) * 16) + 2 + HALO;
   }
   const int nch = (ce + HALO - ps + 1 + CH - 1) / CH;
 
@@ -227,8 +226,10 @@ __device__ __forceinline__ void line_tile(const AxisArgs& a, int seg, C* __restr
     C Rold[NE];
     const long long icell = cell_index(j);
 #pragma unroll
-    for (int n = 0; n < NE; n++) Rold[n] = (K > 0) ? (C)Racc[n * fs + icell] : (C)0;
-    const double dxd = a.dx[K][cell_clamped(j)];
+    for (int n = 0; n < NE; n++) Rold[n] = (K > 0 && !a.fresh) ? (C)Racc[n * fs + icell] : (C)0;
+    const double* dxc = a.dx[K] + cell_clamped(j);
+    const double dxd = dxc[0], dxi = dxc[kDxInv * a.dxs], dxi12 = dxc[kDxInv12 * a.dxs];
+    const double dxh = dxc[kDxHalf * a.dxs];
     // the cell's background: p_Tb (getptotal_bg) and bg_l of the energy terms
     Pt<NDIR, C> pbg;
     pbg.eb = Bg[icell];
@@ -305,12 +306,12 @@ __device__ __forceinline__ void line_tile(const AxisArgs& a, int seg, C* __restr
         int r = r0 - HALO + d;
         return (r < 0) ? r + RR : r;
       };
-      const C dxk = (C)dxd, idx = (C)(1.0 / dxd);
+      const C dxk = (C)dxd, idx = (C)dxi;
       C R[NE];
       {
         const bool fluxc = c >= MloK + 2 && c <= MhiK - 2;
         const int rm2 = row(-2), rm1 = row(-1), rp1 = row(1), rp2 = row(2);
-        const C inv12 = idx / (C)12;
+        const C inv12 = (C)dxi12;
 #pragma unroll
         for (int n = 0; n < NE; n++) {
           C E1, e2;
@@ -364,7 +365,7 @@ __device__ __forceinline__ void line_tile(const AxisArgs& a, int seg, C* __restr
         const bool z1 = (c == MloK && !g.per_lo[K]) || (c == MhiK && !g.per_hi[K]);
         if (do_cross && valid && !z1) {
           const int rp1 = row(1), rm1 = row(-1);
-          const C h = (C)(0.5 / dxd);
+          const C h = (C)dxh;
           const bool inP = c + 1 <= MhiK, inM = c - 1 >= MloK;
           const C rtp = L[at<K, C>(SL::RT, rp1, iw)], rtm = L[at<K, C>(SL::RT, rm1, iw)];
 #pragma unroll
@@ -385,59 +386,49 @@ __device__ __forceinline__ void line_tile(const AxisArgs& a, int seg, C* __restr
 #pragma clang fp contract(off)
         const bool z1 = (c == MloK && !g.per_lo[K]) || (c == MhiK && !g.per_hi[K]);
         const int rw[7] = {row(-3), row(-2), row(-1), row(0), row(1), row(2), row(3)};
-        const C rtm = L[at<K, C>(SL::RT, rw[2], iw)], rt0 = L[at<K, C>(SL::RT, rw[3], iw)],
-                rtp = L[at<K, C>(SL::RT, rw[4], iw)];
-        const C rhoL = (rt0 + rtm) * (C)0.5, rhoR = (rtp + rt0) * (C)0.5;
+        const HyperAxis<C> ha(ctk, dxk, idx);
+        C nmax = 0;
+        const C rt0 = L[at<K, C>(SL::RT, rw[3], iw)];  // twice the means at the faces
+        const C rhoL = rt0 + L[at<K, C>(SL::RT, rw[2], iw)];
+        const C rhoR = L[at<K, C>(SL::RT, rw[4], iw)] + rt0;
 #pragma unroll
         for (int p = 0; p < NP; p++) {
-          C q[7];
+          const bool vel = p >= 2 && p < 2 + NDIM;
+          C q[7], ratL, ratR, tL, tR;
 #pragma unroll
           for (int s = 0; s < 7; s++) q[s] = L[at<K, C>(SL::Q0 + p, rw[s], iw)];
-          const C ch = (p >= 2 && p < 2 + NDIM) ? (C)0.4 : (C)0.04;
-          const C Kc = ctk * ch;
-          C ratL, ratR;
           if constexpr (LEARNED) {
             ratL = (rfc[2 * p] >= 0.f) ? (C)rfc[2 * p] : face_ratio<C>(q);
             ratR = (rfc[2 * p + 1] >= 0.f) ? (C)rfc[2 * p + 1] : face_ratio<C>(q + 1);
           } else {
             face_pair<C>(q, ratL, ratR);
           }
-          const C nuL = Kc * ratL * dxk;
-          const C nuR = Kc * ratR * dxk;
-          numax = valid ? fmax(numax, fmax(nuR, nuL)) : numax;
-          const C qm = q[2], q0 = q[3], qp = q[4];
-          const C gL = z1 ? (C)0 : (q0 - qm) * idx;
-          const C gR = z1 ? (C)0 : (qp - q0) * idx;
-          const C tL = nuL * gL, tR = nuR * gR;
+          const C T = hyper_faces<C>(q, vel ? ha.kv : ha.ks, ratL, ratR, z1, tL, tR, nmax);
           if (p == 0) {
-            R[0] += (tR - tL) * idx;
+            R[0] = fma_(tR - tL, ha.i2, R[0]);
           } else if (p == 1) {
-            R[1 + NDIR] += (tR - tL) * idx;
-          } else if (p < 2 + NDIM) {
+            R[1 + NDIR] = fma_(tR - tL, ha.i2, R[1 + NDIR]);
+          } else if (vel) {
             const int l = p - 2;
             const C m0 = L[at<K, C>(SL::M0 + l, rw[3], iw)];
-            const C mL = (m0 + L[at<K, C>(SL::M0 + l, rw[2], iw)]) * (C)0.5;
-            const C mR = (L[at<K, C>(SL::M0 + l, rw[4], iw)] + m0) * (C)0.5;
-            const C mult = (l == K) ? (C)1 : (C)0.5;  // the i==k branch runs twice for l==k
-            R[1 + l] += mult * (rhoR * tR - rhoL * tL) * idx;
-            R[1 + NDIR] += mult * (mR * tR - mL * tL) * idx;
-            if (l != K && valid) {
-              const C gC = z1 ? (C)0 : (qp - qm) * idx * (C)0.5;
-              Tout[(long long)cross_index(NDIM, K, l) * fs + icell] = (S)(gC * (nuL + nuR) * (C)0.25);
-            }
+            const C mL = m0 + L[at<K, C>(SL::M0 + l, rw[2], iw)];
+            const C mR = L[at<K, C>(SL::M0 + l, rw[4], iw)] + m0;
+            const C f = (l == K) ? ha.i2h : ha.i2q;  // the i==k branch runs twice for l==k
+            R[1 + l] = fma_(fma_(rhoR, tR, -(rhoL * tL)), f, R[1 + l]);
+            R[1 + NDIR] = fma_(fma_(mR, tR, -(mL * tL)), f, R[1 + NDIR]);
+            if (l != K && valid)
+              Tout[(long long)cross_index(NDIM, K, l) * fs + icell] = (S)(T * ha.it);
           } else {
             const int n = p - 2 - NDIM;
             const int lb = (n < K) ? n : n + 1;
-            const C BL = (q0 + qm) * (C)0.5, BR = (qp + q0) * (C)0.5;
-            R[2 + NDIR + lb] += (tR - tL) * idx;
-            R[1 + NDIR] += (tR * BR - tL * BL) * idx;
-            if (valid) {
-              const C gC = z1 ? (C)0 : (qp - qm) * idx * (C)0.5;
-              Tout[(long long)(cross_index(NDIM, K, lb) + 1) * fs + icell] =
-                  (S)(gC * (nuL + nuR) * (C)0.5);
-            }
+            const C BL = q[3] + q[2], BR = q[4] + q[3];
+            R[2 + NDIR + lb] = fma_(tR - tL, ha.i2, R[2 + NDIR + lb]);
+            R[1 + NDIR] = fma_(fma_(BR, tR, -(BL * tL)), ha.i2h, R[1 + NDIR]);
+            if (valid)
+              Tout[(long long)(cross_index(NDIM, K, lb) + 1) * fs + icell] = (S)((C)2 * T * ha.it);
           }
         }
+        numax = valid ? fmax(numax, nmax) : numax;
       }
       if (valid) {
         if (K == 0) {

@@ -26,10 +26,13 @@
 // (75 KB in 3-D) lets two blocks into a CU.  Two axes on twice the
 // wavefronts halve the chain and give four wavefronts per SIMD instead of
 // two.  A 2-D stage of 501 x 299 cells was an x and a y line kernel and an
-// update, 19.8 + 16.3 + 15.5 us; here 21.7.  Reading the cell's background,
-// c_tot and dx before the points, and the base register while the axes are
-// handed over, took that from 24.2 (512 patches: 0.83 -> 0.71 ms).  VALU issue
-// is 350 of the 706 us of 512 patches, the rest waits.
+// update, 19.8 + 16.3 + 15.5 us; here 21.3.  512 patches (4.8 M cells): 0.996
+// ms before, 0.677 now.  Reading the cell's background, c_tot and dx before
+// the points, and the base register while the axes are handed over, is 15 %
+// of that.  In 3-D a tile is bound by both its VALU issue (2350 instructions
+// per 64 cells, 60 % of the time at the 2.07 GHz the card runs FP64 work at)
+// and the waits between its barriers: 128 VGPRs keep the four wavefronts per
+// SIMD (144 let in one block per CU: 2.07 -> 2.78 ms at 256^3).
 //
 // Grid edges follow the line tiles: a point beyond the grid along x (y) is
 // the mirror cell 6 inward (src/vacusr.viscosity.t:378-400), read only by
@@ -86,6 +89,11 @@ struct Smem {
   C v[Lay<NDIM, NDIR, C, DIVB>::END];
 };
 
+template <bool B>
+struct Bool {
+  static constexpr bool value = B;
+};
+
 // flux slot of field n along K
 __host__ __device__ constexpr int fslot(int ndir, int K, int n) {
   return n > 2 + ndir + K ? n - 1 : n;
@@ -101,9 +109,10 @@ __device__ __forceinline__ int cell_row(int t) {
     return t / TX;
 }
 
-// tiles of a plane along x (from grid column 0, so that a tile row fills
-// whole 128-byte lines) and y
-__host__ __device__ inline int ntx(const GridDesc& g) { return (g.Mhi[0] + 1 + TX - 1) / TX; }
+// tiles of a plane along x and y
+__host__ __device__ inline int ntx(const GridDesc& g) {
+  return (g.Mhi[0] - g.Mlo[0] + 1 + TX - 1) / TX;
+}
 __host__ __device__ inline int nty(const GridDesc& g) {
   return (g.Mhi[1] - g.Mlo[1] + 1 + TY - 1) / TY;
 }
@@ -118,22 +127,23 @@ __host__ __device__ inline bool rows_fit(long long pitch) { return pitch < (1LL 
 // setnu face ratios, hyperdiffusion line terms; returns the factors
 // T_{K,1-K} in Tm, Tb.  fget(s, d) is flux slot s at offset d along K,
 // qget(p, d) the q of setnu's variable p of axis K (rho', thermal energy,
-// v_0.., b_l (l != K)), rget(d) rho_t, mget(l, d) m_l.
-template <int NDIM, int NDIR, int K, typename S, typename C, bool DIVB, typename FG, typename QG,
-          typename RG, typename MG>
+// v_0.., b_l (l != K)), rget(d) rho_t, mget(l, d) m_l.  EDGE: some cell of
+// the wavefront may lie within two cells of an end of the mesh along K, where
+// terms are replaced by zero; the other wavefronts go without those selects
+// (about 60 of the 700 instructions of an axis).
+template <int NDIM, int NDIR, int K, typename S, typename C, bool DIVB, bool EDGE, typename FG,
+          typename QG, typename RG, typename MG>
 __device__ __forceinline__ void cell_axis(const FinalArgs& f, const GridDesc& g, long long icell,
                                           const Pt<NDIR, C>& pbg, C (&R)[2 + 2 * NDIR], int c,
-                                          double dxd, C ctk,
+                                          C dxk, C idx, C inv12, C ctk,
                                           bool valid, C& numax, FG fget, QG qget, RG rget, MG mget,
                                           C& Tm, C& Tb) {
   constexpr int NE = 2 + 2 * NDIR, NP = 2 * NDIM + 1;
   const long long fs = g.fs;
   const double* __restrict__ Bg = f.bg;
   const int MloK = g.Mlo[K], MhiK = g.Mhi[K];
-  const C dxk = (C)dxd, idx = (C)(1.0 / dxd);
   {
-    const bool fluxc = c >= MloK + 2 && c <= MhiK - 2;
-    const C inv12 = idx / (C)12;
+    const bool fluxc = !EDGE || (c >= MloK + 2 && c <= MhiK - 2);
 #pragma unroll
     for (int n = 0; n < NE; n++) {
       if (n == 2 + NDIR + K) {
@@ -181,53 +191,40 @@ __device__ __forceinline__ void cell_axis(const FinalArgs& f, const GridDesc& g,
   }
   if (f.visc_on) {
 #pragma clang fp contract(off)
-    const bool z1 = (c == MloK && !g.per_lo[K]) || (c == MhiK && !g.per_hi[K]);
-    const C rtm = rget(-1), rt0 = rget(0), rtp = rget(1);
-    const C rhoL = (rt0 + rtm) * (C)0.5, rhoR = (rtp + rt0) * (C)0.5;
+    const bool z1 =
+        EDGE && ((c == MloK && !g.per_lo[K]) || (c == MhiK && !g.per_hi[K]));
+    C nmax = 0;
+    const HyperAxis<C> ha(ctk, dxk, idx);
+    const C rt0 = rget(0), rhoL = rt0 + rget(-1), rhoR = rget(1) + rt0;  // twice the means
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-      C q[7];
+      const bool vel = p >= 2 && p < 2 + NDIM;
+      C q[7], ratL, ratR, tL, tR;
 #pragma unroll
       for (int s = 0; s < 7; s++) q[s] = qget(p, s - 3);
-      C ratL, ratR;
       face_pair<C>(q, ratL, ratR);
-      const C ch = (p >= 2 && p < 2 + NDIM) ? (C)0.4 : (C)0.04;
-      const C Kc = ctk * ch;
-      const C nuL = Kc * ratL * dxk;
-      const C nuR = Kc * ratR * dxk;
-      numax = valid ? fmax(numax, fmax(nuR, nuL)) : numax;
-      const C qm = q[2], q0 = q[3], qp = q[4];
-      const C gL = z1 ? (C)0 : (q0 - qm) * idx;
-      const C gR = z1 ? (C)0 : (qp - q0) * idx;
-      const C tL = nuL * gL, tR = nuR * gR;
+      const C T = hyper_faces<C>(q, vel ? ha.kv : ha.ks, ratL, ratR, z1, tL, tR, nmax);
       if (p == 0) {
-        R[0] += (tR - tL) * idx;
+        R[0] = fma_(tR - tL, ha.i2, R[0]);
       } else if (p == 1) {
-        R[1 + NDIR] += (tR - tL) * idx;
-      } else if (p < 2 + NDIM) {
+        R[1 + NDIR] = fma_(tR - tL, ha.i2, R[1 + NDIR]);
+      } else if (vel) {
         const int l = p - 2;
-        const C m0 = mget(l, 0);
-        const C mL = (m0 + mget(l, -1)) * (C)0.5;
-        const C mR = (mget(l, 1) + m0) * (C)0.5;
-        const C mult = (l == K) ? (C)1 : (C)0.5;  // the i==k branch runs twice for l==k
-        R[1 + l] += mult * (rhoR * tR - rhoL * tL) * idx;
-        R[1 + NDIR] += mult * (mR * tR - mL * tL) * idx;
-        if (l == 1 - K) {
-          const C gC = z1 ? (C)0 : (qp - qm) * idx * (C)0.5;
-          Tm = gC * (nuL + nuR) * (C)0.25;
-        }
+        const C m0 = mget(l, 0), mL = m0 + mget(l, -1), mR = mget(l, 1) + m0;
+        const C f = (l == K) ? ha.i2h : ha.i2q;  // the i==k branch runs twice for l==k
+        R[1 + l] = fma_(fma_(rhoR, tR, -(rhoL * tL)), f, R[1 + l]);
+        R[1 + NDIR] = fma_(fma_(mR, tR, -(mL * tL)), f, R[1 + NDIR]);
+        if (l == 1 - K) Tm = T * ha.it;
       } else {
         const int n = p - 2 - NDIM;
         const int lb = (n < K) ? n : n + 1;
-        const C BL = (q0 + qm) * (C)0.5, BR = (qp + q0) * (C)0.5;
-        R[2 + NDIR + lb] += (tR - tL) * idx;
-        R[1 + NDIR] += (tR * BR - tL * BL) * idx;
-        if (lb == 1 - K) {
-          const C gC = z1 ? (C)0 : (qp - qm) * idx * (C)0.5;
-          Tb = gC * (nuL + nuR) * (C)0.5;
-        }
+        const C BL = q[3] + q[2], BR = q[4] + q[3];
+        R[2 + NDIR + lb] = fma_(tR - tL, ha.i2, R[2 + NDIR + lb]);
+        R[1 + NDIR] = fma_(fma_(BR, tR, -(BL * tL)), ha.i2h, R[1 + NDIR]);
+        if (lb == 1 - K) Tb = (C)2 * T * ha.it;
       }
     }
+    numax = valid ? nmax : (C)0;
   }
 }
 
@@ -235,16 +232,14 @@ __device__ __forceinline__ void cell_axis(const FinalArgs& f, const GridDesc& g,
 // 0: the velocity, 1: the field), from q[0..6] along K; the same arithmetic
 // as cell_axis.
 template <typename C>
-__device__ __forceinline__ C cross_factor(const C (&q)[7], int which, bool z1, double dxd, C ctk) {
+__device__ __forceinline__ C cross_factor(const C (&q)[7], int which, bool z1, C dxk, C idx,
+                                          C ctk) {
 #pragma clang fp contract(off)
-  const C dxk = (C)dxd, idx = (C)(1.0 / dxd);
-  const C Kc = ctk * (which ? (C)0.04 : (C)0.4);
-  C ratL, ratR;
+  const HyperAxis<C> ha(ctk, dxk, idx);
+  C ratL, ratR, tL, tR, nmax = 0;
   face_pair<C>(q, ratL, ratR);
-  const C nuL = Kc * ratL * dxk;
-  const C nuR = Kc * ratR * dxk;
-  const C gC = z1 ? (C)0 : (q[4] - q[2]) * idx * (C)0.5;
-  return gC * (nuL + nuR) * (which ? (C)0.5 : (C)0.25);
+  const C T = hyper_faces<C>(q, which ? ha.ks : ha.kv, ratL, ratR, z1, tL, tR, nmax);
+  return which ? (C)2 * T * ha.it : T * ha.it;
 }
 
 // The stage of the tile with its first cell at grid column x0 and row y0 of
@@ -269,7 +264,10 @@ __device__ __forceinline__ bool stage_tile(const FinalArgs& f, const GridDesc& g
   const int cxc = (cx > g.G[0] - 1) ? g.G[0] - 1 : cx;
   const int cyc = (cy > g.G[1] - 1) ? g.G[1] - 1 : cy;
   const long long icell = zoff + (long long)cyc * g.st[1] + cxc;
-  const double dxx = f.dx[0][cxc], dxy = f.dx[1][cyc];
+  // the cell's widths: of the wavefront's axis, and half over both
+  const double* dxc = xgrp ? f.dx[0] + cxc : f.dx[1] + cyc;
+  const C dxk = (C)dxc[0], idx = (C)dxc[kDxInv * f.dxs], inv12 = (C)dxc[kDxInv12 * f.dxs];
+  const C hx = (C)f.dx[0][kDxHalf * f.dxs + cxc], hy = (C)f.dx[1][kDxHalf * f.dxs + cyc];
   const C ctk = f.visc_on ? (C)red_get(f.ctot_src, xgrp ? 0 : 1) : (C)0;
   Pt<NDIR, C> own;  // the cell's background
   own.eb = f.bg[icell];
@@ -338,28 +336,31 @@ __device__ __forceinline__ bool stage_tile(const FinalArgs& f, const GridDesc& g
       p.rhob = bv(1);
 #pragma unroll
       for (int cd = 0; cd < NDIR; cd++) p.bg[cd] = bv(2 + cd);
-      if (fx) {
-        C F[NE], v[1];
-        flux_pt<NDIR, 1, C>(p, 0, f.gamma, F, v);
-        C* o = sm + L::FX + (iy - HALO) * L::FXP + ix - 1;
+      const double rtd = (double)p.rho + p.rhob;
+      const double inv = recip<C>(rtd);
+      if (fx || fy) {
+        const FluxPt<C> fc = flux_common<NDIR, C>(p, f.gamma, inv);
+        if (fx) {
+          C F[NE];
+          flux_axis<NDIR, C>(p, fc, 0, F);
+          C* o = sm + L::FX + (iy - HALO) * L::FXP + ix - 1;
 #pragma unroll
-        for (int n = 0; n < NE; n++)
-          if (n != 2 + NDIR) o[fslot(NDIR, 0, n) * TY * L::FXP] = F[n];
-        if constexpr (DIVB) o[(NE - 1) * TY * L::FXP] = (C)((double)p.b[0] + p.bg[0]);
-      }
-      if (fy) {
-        C F[NE], v[1];
-        flux_pt<NDIR, 1, C>(p, 1, f.gamma, F, v);
-        C* o = sm + L::FY + (iy - 1) * L::FYP + ix - HALO;
+          for (int n = 0; n < NE; n++)
+            if (n != 2 + NDIR) o[fslot(NDIR, 0, n) * TY * L::FXP] = F[n];
+          if constexpr (DIVB) o[(NE - 1) * TY * L::FXP] = (C)((double)p.b[0] + p.bg[0]);
+        }
+        if (fy) {
+          C F[NE];
+          flux_axis<NDIR, C>(p, fc, 1, F);
+          C* o = sm + L::FY + (iy - 1) * L::FYP + ix - HALO;
 #pragma unroll
-        for (int n = 0; n < NE; n++)
-          if (n != 3 + NDIR) o[fslot(NDIR, 1, n) * (TY + 4) * L::FYP] = F[n];
-        if constexpr (DIVB) o[(NE - 1) * (TY + 4) * L::FYP] = (C)((double)p.b[1] + p.bg[1]);
+          for (int n = 0; n < NE; n++)
+            if (n != 3 + NDIR) o[fslot(NDIR, 1, n) * (TY + 4) * L::FYP] = F[n];
+          if constexpr (DIVB) o[(NE - 1) * (TY + 4) * L::FYP] = (C)((double)p.b[1] + p.bg[1]);
+        }
       }
       {
 #pragma clang fp contract(off)
-        const double rtd = (double)p.rho + p.rhob;
-        const double inv = recip<C>(rtd);
         double sb = 0.0, smm = 0.0;
 #pragma unroll
         for (int cd = 0; cd < NDIR; cd++) {
@@ -396,48 +397,59 @@ __device__ __forceinline__ bool stage_tile(const FinalArgs& f, const GridDesc& g
   C R[1][NE], Tm = 0, Tb = 0, Th = 0;
   if (xgrp) {
     const C* fc = sm + L::FX + ty * L::FXP + tx + 2;
-    cell_axis<NDIM, NDIR, 0, S, C, DIVB>(
-        f, g, icell, own, R[0], cx, dxx, ctk, valid, numax,
-        [&](int s, int d) { return fc[s * TY * L::FXP + d]; },
-        [&](int p, int d) {
-          return p < 2 + NDIM ? qc[p * QA + d] : (p == 2 + NDIM ? b1[d] : qc[5 * QA + d]);
-        },
-        [&](int d) { return rc[d]; }, [&](int l, int d) { return rc[(1 + l) * RA + d]; }, Tm, Tb);
+    auto work = [&](auto edge) {
+      cell_axis<NDIM, NDIR, 0, S, C, DIVB, decltype(edge)::value>(
+          f, g, icell, own, R[0], cx, dxk, idx, inv12, ctk, valid, numax,
+          [&](int s, int d) { return fc[s * TY * L::FXP + d]; },
+          [&](int p, int d) {
+            return p < 2 + NDIM ? qc[p * QA + d] : (p == 2 + NDIM ? b1[d] : qc[5 * QA + d]);
+          },
+          [&](int d) { return rc[d]; }, [&](int l, int d) { return rc[(1 + l) * RA + d]; }, Tm,
+          Tb);
+    };
+    if (x0 < g.Mlo[0] + 2 || x0 + TX - 1 > g.Mhi[0] - 2) work(Bool<true>{});
+    else work(Bool<false>{});
     // T_{0,1} of the rows below and above the tile, one variable per lane
     if (f.visc_on && t >= NC - 64) {
-      const int hx = t & 15, hy = (t & 16) ? TY : -1, which = (t >> 5) & 1;
-      const int hcx = x0 + hx, hcxc = (hcx > g.G[0] - 1) ? g.G[0] - 1 : hcx;
-      const C* a = which ? sm + L::B1 + (hy + 1) * L::QP + hx + HALO
-                         : sm + 3 * QA + (hy + HALO) * L::QP + hx + HALO;
+      const int hc = t & 15, hr = (t & 16) ? TY : -1, which = (t >> 5) & 1;
+      const int hcx = x0 + hc, hcxc = (hcx > g.G[0] - 1) ? g.G[0] - 1 : hcx;
+      const double* dh = f.dx[0] + hcxc;
+      const C* a = which ? sm + L::B1 + (hr + 1) * L::QP + hc + HALO
+                         : sm + 3 * QA + (hr + HALO) * L::QP + hc + HALO;
       C q[7];
 #pragma unroll
       for (int s = 0; s < 7; s++) q[s] = a[s - 3];
       const bool z1 = (hcx == g.Mlo[0] && xlo) || (hcx == g.Mhi[0] && xhi);
-      Th = cross_factor<C>(q, which, z1, f.dx[0][hcxc], ctk);
+      Th = cross_factor<C>(q, which, z1, (C)dh[0], (C)dh[kDxInv * f.dxs], ctk);
     }
   } else {
     const C* fc = sm + L::FY + (ty + 2) * L::FYP + tx;
-    cell_axis<NDIM, NDIR, 1, S, C, DIVB>(
-        f, g, icell, own, R[0], cy, dxy, ctk, valid, numax,
-        [&](int s, int d) { return fc[(s * (TY + 4) + d) * L::FYP]; },
-        [&](int p, int d) {
-          return p < 2 + NDIM ? qc[p * QA + d * L::QP]
-                              : (p == 2 + NDIM ? b0[d * L::SP] : qc[5 * QA + d * L::QP]);
-        },
-        [&](int d) { return rc[d * L::SP]; },
-        [&](int l, int d) { return rc[(1 + l) * RA + d * L::SP]; }, Tm, Tb);
+    auto work = [&](auto edge) {
+      cell_axis<NDIM, NDIR, 1, S, C, DIVB, decltype(edge)::value>(
+          f, g, icell, own, R[0], cy, dxk, idx, inv12, ctk, valid, numax,
+          [&](int s, int d) { return fc[(s * (TY + 4) + d) * L::FYP]; },
+          [&](int p, int d) {
+            return p < 2 + NDIM ? qc[p * QA + d * L::QP]
+                                : (p == 2 + NDIM ? b0[d * L::SP] : qc[5 * QA + d * L::QP]);
+          },
+          [&](int d) { return rc[d * L::SP]; },
+          [&](int l, int d) { return rc[(1 + l) * RA + d * L::SP]; }, Tm, Tb);
+    };
+    if (y0 < g.Mlo[1] + 2 || y0 + TY - 1 > g.Mhi[1] - 2) work(Bool<true>{});
+    else work(Bool<false>{});
     // T_{1,0} of the columns left and right of the tile
     if (f.visc_on && t >= NC - 64) {
-      const int hy = t & 15, hx = (t & 16) ? TX : -1, which = (t >> 5) & 1;
-      const int hcy = y0 + hy, hcyc = (hcy > g.G[1] - 1) ? g.G[1] - 1 : hcy;
-      const C* a = which ? sm + L::B0 + (hy + HALO) * L::SP + hx + 1
-                         : sm + 2 * QA + (hy + HALO) * L::QP + hx + HALO;
+      const int hr = t & 15, hc = (t & 16) ? TX : -1, which = (t >> 5) & 1;
+      const int hcy = y0 + hr, hcyc = (hcy > g.G[1] - 1) ? g.G[1] - 1 : hcy;
+      const double* dh = f.dx[1] + hcyc;
+      const C* a = which ? sm + L::B0 + (hr + HALO) * L::SP + hc + 1
+                         : sm + 2 * QA + (hr + HALO) * L::QP + hc + HALO;
       const int st = which ? L::SP : L::QP;
       C q[7];
 #pragma unroll
       for (int s = 0; s < 7; s++) q[s] = a[(s - 3) * st];
       const bool z1 = (hcy == g.Mlo[1] && ylo) || (hcy == g.Mhi[1] && yhi);
-      Th = cross_factor<C>(q, which, z1, f.dx[1][hcyc], ctk);
+      Th = cross_factor<C>(q, which, z1, (C)dh[0], (C)dh[kDxInv * f.dxs], ctk);
     }
   }
   // The rate of other kernels, the z factors of the cell's neighbours and the
@@ -486,47 +498,62 @@ __device__ __forceinline__ bool stage_tile(const FinalArgs& f, const GridDesc& g
     for (int n = 0; n < NE; n++) R[0][n] = R[0][n] + Rin[n];
   }
   if (f.visc_on) {
-    // cross terms with derivatives along l of the factors made along k
+    // Cross terms with derivatives along l of the factors made along k.  The
+    // factors of the z lines are zero outside the mesh in memory (never
+    // written there), the tile's own are selected at the ends of the mesh.
     const C* t10 = sm + L::T10 + ty * L::SP + tx + 1;
     const C* t01 = sm + L::T01 + (ty + 1) * L::FYP + tx;
+    auto cross = [&](auto ends) {
+#pragma clang fp contract(off)
+      constexpr bool E = decltype(ends)::value;
 #pragma unroll
-    for (int l = 0; l < 2; l++) {
-      const int cl = (l == 0) ? cx : cy;
-      const bool edge = (l == 0) ? ((cx == g.Mlo[0] && xlo) || (cx == g.Mhi[0] && xhi))
-                                 : ((cy == g.Mlo[1] && ylo) || (cy == g.Mhi[1] && yhi));
-      const C h = (C)(0.5 / ((l == 0) ? dxx : dxy));
-      const bool inP = cl + 1 <= g.Mhi[l], inM = cl - 1 >= g.Mlo[l];
-      const int rs = (l == 0) ? 1 : L::SP;  // neighbour along l in the 18-wide planes
-      const int qs = (l == 0) ? 1 : L::QP;
-      const C rtp = rc[rs], rtm = rc[-rs];
+      for (int l = 0; l < 2; l++) {
+        const int cl = (l == 0) ? cx : cy;
+        const bool edge = (l == 0) ? ((cx == g.Mlo[0] && xlo) || (cx == g.Mhi[0] && xhi))
+                                   : ((cy == g.Mlo[1] && ylo) || (cy == g.Mhi[1] && yhi));
+        const C h = (l == 0) ? hx : hy;
+        const bool inP = cl + 1 <= g.Mhi[l], inM = cl - 1 >= g.Mlo[l];
+        const int rs = (l == 0) ? 1 : L::SP;  // neighbour along l in the 18-wide planes
+        const int qs = (l == 0) ? 1 : L::QP;
+        const C rtp = rc[rs], rtm = rc[-rs];
 #pragma unroll
-      for (int k = 0; k < NDIM; k++) {
-        if (k == l) continue;
-        C Tmp0, Tmm0, Tbp0, Tbm0, bkp, bkm;
-        if (k == 2) {
-          Tmp0 = Tz[4 * l], Tmm0 = Tz[4 * l + 1], Tbp0 = Tz[4 * l + 2], Tbm0 = Tz[4 * l + 3];
-          bkp = qc[5 * QA + qs], bkm = qc[5 * QA - qs];
-        } else if (l == 0) {
-          Tmp0 = t10[1], Tmm0 = t10[-1], Tbp0 = t10[TY * L::SP + 1], Tbm0 = t10[TY * L::SP - 1];
-          bkp = b1[1], bkm = b1[-1];
-        } else {
-          Tmp0 = t01[L::FYP], Tmm0 = t01[-L::FYP];
-          Tbp0 = t01[(TY + 3) * L::FYP], Tbm0 = t01[(TY + 1) * L::FYP];
-          bkp = b0[L::SP], bkm = b0[-L::SP];
+        for (int k = 0; k < NDIM; k++) {
+          if (k == l) continue;
+          C Tmp, Tmm, Tbp, Tbm, bkp, bkm;
+          if (k == 2) {
+            Tmp = Tz[4 * l], Tmm = Tz[4 * l + 1], Tbp = Tz[4 * l + 2], Tbm = Tz[4 * l + 3];
+            bkp = qc[5 * QA + qs], bkm = qc[5 * QA - qs];
+          } else if (l == 0) {
+            Tmp = t10[1], Tmm = t10[-1], Tbp = t10[TY * L::SP + 1], Tbm = t10[TY * L::SP - 1];
+            bkp = b1[1], bkm = b1[-1];
+          } else {
+            Tmp = t01[L::FYP], Tmm = t01[-L::FYP];
+            Tbp = t01[(TY + 3) * L::FYP], Tbm = t01[(TY + 1) * L::FYP];
+            bkp = b0[L::SP], bkm = b0[-L::SP];
+          }
+          if constexpr (E) {
+            if (k < 2) {
+              Tmp = inP ? Tmp : (C)0, Tmm = inM ? Tmm : (C)0;
+              Tbp = inP ? Tbp : (C)0, Tbm = inM ? Tbm : (C)0;
+            }
+          }
+          const C mkp = rc[(1 + k) * RA + rs], mkm = rc[(1 + k) * RA - rs];
+          const C dm = fma_(rtp, Tmp, -(rtm * Tmm)) * h;
+          const C de1 = fma_(mkp, Tmp, -(mkm * Tmm)) * h;
+          const C db = (Tbp - Tbm) * h;
+          const C de2 = fma_(Tbp, bkp, -(Tbm * bkm)) * h;
+          const bool no = E && edge;
+          R[0][1 + k] += no ? (C)0 : dm;
+          R[0][1 + NDIR] += no ? (C)0 : de1;
+          R[0][2 + NDIR + k] -= no ? (C)0 : db;
+          R[0][1 + NDIR] -= no ? (C)0 : de2;
         }
-        const C Tmp = inP ? Tmp0 : (C)0, Tmm = inM ? Tmm0 : (C)0;
-        const C Tbp = inP ? Tbp0 : (C)0, Tbm = inM ? Tbm0 : (C)0;
-        const C mkp = rc[(1 + k) * RA + rs], mkm = rc[(1 + k) * RA - rs];
-        const C dm = (rtp * Tmp - rtm * Tmm) * h;
-        const C de1 = (mkp * Tmp - mkm * Tmm) * h;
-        const C db = (Tbp - Tbm) * h;
-        const C de2 = (Tbp * bkp - Tbm * bkm) * h;
-        R[0][1 + k] += edge ? (C)0 : dm;
-        R[0][1 + NDIR] += edge ? (C)0 : de1;
-        R[0][2 + NDIR + k] -= edge ? (C)0 : db;
-        R[0][1 + NDIR] -= edge ? (C)0 : de2;
       }
-    }
+    };
+    if (x0 <= g.Mlo[0] || x0 + TX > g.Mhi[0] || y0 <= g.Mlo[1] || y0 + TY > g.Mhi[1])
+      cross(Bool<true>{});
+    else
+      cross(Bool<false>{});
   }
   c[0] = cx;
   c[1] = cy;
@@ -546,6 +573,87 @@ __device__ __forceinline__ bool stage_tile(const FinalArgs& f, const GridDesc& g
   }
   update_cell<NDIM, NDIR, S, C, RK4L>(f, g, c, icell, base, own, R[0], redv);
   return true;
+}
+
+// ---------------------------------------------------------------------
+// 3-D: the factors T_{0,2} and T_{1,2} of a tile's cells, made along x and y
+// from v_2 and b_2, which the z line tiles differentiate along z.  Making
+// them in a pass of its own (4 fields read, 4 written) lets the z pass come
+// before the x and y work, whose kernel can then finish the cell: the rate of
+// x and y stays in registers and there is no combining pass.  A stage at
+// 256^3 in FP64: plane tiles 1.84 ms, z lines 1.29, update 1.10 (1.68 RK4's
+// last); now factors 0.27, z lines 0.97, this file's tiles 2.07 (2.37).  At
+// 128^3: 0.266 + 0.177 + 0.158 (0.222), now 0.041 + 0.146 + 0.270 (0.319).
+template <typename C>
+struct TzSmem {
+  C v[2][PY][PX];  // v_2, b_2
+};
+
+template <typename S, typename C>
+__device__ __forceinline__ void tz_tile(const AxisArgs& a, int x0, int y0, int z, TzSmem<C>& sm) {
+  constexpr int NDIM = 3, NDIR = 3;
+  const GridDesc& g = a.g;
+  const long long fs = g.fs, zoff = (long long)z * g.st[2];
+  const int t = (int)threadIdx.x;
+  const int tx = t % TX, ty = cell_row<C>(t);
+  const int cx = x0 + tx, cy = y0 + ty;
+  const int cxc = (cx > g.G[0] - 1) ? g.G[0] - 1 : cx;
+  const int cyc = (cy > g.G[1] - 1) ? g.G[1] - 1 : cy;
+  const C dxx = (C)a.dx[0][cxc], dxy = (C)a.dx[1][cyc];
+  const C ix0 = (C)a.dx[0][kDxInv * a.dxs + cxc], iy0 = (C)a.dx[1][kDxInv * a.dxs + cyc];
+  const C ctx = (C)red_get(a.ctot_src, 0), cty = (C)red_get(a.ctot_src, 1);
+  const int yb = y0 > HALO ? y0 - HALO : 0;
+  const long long ob = zoff + yb * g.st[1];
+  const S* __restrict__ W = (const S*)a.wct + ob;
+  const double* __restrict__ B = a.bg + ob;
+  // the tile's points, then the columns and rows beside it (as in stage_tile)
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    int ix = tx + HALO, iy = ty + HALO;
+    if (k == 1) {
+      if (t >= 192) break;
+      if (t < 96) {
+        const int r = t / 6, u = t - 6 * r;
+        ix = u < 3 ? u : u + TX;
+        iy = r + HALO;
+      } else {
+        const int u = (t - 96) / TX;
+        ix = (t - 96) % TX + HALO;
+        iy = u < 3 ? u : u + TY;
+      }
+    }
+    int gx = x0 - HALO + ix, gy = y0 - HALO + iy;
+    if (gx < 0) gx = g.Mlo[0] + 3;
+    if (gx > g.G[0] - 1) gx = g.Mhi[0] - 3;
+    if (gy < 0) gy = g.Mlo[1] + 3;
+    if (gy > g.G[1] - 1) gy = g.Mhi[1] - 3;
+    const unsigned i = (unsigned)(gy - yb) * (unsigned)g.st[1] + (unsigned)gx;
+    const unsigned ow = i * (unsigned)sizeof(S), o8 = i * 8u;
+    auto wv = [&](int n) { return (C) * (const S*)((const char*)(W + (size_t)n * fs) + ow); };
+    const C rho = wv(0), m = wv(1 + 2), b = wv(2 + NDIR + 2);
+    const double rhob = *(const double*)((const char*)(B + fs) + o8);
+    sm.v[0][iy][ix] = m * (C)recip<C>((double)rho + rhob);  // nothing to contract
+    sm.v[1][iy][ix] = b;
+  }
+  __syncthreads();
+  if (cx < g.Mlo[0] || cx > g.Mhi[0] || cy > g.Mhi[1]) return;
+  const bool zx = (cx == g.Mlo[0] && !g.per_lo[0]) || (cx == g.Mhi[0] && !g.per_hi[0]);
+  const bool zy = (cy == g.Mlo[1] && !g.per_lo[1]) || (cy == g.Mhi[1] && !g.per_hi[1]);
+  const long long icell = zoff + (long long)cy * g.st[1] + cx;
+  S* __restrict__ T = (S*)a.T;
+#pragma unroll
+  for (int w = 0; w < 2; w++) {
+    const C* q0 = &sm.v[w][ty + HALO][tx + HALO];
+    C q[7];
+#pragma unroll
+    for (int s = 0; s < 7; s++) q[s] = q0[s - 3];
+    T[(long long)(cross_index(NDIM, 0, 2) + w) * fs + icell] =
+        (S)cross_factor<C>(q, w, zx, dxx, ix0, ctx);
+#pragma unroll
+    for (int s = 0; s < 7; s++) q[s] = q0[(s - 3) * PX];
+    T[(long long)(cross_index(NDIM, 1, 2) + w) * fs + icell] =
+        (S)cross_factor<C>(q, w, zy, dxy, iy0, cty);
+  }
 }
 
 }  // namespace tile
