@@ -15,6 +15,7 @@
 #include "../../include/sac_amd.h"
 #include "sac_closure.h"
 #include "sac_kernels.h"
+#include "sac_xfer.h"
 
 namespace {
 
@@ -118,7 +119,7 @@ struct Dev {
   // combine overwrites it
   bool visc_taken = false;
   bool red_valid[kSlots] = {false, false, false, false};
-  std::vector<double> stage;  // host staging
+  void* pin = nullptr;  // pinned buffer of small copies (sac_xfer.h)
   long long bytes = 0;
   bool timing = false;
   std::vector<TimedLaunch> timed;
@@ -420,53 +421,22 @@ int check_handle(sac_handle h) {
   return 0;
 }
 
-// host (unpadded, FP64) <-> device (padded rows, element size esz) copies of
-// nfield fields; FP32 device fields are converted on the host, one field at
-// a time
-int copy_in(Dev& d, void* dst, const double* src, int nfield, size_t esz) {
-  const size_t w = esz * (size_t)d.g.G[0];
-  const size_t spitch = w;
-  const size_t dpitch = esz * (size_t)d.g.st[1];
-  const size_t rows = (size_t)d.g.G[1] * (size_t)d.g.G[2];
-  std::vector<float> tmp;
-  for (int f = 0; f < nfield; f++) {
-    const double* s = src + (size_t)f * d.ncell_grid;
-    char* dp = (char*)dst + esz * (size_t)f * d.g.fs;
-    if (esz == sizeof(double)) {
-      HIPCHK(hipMemcpy2DAsync(dp, dpitch, s, spitch, w, rows, hipMemcpyHostToDevice, d.stream));
-    } else {
-      tmp.resize((size_t)d.ncell_grid);
-      for (long long i = 0; i < d.ncell_grid; i++) tmp[i] = (float)s[i];
-      HIPCHK(hipMemcpy2DAsync(dp, dpitch, tmp.data(), spitch, w, rows, hipMemcpyHostToDevice,
-                              d.stream));
-      HIPCHK(hipStreamSynchronize(d.stream));
-    }
-  }
-  HIPCHK(hipStreamSynchronize(d.stream));
-  return 0;
+// register `slot` and, with bg, the background, to or from the host array w
+// (register fields, then background fields)
+int copy_state(Dev& d, int slot, bool bg, double* w, bool to_host) {
+  const sac::xfer::Fields f[2] = {
+      {d.reg[slot], (int)d.esz, d.ne, w},
+      {d.bg, (int)sizeof(double), d.nbg, w + (size_t)d.ne * d.ncell_grid}};
+  std::string err;
+  const int rc = sac::xfer::copy(d.g, d.device, d.stream, f, bg ? 2 : 1, to_host, &d.pin, err);
+  return rc ? fail(rc, "%s", err.c_str()) : 0;
 }
 
-int copy_out(Dev& d, double* dst, const void* src, int nfield, size_t esz) {
-  const size_t w = esz * (size_t)d.g.G[0];
-  const size_t dpitch = w;
-  const size_t spitch = esz * (size_t)d.g.st[1];
-  const size_t rows = (size_t)d.g.G[1] * (size_t)d.g.G[2];
-  std::vector<float> tmp;
-  for (int f = 0; f < nfield; f++) {
-    double* o = dst + (size_t)f * d.ncell_grid;
-    const char* sp = (const char*)src + esz * (size_t)f * d.g.fs;
-    if (esz == sizeof(double)) {
-      HIPCHK(hipMemcpy2DAsync(o, dpitch, sp, spitch, w, rows, hipMemcpyDeviceToHost, d.stream));
-    } else {
-      tmp.resize((size_t)d.ncell_grid);
-      HIPCHK(hipMemcpy2DAsync(tmp.data(), dpitch, sp, spitch, w, rows, hipMemcpyDeviceToHost,
-                              d.stream));
-      HIPCHK(hipStreamSynchronize(d.stream));
-      for (long long i = 0; i < d.ncell_grid; i++) o[i] = (double)tmp[i];
-    }
-  }
-  HIPCHK(hipStreamSynchronize(d.stream));
-  return 0;
+int copy_bg_out(Dev& d, double* dst) {
+  const sac::xfer::Fields f = {d.bg, (int)sizeof(double), d.nbg, dst};
+  std::string err;
+  const int rc = sac::xfer::copy(d.g, d.device, d.stream, &f, 1, true, &d.pin, err);
+  return rc ? fail(rc, "%s", err.c_str()) : 0;
 }
 
 // `n` reduction words from p on, on the host (one copy, one wait), or as
@@ -713,6 +683,7 @@ int sac_dev_free(sac_handle h) {
   hipFree(d->dx_all);
   hipFree(d->red);
   if (d->red_host) hipHostFree(d->red_host);
+  if (d->pin) hipHostFree(d->pin);
   if (d->cl) {
     Closure* c = d->cl;
     hipFree(c->P32);
@@ -741,8 +712,7 @@ int sac_dev_upload(sac_handle h, const double* w) {
   if (int rc = check_handle(h)) return rc;
   if (!w) return fail(SAC_E_ARG, "w is null");
   Dev& d = *(Dev*)h;
-  if (int rc = copy_in(d, d.reg[SAC_SLOT_W], w, d.ne, d.esz)) return rc;
-  if (int rc = copy_in(d, d.bg, w + (size_t)d.ne * d.ncell_grid, d.nbg, sizeof(double))) return rc;
+  if (int rc = copy_state(d, SAC_SLOT_W, true, const_cast<double*>(w), false)) return rc;
   d.red_valid[SAC_SLOT_W] = false;
   d.bg_host.clear();  // the ghosts of the background change at the next getboundary
   d.bg_ghosts_stale = d.initialized;
@@ -753,8 +723,7 @@ int sac_dev_download(sac_handle h, double* w) {
   if (int rc = check_handle(h)) return rc;
   if (!w) return fail(SAC_E_ARG, "w is null");
   Dev& d = *(Dev*)h;
-  if (int rc = copy_out(d, w, d.reg[SAC_SLOT_W], d.ne, d.esz)) return rc;
-  return copy_out(d, w + (size_t)d.ne * d.ncell_grid, d.bg, d.nbg, sizeof(double));
+  return copy_state(d, SAC_SLOT_W, true, w, true);
 }
 
 int sac_dev_upload_slot(sac_handle h, int slot, const double* w) {
@@ -762,15 +731,14 @@ int sac_dev_upload_slot(sac_handle h, int slot, const double* w) {
   if (slot < 0 || slot >= kSlots || !w) return fail(SAC_E_ARG, "bad slot %d", slot);
   Dev& d = *(Dev*)h;
   d.red_valid[slot] = false;
-  return copy_in(d, d.reg[slot], w, d.ne, d.esz);
+  return copy_state(d, slot, false, const_cast<double*>(w), false);
 }
 
 int sac_dev_download_slot(sac_handle h, int slot, double* w) {
   if (int rc = check_handle(h)) return rc;
   if (slot < 0 || slot >= kSlots || !w) return fail(SAC_E_ARG, "bad slot %d", slot);
   Dev& d = *(Dev*)h;
-  if (int rc = copy_out(d, w, d.reg[slot], d.ne, d.esz)) return rc;
-  return copy_out(d, w + (size_t)d.ne * d.ncell_grid, d.bg, d.nbg, sizeof(double));
+  return copy_state(d, slot, true, w, true);
 }
 
 // ---------------------------------------------------------------------
@@ -783,32 +751,25 @@ int sac_dev_save_begin(sac_handle h) {
   if (int rc = check_handle(h)) return rc;
   Dev& d = *(Dev*)h;
   if (d.save_pending) return fail(SAC_E_ARG, "a save is already in progress");
-  const size_t fbytes = d.esz * (size_t)d.g.fs;
+  const size_t bytes = d.esz * (size_t)d.ncell_grid * (size_t)d.ne;
   if (!d.save_stream) {
     HIPCHK(hipStreamCreateWithFlags(&d.save_stream, hipStreamNonBlocking));
     HIPCHK(hipEventCreateWithFlags(&d.save_taken, hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&d.save_done, hipEventDisableTiming));
-    if (int rc = balloc(d, &d.save_dev, fbytes * (size_t)d.ne)) return rc;
-    HIPCHK(hipHostMalloc(&d.save_host, d.esz * (size_t)d.ncell_grid * (size_t)d.ne,
-                         hipHostMallocDefault));
+    if (int rc = balloc(d, &d.save_dev, bytes)) return rc;
+    HIPCHK(hipHostMalloc(&d.save_host, bytes, hipHostMallocDefault));
   }
   if (d.bg_host.empty()) {  // the background is static: one synchronous copy
     d.bg_host.resize((size_t)d.nbg * (size_t)d.ncell_grid);
-    if (int rc = copy_out(d, d.bg_host.data(), d.bg, d.nbg, sizeof(double))) return rc;
+    if (int rc = copy_bg_out(d, d.bg_host.data())) return rc;
   }
-  HIPCHK(hipMemcpyAsync(d.save_dev, d.reg[SAC_SLOT_W], fbytes * (size_t)d.ne,
-                        hipMemcpyDeviceToDevice, d.stream));
+  // the snapshot in the host's layout, so that one plain copy takes it over
+  const sac::xfer::Fields f = {d.reg[SAC_SLOT_W], (int)d.esz, d.ne, nullptr};
+  sac::xfer::launch_pack(d.g, f, d.save_dev, d.stream);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(d.save_taken, d.stream));
   HIPCHK(hipStreamWaitEvent(d.save_stream, d.save_taken, 0));
-  const size_t w = d.esz * (size_t)d.g.G[0];
-  const size_t spitch = d.esz * (size_t)d.g.st[1];
-  const size_t rows = (size_t)d.g.G[1] * (size_t)d.g.G[2];
-  for (int f = 0; f < d.ne; f++) {
-    char* dst = (char*)d.save_host + d.esz * (size_t)f * (size_t)d.ncell_grid;
-    const char* src = (const char*)d.save_dev + fbytes * (size_t)f;
-    HIPCHK(hipMemcpy2DAsync(dst, w, src, spitch, w, rows, hipMemcpyDeviceToHost,
-                            d.save_stream));
-  }
+  HIPCHK(hipMemcpyAsync(d.save_host, d.save_dev, bytes, hipMemcpyDeviceToHost, d.save_stream));
   HIPCHK(hipEventRecord(d.save_done, d.save_stream));
   d.save_pending = true;
   return 0;
@@ -834,13 +795,11 @@ int sac_dev_save_end(sac_handle h, double* w) {
   d.save_pending = false;
   HIPCHK(hipEventSynchronize(d.save_done));
   const size_t n = (size_t)d.ne * (size_t)d.ncell_grid;
-  if (d.esz == sizeof(double)) {
-    memcpy(w, d.save_host, sizeof(double) * n);
-  } else {
-    const float* s = (const float*)d.save_host;
-    for (size_t i = 0; i < n; i++) w[i] = (double)s[i];
-  }
-  memcpy(w + n, d.bg_host.data(), sizeof(double) * d.bg_host.size());
+  if (d.esz == sizeof(double))
+    sac::xfer::host_copy(w, (const double*)d.save_host, n);
+  else
+    sac::xfer::host_copy(w, (const float*)d.save_host, n);
+  sac::xfer::host_copy(w + n, d.bg_host.data(), d.bg_host.size());
   return 0;
 }
 

@@ -32,6 +32,7 @@
 #include "../../include/sac_amd.h"
 #include "sac_device.h"
 #include "sac_tile.h"
+#include "sac_xfer.h"
 
 namespace sac {
 namespace batch {
@@ -383,6 +384,22 @@ __global__ void kb_tick(Args a) {
 
 __global__ void kb_zero_u32(unsigned int* p) { *p = 0u; }
 
+// The state of tubes m0.. in the host's layout (per tube the NE + NBG fields,
+// unpadded, from element off[tube] of the whole) to `out`, which holds it from
+// element off[m0] on: one block per tube and field.
+__global__ void __launch_bounds__(256) kb_pack(Args a, const long long* off, int m0, double* out) {
+  const int tube = m0 + (int)blockIdx.x / (NE + NBG), v = (int)blockIdx.x % (NE + NBG);
+  const unsigned G0 = (unsigned)a.nxy[2 * tube] + 4;
+  const unsigned G1 = a.ndim == 2 ? (unsigned)a.nxy[2 * tube + 1] + 4 : 1;
+  const long long p = a.pitch[tube], n = (long long)G0 * G1;
+  const double* f = (v < NE ? a.reg[SAC_SLOT_W] + v * a.fs : a.bg + (v - NE) * a.fs) + a.start[tube];
+  double* o = out + (off[tube] - off[m0]) + v * n;
+  for (long long i = threadIdx.x; i < n; i += 256) {
+    const long long r = (n >> 32) ? i / G0 : (long long)((unsigned)i / G0);
+    o[i] = f[r * p + (i - r * G0)];
+  }
+}
+
 }  // namespace batch
 }  // namespace sac
 
@@ -454,6 +471,8 @@ struct Batch {
   int* d_it = nullptr;
   int* d_state = nullptr;
   double* d_dxmin = nullptr;
+  std::vector<long long> hoff;   // element of each tube in the host's layout, and the end
+  long long* d_hoff = nullptr;
   unsigned int* d_running = nullptr;
   Shape shape{2, 128, 0};
   int ntiles = 0;
@@ -862,6 +881,7 @@ int sac_batch_free(sac_batch_handle h) {
   hipFree(b->d_it);
   hipFree(b->d_state);
   hipFree(b->d_dxmin);
+  hipFree(b->d_hoff);
   hipFree(b->d_running);
   if (b->stream) hipStreamDestroy(b->stream);
   delete b;
@@ -1001,21 +1021,43 @@ int sac_batch_status(sac_batch_handle h, double* t, int* it, int* state) {
 int sac_batch_download(sac_batch_handle h, double* w) {
   if (!h || !w) return bfail(SAC_E_ARG, "null argument");
   Batch& b = *(Batch*)h;
-  BCHK(hipStreamSynchronize(b.stream));
-  const size_t fb = sizeof(double) * (size_t)b.fs;
-  std::vector<double> pk((size_t)b.fs * (NE + NBG));
-  BCHK(hipMemcpy(pk.data(), b.d_reg[SAC_SLOT_W], fb * NE, hipMemcpyDeviceToHost));
-  BCHK(hipMemcpy(pk.data() + (size_t)b.fs * NE, b.d_bg, fb * NBG, hipMemcpyDeviceToHost));
-  long long hoff = 0;
-  for (int i = 0; i < b.ntubes; i++) {
-    const int G0 = b.gx(i), G1 = b.gy(i);
-    for (int v = 0; v < NE + NBG; v++)
-      for (int r = 0; r < G1; r++)
-        memcpy(w + hoff + ((size_t)v * G1 + r) * G0,
-               &pk[(size_t)v * b.fs + b.start[i] + (size_t)r * b.pitch[i]], sizeof(double) * G0);
-    hoff += (long long)G0 * G1 * (NE + NBG);
+  // Chunks of consecutive members through pinned buffers (sac_xfer.h); a
+  // member larger than a buffer gets one of its size.
+  if (!b.d_hoff) {
+    b.hoff.assign((size_t)b.ntubes + 1, 0);
+    for (int i = 0; i < b.ntubes; i++)
+      b.hoff[i + 1] = b.hoff[i] + (long long)b.gx(i) * b.gy(i) * (NE + NBG);
+    if (int rc = balloc(b, (void**)&b.d_hoff, sizeof(long long) * b.hoff.size())) return rc;
+    BCHK(hipMemcpy(b.d_hoff, b.hoff.data(), sizeof(long long) * b.hoff.size(),
+                   hipMemcpyHostToDevice));
   }
-  return 0;
+  constexpr long long kMost = (4LL << 20) / sizeof(double);
+  std::vector<int> first(1, 0);
+  long long most = 0;
+  for (int i = 0; i < b.ntubes;) {
+    int j = i + 1;
+    while (j < b.ntubes && b.hoff[j + 1] - b.hoff[i] <= kMost) j++;
+    most = std::max(most, b.hoff[j] - b.hoff[i]);
+    first.push_back(i = j);
+  }
+  std::string err;
+  const int rc = sac::xfer::for_chunks(
+      b.device, (long long)first.size() - 1, sizeof(double) * (size_t)most,
+      [&](long long c, void* pin, hipEvent_t ev, std::string& e) -> int {
+        const int m0 = first[c], m1 = first[c + 1];
+        hipLaunchKernelGGL(kb_pack, dim3((unsigned)(m1 - m0) * (NE + NBG)), dim3(256), 0, b.stream,
+                           b.a, b.d_hoff, m0, (double*)pin);
+        hipError_t s = hipEventRecord(ev, b.stream);
+        if (s == hipSuccess) s = hipEventSynchronize(ev);
+        if (s != hipSuccess) {
+          e = std::string("download: ") + hipGetErrorString(s);
+          return SAC_E_HIP;
+        }
+        memcpy(w + b.hoff[m0], pin, sizeof(double) * (size_t)(b.hoff[m1] - b.hoff[m0]));
+        return 0;
+      },
+      err);
+  return rc ? bfail(rc, "%s", err.c_str()) : 0;
 }
 
 int sac_batch_memory(sac_batch_handle h, long long* bytes) {

@@ -1,0 +1,245 @@
+// sac_xfer.hip -- states between host memory and the device (sac_xfer.h).
+//
+// The host keeps unpadded arrays in ordinary memory, the device padded rows.
+// A 2-D copy between the two (hipMemcpy2D) moved row after row through the
+// runtime's own staging, about 9 us a row: 8.0 s up and 6.1 s down for a
+// 256^3 state of 1.85 GB, 0.16 and 0.11 s for 32^3.  Here the state goes in
+// chunks: a kernel reads or writes the padded rows and a pinned buffer in the
+// host's order (over the bus, coalesced), and a few host threads, each with a
+// buffer of its own, copy between the buffers and the caller's array while
+// the other chunks move.  One thread alone fills fresh pages at 2.7 GB/s, the
+// bus takes 57.  Now 36 ms up and 37 ms down for the 256^3 state, 0.4 and 0.5 ms for
+// 31x27x35 (0.16 and 0.11 s before), 12 ms for the states of 4096 tubes (150).
+#include "sac_xfer.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstdint>
+#include <cstring>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+#include "../../include/sac_amd.h"
+
+namespace sac {
+namespace xfer {
+
+namespace {
+
+constexpr int kWorkers = 8;
+constexpr size_t kChunk = size_t(4) << 20;  // bytes of a pinned buffer
+
+// n elements in host order from element x0 of row R0 on (rows of all fields
+// counted through), between padded rows and contiguous memory
+template <typename T, bool OUT>
+__global__ void __launch_bounds__(256) k_rows(T* dev, T* flat, unsigned n, unsigned x0, unsigned R0,
+                                              unsigned G0, unsigned rows, long long pitch,
+                                              long long fs) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  const unsigned r = (x0 + i) / G0, x = x0 + i - r * G0;
+  const unsigned R = R0 + r, f = R / rows;
+  T* p = dev + (long long)f * fs + (long long)(R - f * rows) * pitch + x;
+  if (OUT)
+    flat[i] = *p;
+  else
+    *p = flat[i];
+}
+
+template <bool OUT>
+void launch_rows(const GridDesc& g, const Fields& f, long long first, unsigned n, void* flat,
+                 hipStream_t st) {
+  const unsigned G0 = (unsigned)g.G[0], rows = (unsigned)g.G[1] * (unsigned)g.G[2];
+  const unsigned R0 = (unsigned)(first / G0), x0 = (unsigned)(first % G0);
+  const dim3 nb((n + 255) / 256), bs(256);
+  if (f.esz == 8)
+    hipLaunchKernelGGL((k_rows<uint64_t, OUT>), nb, bs, 0, st, (uint64_t*)f.dev, (uint64_t*)flat, n,
+                       x0, R0, G0, rows, g.st[1], g.fs);
+  else
+    hipLaunchKernelGGL((k_rows<uint32_t, OUT>), nb, bs, 0, st, (uint32_t*)f.dev, (uint32_t*)flat, n,
+                       x0, R0, G0, rows, g.st[1], g.fs);
+}
+
+// fn(begin, end) on slices of [0, n), on several threads where it pays
+template <typename F>
+void parallel_slices(size_t n, size_t per_thread, const F& fn) {
+  const size_t hw = std::max(1u, std::thread::hardware_concurrency());
+  const size_t nt = std::min<size_t>({(size_t)kWorkers, hw, n / per_thread + 1});
+  std::vector<std::thread> th;
+  auto slice = [&](size_t t) { fn(n * t / nt, n * (t + 1) / nt); };
+  size_t t = 1;
+  try {
+    for (; t < nt; t++) th.emplace_back(slice, t);
+  } catch (const std::system_error&) {  // no more threads: the rest here
+  }
+  slice(0);
+  for (; t < nt; t++) slice(t);
+  for (auto& x : th) x.join();
+}
+
+// between the host's FP64 and a buffer of elements of esz bytes
+void from_pinned(double* h, const void* pin, int esz, size_t m) {
+  if (esz == 8) {
+    memcpy(h, pin, sizeof(double) * m);
+  } else {
+    const float* p = (const float*)pin;
+    for (size_t i = 0; i < m; i++) h[i] = (double)p[i];
+  }
+}
+void to_pinned(void* pin, const double* h, int esz, size_t m) {
+  if (esz == 8) {
+    memcpy(pin, h, sizeof(double) * m);
+  } else {
+    float* p = (float*)pin;
+    for (size_t i = 0; i < m; i++) p[i] = (float)h[i];
+  }
+}
+
+int hip_err(hipError_t e, const char* what, std::string& err) {
+  if (e == hipSuccess) return 0;
+  err = std::string(what) + ": " + hipGetErrorString(e);
+  return SAC_E_HIP;
+}
+
+}  // namespace
+
+void host_copy(double* dst, const double* src, size_t n) {
+  parallel_slices(n, size_t(1) << 18, [&](size_t b, size_t e) {
+    memcpy(dst + b, src + b, sizeof(double) * (e - b));
+  });
+}
+
+void host_copy(double* dst, const float* src, size_t n) {
+  parallel_slices(n, size_t(1) << 18, [&](size_t b, size_t e) {
+    for (size_t i = b; i < e; i++) dst[i] = (double)src[i];
+  });
+}
+
+int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::string& err) {
+  if (n <= 0) return 0;
+  const long long hw = std::max(1u, std::thread::hardware_concurrency());
+  const int nt = (int)std::min<long long>({(long long)kWorkers, hw, n});
+  std::vector<std::string> errs((size_t)nt);
+  std::vector<int> rcs((size_t)nt, 0);
+  std::atomic<long long> next{0};
+  std::atomic<bool> stop{false};
+  auto worker = [&](int t) {
+    void* pin = nullptr;
+    hipEvent_t ev = nullptr;
+    int rc = hip_err(hipSetDevice(device), "hipSetDevice", errs[t]);
+    if (!rc && hipHostMalloc(&pin, bytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      if (t > 0) return;  // the other threads take the chunks
+      errs[t] = "no pinned memory";
+      rc = SAC_E_NOMEM;
+    }
+    if (!rc) rc = hip_err(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate", errs[t]);
+    while (!rc && !stop) {
+      const long long c = next.fetch_add(1);
+      if (c >= n) break;
+      rc = fn(c, pin, ev, errs[t]);
+    }
+    // the buffer's last chunk may still be on its way to the device
+    if (ev) {
+      const int e = hip_err(hipEventSynchronize(ev), "hipEventSynchronize", errs[t]);
+      if (!rc) rc = e;
+      hipEventDestroy(ev);
+    }
+    if (pin) hipHostFree(pin);
+    if (rc) stop = true;
+    rcs[t] = rc;
+  };
+  std::vector<std::thread> th;
+  try {
+    for (int t = 1; t < nt; t++) th.emplace_back(worker, t);
+  } catch (const std::system_error&) {  // the threads there are take the chunks
+  }
+  worker(0);
+  for (auto& x : th) x.join();
+  for (int t = 0; t < nt; t++)
+    if (rcs[t]) {
+      err = errs[t];
+      return rcs[t];
+    }
+  return 0;
+}
+
+// a copy that fits one buffer: all groups' kernels, one wait (a tube of
+// 800 cells: 20 us each way, 180 with a thread and a buffer of its own)
+static int copy_small(const GridDesc& g, hipStream_t stream, const Fields* f, int n, bool to_host,
+                      void** small, std::string& err) {
+  const size_t ncell = (size_t)g.G[0] * g.G[1] * g.G[2];
+  if (!*small && hipHostMalloc(small, kSmall, hipHostMallocDefault) != hipSuccess) {
+    *small = nullptr;
+    err = "no pinned memory";
+    return SAC_E_NOMEM;
+  }
+  size_t at = 0;
+  for (int k = 0; k < n; k++) {
+    const size_t m = ncell * f[k].nfield;
+    char* p = (char*)*small + at;
+    if (to_host) {
+      launch_rows<true>(g, f[k], 0, (unsigned)m, p, stream);
+    } else {
+      to_pinned(p, f[k].host, f[k].esz, m);
+      launch_rows<false>(g, f[k], 0, (unsigned)m, p, stream);
+    }
+    at += (m * f[k].esz + 15) / 16 * 16;
+  }
+  if (int rc = hip_err(hipStreamSynchronize(stream), "copy", err)) return rc;
+  at = 0;
+  for (int k = 0; k < n && to_host; k++) {
+    const size_t m = ncell * f[k].nfield;
+    from_pinned(f[k].host, (char*)*small + at, f[k].esz, m);
+    at += (m * f[k].esz + 15) / 16 * 16;
+  }
+  return hip_err(hipGetLastError(), "copy kernels", err);
+}
+
+int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n, bool to_host,
+         void** small, std::string& err) {
+  const long long ncell = (long long)g.G[0] * g.G[1] * g.G[2];
+  size_t all = 0;
+  for (int k = 0; k < n; k++) all += (size_t)ncell * f[k].nfield * f[k].esz + 16;
+  if (small && all <= kSmall) return copy_small(g, stream, f, n, to_host, small, err);
+  // chunks of each group, one after another
+  std::vector<long long> first((size_t)n + 1, 0);
+  size_t bytes = 0;
+  for (int k = 0; k < n; k++) {
+    const long long total = ncell * f[k].nfield, per = (long long)(kChunk / f[k].esz);
+    first[k + 1] = first[k] + (total + per - 1) / per;
+    bytes = std::max(bytes, (size_t)std::min(total, per) * f[k].esz);
+  }
+  auto fn = [&](long long c, void* pin, hipEvent_t ev, std::string& e) -> int {
+    const int k = (int)(std::upper_bound(first.begin(), first.end(), c) - first.begin()) - 1;
+    const Fields& s = f[k];
+    const long long per = (long long)(kChunk / s.esz), lo = (c - first[k]) * per;
+    const unsigned m = (unsigned)std::min(per, ncell * s.nfield - lo);
+    double* h = s.host + lo;
+    if (to_host) {
+      launch_rows<true>(g, s, lo, m, pin, stream);
+      if (int rc = hip_err(hipEventRecord(ev, stream), "hipEventRecord", e)) return rc;
+      if (int rc = hip_err(hipEventSynchronize(ev), "download", e)) return rc;
+      from_pinned(h, pin, s.esz, m);
+      return 0;
+    }
+    // the buffer is free once its previous chunk has been read
+    if (int rc = hip_err(hipEventSynchronize(ev), "upload", e)) return rc;
+    to_pinned(pin, h, s.esz, m);
+    launch_rows<false>(g, s, lo, m, pin, stream);
+    return hip_err(hipEventRecord(ev, stream), "hipEventRecord", e);
+  };
+  if (int rc = for_chunks(device, first[n], bytes, fn, err)) return rc;
+  return hip_err(hipGetLastError(), "copy kernels", err);
+}
+
+void launch_pack(const GridDesc& g, const Fields& f, void* out, hipStream_t stream) {
+  const long long ncell = (long long)g.G[0] * g.G[1] * g.G[2], total = ncell * f.nfield;
+  const long long per = 1LL << 30;  // elements of a launch (32-bit thread numbers)
+  for (long long lo = 0; lo < total; lo += per)
+    launch_rows<true>(g, f, lo, (unsigned)std::min(per, total - lo), (char*)out + lo * f.esz, stream);
+}
+
+}  // namespace xfer
+}  // namespace sac
