@@ -332,21 +332,20 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
     t_end(d, SAC_K_PLANE, e0);
   }
   x.fresh = stage3 ? 1 : 0;
+  if (learned) {
+    hipEvent_t ei{};
+    t_begin(d, SAC_K_CLOSURE, &ei);
+    sac::closure::launch_infer(d.ndim, d.ndir, d.g, (const double*)d.reg[wct], d.bg, d.gamma,
+                               d.cl->sensor, d.cl->P16, d.cl->P32, d.cl->RF, d.cl->on, d.stream);
+    t_end(d, SAC_K_CLOSURE, ei);
+  }
   for (int k = stage3 ? 2 : 0; k < d.ndim && !stage1 && !stage2; k++) {
     // axis 1 (rows of a plane): neighbour rows in one XCD's L2.  Axes 0 and 2
     // keep the hardware order, whose round-robin already places the
     // neighbour planes of a row in the same XCD.
     x.xcd = (k == 1) ? d.xcd : 1;
     x.RF = nullptr;
-    if (learned) {
-      hipEvent_t ei{};
-      t_begin(d, SAC_K_CLOSURE, &ei);
-      sac::closure::launch_infer(d.ndim, d.ndir, k, d.g, (const double*)d.reg[wct], d.bg, d.gamma,
-                                 d.cl->sensor, d.cl->P16, d.cl->P32, d.cl->RF[k], d.cl->on,
-                                 d.stream);
-      t_end(d, SAC_K_CLOSURE, ei);
-      x.RF = d.cl->RF[k];
-    }
+    if (learned) x.RF = d.cl->RF[k];
     x.cross_last = (k == d.ndim - 1) ? 1 : 0;
     x.divbfix = d.divbfix;
     hipEvent_t e0{};

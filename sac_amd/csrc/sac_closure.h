@@ -45,13 +45,14 @@ void launch_adam(float* P32, uint16_t* P16, float* m1, float* m2, const float* p
 // BF16 copy of FP32 parameters.
 void launch_to_bf16(const float* P32, uint16_t* P16, hipStream_t st);
 
-// Inference for axis K on state w: face ratios for the 2*ndim+1 variables
-// of setnu on that axis (order rho', thermal energy, v_0.., b_l (l != K)),
-// stored at the face's left cell, or -1 where the exact ratio is to be used.
-// mode 1: the network; mode 2: the exact ratios through the same path.
-void launch_infer(int ndim, int ndir, int axis, const GridDesc& g, const double* w,
-                  const double* bg, double gamma, float sensor, const uint16_t* P16,
-                  const float* P32, float* RF, int mode, hipStream_t st);
+// Inference for every axis K on state w: face ratios for the 2*ndim+1
+// variables of setnu on that axis (order rho', thermal energy, v_0.., b_l (l
+// != K)) in RF[K], stored at the face's left cell, or -1 where the exact ratio
+// is to be used.  mode 1: the network; mode 2: the exact ratios through the
+// same path.
+void launch_infer(int ndim, int ndir, const GridDesc& g, const double* w, const double* bg,
+                  double gamma, float sensor, const uint16_t* P16, const float* P32,
+                  float* const* RF, int mode, hipStream_t st);
 
 }  // namespace closure
 }  // namespace sac

@@ -265,12 +265,12 @@ __device__ __forceinline__ int var_of_slot(int o) {
 // same storage (a check of the plumbing: the run then follows the exact one
 // to FP32 rounding of the ratio)
 template <int NDIM, int NDIR, int K>
-__global__ void __launch_bounds__(256) k_infer(GridDesc g, const double* w, const double* bg,
-                                               double gamma, float thr, const uint16_t* P16,
-                                               const float* P32, float* RF, int mode) {
+__device__ __forceinline__ void infer_axis(const GridDesc& g, const double* w, const double* bg,
+                                           double gamma, float thr, const uint16_t* P16,
+                                           const float* P32, float* RF, int mode,
+                                           uint16_t (&xs)[4][mlp::WAVE * mlp::IN]) {
   using namespace mlp;
   constexpr int NP = 2 * NDIM + 1;
-  __shared__ __attribute__((aligned(16))) uint16_t xs[4][WAVE * IN];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // faces c+1/2 for c = Mlo-1 .. Mhi along K, mesh along the other axes
   int lo[3], ext[3];
@@ -303,8 +303,9 @@ __global__ void __launch_bounds__(256) k_infer(GridDesc g, const double* w, cons
 #pragma unroll
   for (int k = 0; k < IN; k++) xs[wv][lane * IN + k] = use ? f2bf(x[k]) : (uint16_t)0;
   __syncthreads();
-  f32x4 out[WAVE / 16];
-  forward_regs(P16, P32, xs[wv], out, lane);
+  f32x4 out[WAVE / 16] = {};
+  // flat and shocked regions have whole waves of exact faces
+  if (__ballot(use)) forward_regs(P16, P32, xs[wv], out, lane);
   // lane (r, q) holds outputs 4q..4q+3 of samples 16nb + r: each writes those
   // of its samples, with the sample's cell index and flags from its lane
   const int r = lane & 15, q = lane >> 4;
@@ -321,6 +322,29 @@ __global__ void __launch_bounds__(256) k_infer(GridDesc g, const double* w, cons
         RF[(long long)p * g.fs + ics] = uses ? fminf(fmaxf(6.f * out[nb][i], 0.f), 6.f) : -1.f;
     }
   }
+}
+
+// The axes of a stage in one launch (blockIdx.y = axis): one axis of a small
+// grid is half a round of blocks (136 registers: three blocks on a CU).  At
+// 64x48x48 the axes took 28 us each in three launches, 60 us in one, and
+// 24 us in one with the network left out by waves all of whose faces keep
+// the exact ratio; then the features' loads and divisions bound it.
+struct RatioFields {
+  float* f[3];
+};
+template <int NDIM, int NDIR>
+__global__ void __launch_bounds__(256) k_infer(GridDesc g, const double* w, const double* bg,
+                                               double gamma, float thr, const uint16_t* P16,
+                                               const float* P32, RatioFields RF, int mode) {
+  __shared__ __attribute__((aligned(16))) uint16_t xs[4][mlp::WAVE * mlp::IN];
+  if (blockIdx.y == 0)
+    infer_axis<NDIM, NDIR, 0>(g, w, bg, gamma, thr, P16, P32, RF.f[0], mode, xs);
+  if constexpr (NDIM > 1)
+    if (blockIdx.y == 1)
+      infer_axis<NDIM, NDIR, 1>(g, w, bg, gamma, thr, P16, P32, RF.f[1], mode, xs);
+  if constexpr (NDIM > 2)
+    if (blockIdx.y == 2)
+      infer_axis<NDIM, NDIR, 2>(g, w, bg, gamma, thr, P16, P32, RF.f[2], mode, xs);
 }
 
 // ---------------------------------------------------------------------
@@ -372,34 +396,28 @@ void launch_to_bf16(const float* P32, uint16_t* P16, hipStream_t st) {
 }
 
 template <int NDIM, int NDIR>
-static void infer_nd(int axis, const GridDesc& g, const double* w, const double* bg, double gamma,
-                     float thr, const uint16_t* P16, const float* P32, float* RF, int mode,
+static void infer_nd(const GridDesc& g, const double* w, const double* bg, double gamma, float thr,
+                     const uint16_t* P16, const float* P32, float* const* RF, int mode,
                      hipStream_t st) {
-  long long n = 1;
-  for (int d = 0; d < 3; d++) n *= g.Mhi[d] - g.Mlo[d] + 1 + (d == axis ? 1 : 0);
-  const dim3 grid((unsigned)((n + 255) / 256)), blk(256);
-  if (axis == 0)
-    hipLaunchKernelGGL((k_infer<NDIM, NDIR, 0>), grid, blk, 0, st, g, w, bg, gamma, thr, P16, P32,
-                       RF, mode);
-  if constexpr (NDIM > 1)
-    if (axis == 1)
-      hipLaunchKernelGGL((k_infer<NDIM, NDIR, 1>), grid, blk, 0, st, g, w, bg, gamma, thr, P16,
-                         P32, RF, mode);
-  if constexpr (NDIM > 2)
-    if (axis == 2)
-      hipLaunchKernelGGL((k_infer<NDIM, NDIR, 2>), grid, blk, 0, st, g, w, bg, gamma, thr, P16,
-                         P32, RF, mode);
+  long long n = 0;  // faces of the axis that has most
+  for (int k = 0; k < NDIM; k++) {
+    long long m = 1;
+    for (int d = 0; d < 3; d++) m *= g.Mhi[d] - g.Mlo[d] + 1 + (d == k ? 1 : 0);
+    n = m > n ? m : n;
+  }
+  hipLaunchKernelGGL((k_infer<NDIM, NDIR>), dim3((unsigned)((n + 255) / 256), NDIM), dim3(256), 0,
+                     st, g, w, bg, gamma, thr, P16, P32, RatioFields{{RF[0], RF[1], RF[2]}}, mode);
 }
 
-void launch_infer(int ndim, int ndir, int axis, const GridDesc& g, const double* w,
-                  const double* bg, double gamma, float sensor, const uint16_t* P16,
-                  const float* P32, float* RF, int mode, hipStream_t st) {
-  if (ndim == 1 && ndir == 1) infer_nd<1, 1>(axis, g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
-  else if (ndim == 1 && ndir == 2) infer_nd<1, 2>(axis, g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
-  else if (ndim == 1 && ndir == 3) infer_nd<1, 3>(axis, g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
-  else if (ndim == 2 && ndir == 2) infer_nd<2, 2>(axis, g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
-  else if (ndim == 2 && ndir == 3) infer_nd<2, 3>(axis, g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
-  else if (ndim == 3 && ndir == 3) infer_nd<3, 3>(axis, g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
+void launch_infer(int ndim, int ndir, const GridDesc& g, const double* w, const double* bg,
+                  double gamma, float sensor, const uint16_t* P16, const float* P32,
+                  float* const* RF, int mode, hipStream_t st) {
+  if (ndim == 1 && ndir == 1) infer_nd<1, 1>(g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
+  else if (ndim == 1 && ndir == 2) infer_nd<1, 2>(g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
+  else if (ndim == 1 && ndir == 3) infer_nd<1, 3>(g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
+  else if (ndim == 2 && ndir == 2) infer_nd<2, 2>(g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
+  else if (ndim == 2 && ndir == 3) infer_nd<2, 3>(g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
+  else if (ndim == 3 && ndir == 3) infer_nd<3, 3>(g, w, bg, gamma, sensor, P16, P32, RF, mode, st);
 }
 
 }  // namespace closure
