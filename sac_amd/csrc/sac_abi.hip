@@ -350,7 +350,8 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
     x.divbfix = d.divbfix;
     hipEvent_t e0{};
     t_begin(d, SAC_K_AXIS, &e0);
-    skip_last = sac::launch_axis(x, k, d.stream);
+    if (!(stage3 && sac::launch_columns(x, d.stream)))
+      skip_last = sac::launch_axis(x, k, d.stream);
     t_end(d, SAC_K_AXIS, e0, 5 + k);
   }
   if (d.eta > 0.0) {  // resistive sources into R (addsource, src/vacphys.mhd0.t:240-249)

@@ -114,6 +114,9 @@ void launch_resistive(const ResistArgs& a, hipStream_t st);
 // returns 1 if the cross-term derivatives along `axis` were added (requested
 // by a.cross_last and done by the line-tile kernel), else 0
 int launch_axis(const AxisArgs& a, int axis, hipStream_t st);
+// the z work of a 3-D stage with viscosity by columns, R written (a.fresh);
+// 0 if the grid has too few of them (nothing is launched: use launch_axis)
+int launch_columns(const AxisArgs& a, hipStream_t st);
 // 1 if the line-tile kernels (which carry the Powell sources) are built
 int line_tiles_built();
 // 3-D grids: the cross-term factors T_{0,2} and T_{1,2} (sac_tile.h)

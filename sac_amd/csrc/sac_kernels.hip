@@ -24,6 +24,7 @@
 //   gradient1/1L/1R    src/vacusr.viscosity.t:547-675
 //   getboundary        src/vacgrid.t:195-512
 #include "sac_device.h"
+#include "sac_column.h"
 #include "sac_line.h"
 #include "sac_tile.h"
 
@@ -82,6 +83,16 @@ __global__ void __launch_bounds__((line::Tile<K, C>::T)) k_line(AxisArgs a, int 
     double r2[1] = {(double)numax};
     block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
   }
+}
+
+// z work of 3-D grids with enough columns (see march and launch_columns)
+template <typename S, typename C, bool DIVB>
+__global__ void __launch_bounds__(column::NT, 2) k_column(AxisArgs a, int seg) {
+  __shared__ C L[column::Lay<C, DIVB>::END];
+  C numax = 0;
+  column::march<S, C, DIVB>(a, seg, L, numax);
+  double r2[1] = {(double)numax};
+  block_max_atomic<1>(r2, red_line(a.acc) + kRedVisc);
 }
 
 // kernel 1, 1-D grids in FP64 whose rate gets further terms before the
@@ -585,6 +596,33 @@ int launch_axis(const AxisArgs& a, int axis, hipStream_t st) {
   dispatch(a.prec, g.ndim, g.ndir, 0, axis, &a, st, n);
   const bool line = SAC_LINE_TILES && g.ndim > 1;
   return (line && a.cross_last && a.visc_on && axis == g.ndim - 1) ? 1 : 0;
+}
+
+// A CU holds two blocks: as many segments as fill the chip once, of 16 to
+// column::SEG cells (a segment loads and evaluates six points more than it has
+// cells).  By columns where that makes enough blocks, by line tiles (which
+// work on 16 points of a line at once) below: FP64 us 46 against 40 at 80^3
+// (125 blocks), 57 against 68 at 96^3 (216), 61 against 83 at 128 x 128 x 64
+// (256); FP32 storage 43 against 41 at 96^3, 44 against 49 at 128 x 128 x 64.
+int launch_columns(const AxisArgs& a, hipStream_t st) {
+  const GridDesc& g = a.g;
+  if (!a.visc_on || g.st[2] >= (1LL << 29)) return 0;  // 32-bit byte offsets in a plane
+  const long long nb = (column::ncolumns(g) + column::NT - 1) / column::NT;
+  const int ext = g.Mhi[2] - g.Mlo[2] + 1, few = (int)(512 / nb);
+  int seg = few > 1 ? (ext + few - 1) / few : ext;
+  if (seg < 16) seg = 16;
+  if (seg > column::SEG) seg = column::SEG;
+  const int nseg = (ext + seg - 1) / seg;
+  if (nb * nseg < (a.prec == PREC_MIXED ? 256 : 192) || nseg > 65535) return 0;
+  const dim3 grid((unsigned)nb, (unsigned)nseg), bs(column::NT);
+  if (a.prec == PREC_MIXED) {
+    if (a.divbfix) hipLaunchKernelGGL((k_column<float, float, true>), grid, bs, 0, st, a, seg);
+    else hipLaunchKernelGGL((k_column<float, float, false>), grid, bs, 0, st, a, seg);
+  } else {
+    if (a.divbfix) hipLaunchKernelGGL((k_column<double, double, true>), grid, bs, 0, st, a, seg);
+    else hipLaunchKernelGGL((k_column<double, double, false>), grid, bs, 0, st, a, seg);
+  }
+  return 1;
 }
 
 // Tile length of k_stage1: 64 cells while that gives at most two blocks per
