@@ -11,8 +11,8 @@ resident in HBM when the timed region starts.
 
 Metric: Mcell-updates/s per RK stage = N_mesh * steps * 4 / wall time.
 Roofline: the unit is one RK stage, which the library issues as a fixed
-kernel sequence (k_plane for the x and y work, k_line for z, k_final,
-k_ghost); algorithmic bytes =
+kernel sequence (k_tz for the cross-term factors that z takes, k_column for
+the z work, k_stage for the x and y work and the update, k_ghost); algorithmic bytes =
 296 B per mesh cell per stage (4*n_evolve*8 + n_background*8 for 8 evolving
 and 5 background FP64 fields) x N_mesh, divided by the summed average
 durations of that sequence, measured with HIP events on the library's
@@ -169,7 +169,7 @@ def main():
     ncell = n ** 3
     stages = args.steps * 4
     value = ncell * stages / el / 1e6
-    # kernel time of one stage: k_plane (x and y) + k_line (z) + k_final + k_ghost
+    # kernel time of one stage: k_tz + k_column (z) + k_stage (x, y, update) + k_ghost
     per_stage_ms = (p_ms + a_ms + f_ms + g_ms) / max(f_n, 1)
     alg_bytes = BYTES_PER_CELL_STAGE["fp64"] * ncell
     achieved = alg_bytes / (per_stage_ms / 1e3) / 1e9
@@ -194,17 +194,17 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
-                     "kernel": "RK stage = k_plane (x and y) + k_line<3,3,2> (z) + k_final<3,3> "
-                               "+ k_ghost",
+                     "kernel": "RK stage = k_tz (factors for z) + k_column (z) + k_stage<3,3> "
+                               "(x, y, update) + k_ghost",
                      "avg_ms": round(per_stage_ms, 4),
                      "launches": f_n,
                      # the measured HBM traffic (rocprof, copy-calibrated) over the
                      # same time: how close the kernels run to the memory system
                      "traffic_rate_GBs": (round(traffic / 1e9 / (per_stage_ms / 1e3), 1)
                                           if traffic else None)},
-        "stage_breakdown_ms": {"k_plane": round(p_ms / max(p_n, 1), 4),
-                               "k_line_z": round(tim["K_AXIS3"][0] / max(tim["K_AXIS3"][1], 1), 4),
-                               "k_final": round(f_ms / max(f_n, 1), 4),
+        "stage_breakdown_ms": {"k_tz": round(p_ms / max(p_n, 1), 4),
+                               "k_column_z": round(tim["K_AXIS3"][0] / max(tim["K_AXIS3"][1], 1), 4),
+                               "k_stage": round(f_ms / max(f_n, 1), 4),
                                "k_ghost": round(g_ms / max(g_n, 1), 4),
                                "stage_wall": round(stage_wall_s * 1e3, 4)},
         "stage_roofline_frac": round(alg_bytes / stage_wall_s / 1e9 / HBM_PEAK_GBS, 4),

@@ -65,16 +65,16 @@ extern "C" {
 #define SAC_SLOT_S3 3 /* RK4's third stage register */
 
 /* kernels reported by sac_dev_timing_get */
-#define SAC_K_FINAL 0 /* cross terms, gravity, register update, cmax reductions */
-#define SAC_K_AXIS 1  /* per-axis fluxes, setnu and hyperdiffusion (ndim launches) */
+#define SAC_K_FINAL 0 /* the launch that updates: cross terms, gravity, register update, cmax (1-D FP64 and tiled grids: the x and y work too) */
+#define SAC_K_AXIS 1  /* fluxes, setnu and hyperdiffusion by axis (tiled 3-D grids: z only) */
 #define SAC_K_GHOST 2
 #define SAC_K_CMAX 3
 #define SAC_K_COPY 4
 #define SAC_K_AXIS1 5 /* k_axis launches of axis 1, 2, 3 separately */
 #define SAC_K_AXIS2 6
 #define SAC_K_AXIS3 7
-#define SAC_K_CLOSURE 8 /* learned-closure inference launches (one per axis) */
-#define SAC_K_PLANE 9   /* 3-D grids: the x and y work of z-plane tiles (one launch per stage) */
+#define SAC_K_CLOSURE 8 /* learned-closure inference (one launch per stage) */
+#define SAC_K_PLANE 9   /* tiled 3-D grids: the cross-term factors for z (one launch per stage) */
 
 typedef void *sac_handle;
 
@@ -173,14 +173,15 @@ int sac_dev_getdt_special(sac_handle h, double *dt);
  * one full Runge-Kutta step of the state including every getboundary. */
 int sac_dev_advance(sac_handle h, double dt);
 
-/* Kernel schedule of the stages of 3-D grids: with on=1 (the default) the x
- * and y work of a stage runs in one pass over 2-D tiles of each z-plane
- * (the x-y cross terms included), then the z line tiles; with on=0 one
- * line-tile pass per axis.  Both evaluate the same terms of centdiff4,
- * setnu and addsource_visc (src/vaccd.t:7-78, src/vacusr.viscosity.t:2-455)
- * and agree to rounding (the cross terms are summed in another order).  The
- * learned closure and Powell's sources use the per-axis passes.  No
- * counterpart in the reference (a schedule choice of this library). */
+/* Kernel schedule of the stages of 2-D and 3-D grids: with on=1 (the
+ * default) the x and y work of a stage and its update run in one launch over
+ * 2-D tiles, in 3-D after one for the cross-term factors that z takes and one
+ * for the z work; with on=0 one line-tile pass per axis and an update.  Both
+ * evaluate the same terms of centdiff4, setnu and addsource_visc
+ * (src/vaccd.t:7-78, src/vacusr.viscosity.t:2-455) and agree to rounding (the
+ * terms are summed in another order).  The learned closure uses the per-axis
+ * passes.  No counterpart in the reference (a schedule choice of this
+ * library). */
 int sac_dev_set_plane_tiles(sac_handle h, int on);
 
 /* divbfix: Powell's div B source terms (addsource_divb,

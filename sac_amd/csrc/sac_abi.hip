@@ -125,7 +125,7 @@ struct Dev {
   std::vector<TimedLaunch> timed;
   double t_ms[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   long long t_n[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  // 3-D stages: the x and y work in one pass over z-plane tiles (k_plane)
+  // 2-D and 3-D stages on tiles (k_stage)
   // instead of one line-tile pass per axis
   int plane = 1;
   int xcd = 8;  // XCDs of the device (block renumbering of the line kernels)

@@ -381,7 +381,7 @@ __device__ __forceinline__ void face_pair(const C* q, C& ratL, C& ratR) {
 }
 
 // Hyperdiffusion along an axis (setnu, addsource_visc) of one cell, shared by
-// the line and plane tiles.  For one variable, nu dq at the cell's two faces
+// the line tiles, stage tiles and columns.  For one variable, nu dq at the cell's two faces
 // from its q window; with nu = c_tot c_hyp dx ratio:
 //   t = nu dq,  terms = (a_R t_R - a_L t_L) / dx^2 with the face means a
 // (the factors 1/2 of the means and of the momentum terms are taken into the

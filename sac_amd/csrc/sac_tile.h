@@ -577,13 +577,13 @@ __device__ __forceinline__ bool stage_tile(const FinalArgs& f, const GridDesc& g
 
 // ---------------------------------------------------------------------
 // 3-D: the factors T_{0,2} and T_{1,2} of a tile's cells, made along x and y
-// from v_2 and b_2, which the z line tiles differentiate along z.  Making
+// from v_2 and b_2, which the z work differentiates along z.  Making
 // them in a pass of its own (4 fields read, 4 written) lets the z pass come
 // before the x and y work, whose kernel can then finish the cell: the rate of
 // x and y stays in registers and there is no combining pass.  A stage at
 // 256^3 in FP64: plane tiles 1.84 ms, z lines 1.29, update 1.10 (1.68 RK4's
-// last); now factors 0.27, z lines 0.97, this file's tiles 2.07 (2.37).  At
-// 128^3: 0.266 + 0.177 + 0.158 (0.222), now 0.041 + 0.146 + 0.270 (0.319).
+// last); now factors 0.27, z columns 0.83, this file's tiles 2.07 (2.37).  At
+// 128^3: 0.266 + 0.177 + 0.158 (0.222), now 0.041 + 0.113 + 0.270 (0.319).
 template <typename C>
 struct TzSmem {
   C v[2][PY][PX];  // v_2, b_2

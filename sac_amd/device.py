@@ -228,8 +228,8 @@ class Device:
         _check(load_library().sac_dev_set_resistive(self._h, 1 if compactres else 0, dtdiffpar))
 
     def set_plane_tiles(self, on=True):
-        """3-D stages: x and y work in one pass over z-plane tiles (default)
-        or one line-tile pass per axis."""
+        """2-D and 3-D stages: x and y work and update in one launch over 2-D
+        tiles (default) or one line-tile pass per axis."""
         _check(load_library().sac_dev_set_plane_tiles(self._h, 1 if on else 0))
 
     def set_divbfix(self, on=True):
