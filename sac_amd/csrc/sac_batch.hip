@@ -219,8 +219,9 @@ __global__ void __launch_bounds__(tile::NT, 4) kb_patch_stage(Args a, int wct, i
 // as an LDS line tile (line1_tile, sac_device.h, also used by 1-D FP64
 // grids), then the update of the thread's cell from the rate in its
 // registers, with the 'cont' ghosts.  With R stored and read back a
-// stage of 4.5 M cells took 0.383 ms (0.478 ms RK4's last), now 0.314 (0.388);
-// 232 B per cell without R, 3.3 TB/s: latency of two waits per block.
+// stage of 4.5 M cells took 0.383 ms (0.478 ms RK4's last) in tiles of 256,
+// then 0.312 (0.380), and 0.283 (0.363) in tiles of 128: 232 B per cell without
+// R, 3.7 TB/s; latency of two waits per block.
 template <int LT, bool RK4L>
 __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, int out, double da) {
   __shared__ double L[line1::LV<NDIR> * (LT + 6)];
@@ -433,6 +434,10 @@ int bfail(int code, const char* fmt, ...) {
 struct Shape {
   int ck, tb, tbx;
 };
+// Tubes start with 128: of tubes of 200 to 2000 cells the last tile leaves 5 %
+// of the threads idle instead of 10 (stage 0.283 ms against 0.312; 64 cells
+// 0.281 but 0.366 against 0.363 in RK4's last); on one tube of 10^6 cells, where
+// no tile is idle, the two lengths differ by 1 % (61.0 and 60.2 us).
 const Shape kShapes1[] = {{1, 64, 0}, {1, 128, 0}, {1, 256, 0}};
 const Shape kShapes2[] = {{1, 64, 16},  {1, 64, 32},  {1, 64, 64},   {1, 128, 16},
                           {1, 128, 32}, {1, 128, 64}, {1, 128, 128}, {1, 256, 16},
@@ -840,7 +845,7 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   a.dtmin = 1.0e-99;
   a.itmax = itmax;
   a.running = b->d_running;
-  if ((rc = set_shape(*b, ndim == 1 ? Shape{1, 256, 0} : Shape{1, 256, 64}))) return bail(rc);
+  if ((rc = set_shape(*b, ndim == 1 ? Shape{1, 128, 0} : Shape{1, 256, 64}))) return bail(rc);
   // initial getboundary (background and state) and cmax of W
   enqueue_ghost(*b, b->d_bg, NBG);
   enqueue_ghost(*b, b->d_reg[SAC_SLOT_W], NE);
