@@ -295,8 +295,9 @@ int sac_batch_free(sac_batch_handle h);
 /* Autotuner: times trial_steps steps for every launch shape from the
  * current state, restores the state, keeps the fastest shape.  Tubes: LDS
  * line tiles of tb in {64,128,256} cells, one per thread (ck = 1).
- * Patches: one cell per thread, tiles of tbx x tb/tbx cells for tb in
- * {64,128,256} and tbx in {16,...,tb} (12 shapes). */
+ * Patches: a stage has one tile (16 x 16 cells), so one shape is timed; the
+ * shapes, tiles of tbx x tb/tbx cells for tb in {64,128,256} and tbx in
+ * {16,...,tb} (12 of them), are those of the first cmax sweep. */
 int sac_batch_tune(sac_batch_handle h, int trial_steps, int *ck, int *tb, double *ms_per_step);
 /* Use launch shape `index` of the autotuner's list (tubes 0..2, patches
  * 0..11) without timing. */
