@@ -358,7 +358,7 @@ __device__ __forceinline__ void march(const AxisArgs& a, int seg, C* __restrict_
         q0(v) = q[v][0];
         __builtin_amdgcn_sched_barrier(0);
       }
-      numax = fmax(numax, c < cs ? (C)0 : nmax);
+      numax = fmax(numax, c < cs ? (C)0 : ha.nu(nmax));
 #pragma unroll
       for (int n = 0; n < NE; n++) put(a.R, n, cd, R[n]);
     }

@@ -386,28 +386,37 @@ __device__ __forceinline__ void face_pair(const C* q, C& ratL, C& ratR) {
 //   t = nu dq,  terms = (a_R t_R - a_L t_L) / dx^2 with the face means a
 // (the factors 1/2 of the means and of the momentum terms are taken into the
 // power-of-two multiples of 1/dx^2, so nothing is rounded by them).
+// In FP32 the same with t = nu dq / dx and one 1/dx: 1/dx^2 leaves FP32's
+// range at widths above 1e19 and below 1e-19 (lengths of a galaxy in
+// centimetres), and the dx of nu cancels, so this takes no operation more.
 template <typename C>
 struct HyperAxis {
-  C kv, ks;      // c_tot c_hyp dx of the velocities (c_hyp 0.4) and the others (0.04)
-  C i2, i2h, i2q;  // 1/dx^2 and its half and quarter
-  C it;          // 1/dx / 8
+  static constexpr bool F32 = sizeof(C) == 4;
+  C kv, ks;      // c_tot c_hyp (dx) of the velocities (c_hyp 0.4) and the others (0.04)
+  C i2, i2h, i2q;  // 1/dx^2 (1/dx) and its half and quarter
+  C it;          // 1/dx / 8 (1/8)
+  C w;           // what the largest k ratio takes to be nu: 1 (dx)
   __device__ __forceinline__ HyperAxis(C ctk, C dxk, C idx) {
-    kv = ctk * (C)0.4 * dxk;
-    ks = ctk * (C)0.04 * dxk;
-    i2 = idx * idx;
+    kv = F32 ? ctk * (C)0.4 : ctk * (C)0.4 * dxk;
+    ks = F32 ? ctk * (C)0.04 : ctk * (C)0.04 * dxk;
+    i2 = F32 ? idx : idx * idx;
     i2h = (C)0.5 * i2;
     i2q = (C)0.25 * i2;
-    it = (C)0.125 * idx;
+    it = F32 ? (C)0.125 : (C)0.125 * idx;
+    w = dxk;
   }
+  // the largest nu, from the largest k ratio
+  __device__ __forceinline__ C nu(C kmax) const { return F32 ? kmax * w : kmax; }
 };
 // the two faces' t (zero: gradients replaced by zero, at a mesh end); returns
-// (q_+ - q_-) (nu_L + nu_R), the cross factor's product, and adds to numax
+// (q_+ - q_-) (nu_L + nu_R), or that over dx in FP32, the cross factor's
+// product, and adds to kmax (see HyperAxis::nu)
 template <typename C>
 __device__ __forceinline__ C hyper_faces(const C* q, C k, C ratL, C ratR, bool zero, C& tL, C& tR,
-                                         C& numax) {
+                                         C& kmax) {
 #pragma clang fp contract(off)
   const C nuL = k * ratL, nuR = k * ratR;
-  numax = fmax(numax, fmax(nuR, nuL));
+  kmax = fmax(kmax, fmax(nuR, nuL));
   tL = zero ? (C)0 : nuL * (q[3] - q[2]);
   tR = zero ? (C)0 : nuR * (q[4] - q[3]);
   return zero ? (C)0 : (q[4] - q[2]) * (nuL + nuR);

@@ -426,7 +426,7 @@ __device__ __forceinline__ void line_tile(const AxisArgs& a, int seg, C* __restr
               Tout[(long long)(cross_index(NDIM, K, lb) + 1) * fs + icell] = (S)((C)2 * T * ha.it);
           }
         }
-        numax = valid ? fmax(numax, nmax) : numax;
+        numax = valid ? fmax(numax, ha.nu(nmax)) : numax;
       }
       if (valid) {
         if (K == 0) {

@@ -224,7 +224,7 @@ __device__ __forceinline__ void cell_axis(const FinalArgs& f, const GridDesc& g,
         if (lb == 1 - K) Tb = (C)2 * T * ha.it;
       }
     }
-    numax = valid ? nmax : (C)0;
+    numax = valid ? ha.nu(nmax) : (C)0;
   }
 }
 
