@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -138,7 +139,9 @@ struct Dev {
   hipStream_t save_stream = nullptr;
   hipEvent_t save_taken = nullptr, save_done = nullptr;
   bool save_pending = false;
-  std::vector<double> bg_host;   // background of the last upload (static)
+  // the background on the host, copied by the first save after an upload or a
+  // fill changed it (null: not copied), and that of the pending save
+  std::shared_ptr<const std::vector<double>> bg_host, save_bg;
 };
 
 long long fieldsz(const Dev& d) { return d.g.fs; }
@@ -714,7 +717,7 @@ int sac_dev_upload(sac_handle h, const double* w) {
   Dev& d = *(Dev*)h;
   if (int rc = copy_state(d, SAC_SLOT_W, true, const_cast<double*>(w), false)) return rc;
   d.red_valid[SAC_SLOT_W] = false;
-  d.bg_host.clear();  // the ghosts of the background change at the next getboundary
+  d.bg_host.reset();  // the ghosts of the background change at the next getboundary
   d.bg_ghosts_stale = d.initialized;
   return 0;
 }
@@ -759,9 +762,10 @@ int sac_dev_save_begin(sac_handle h) {
     if (int rc = balloc(d, &d.save_dev, bytes)) return rc;
     HIPCHK(hipHostMalloc(&d.save_host, bytes, hipHostMallocDefault));
   }
-  if (d.bg_host.empty()) {  // the background is static: one synchronous copy
-    d.bg_host.resize((size_t)d.nbg * (size_t)d.ncell_grid);
-    if (int rc = copy_bg_out(d, d.bg_host.data())) return rc;
+  if (!d.bg_host) {  // the background is static: one synchronous copy
+    auto bg = std::make_shared<std::vector<double>>((size_t)d.nbg * (size_t)d.ncell_grid);
+    if (int rc = copy_bg_out(d, bg->data())) return rc;
+    d.bg_host = bg;
   }
   // the snapshot in the host's layout, so that one plain copy takes it over
   const sac::xfer::Fields f = {d.reg[SAC_SLOT_W], (int)d.esz, d.ne, nullptr};
@@ -771,6 +775,7 @@ int sac_dev_save_begin(sac_handle h) {
   HIPCHK(hipStreamWaitEvent(d.save_stream, d.save_taken, 0));
   HIPCHK(hipMemcpyAsync(d.save_host, d.save_dev, bytes, hipMemcpyDeviceToHost, d.save_stream));
   HIPCHK(hipEventRecord(d.save_done, d.save_stream));
+  d.save_bg = d.bg_host;
   d.save_pending = true;
   return 0;
 }
@@ -793,13 +798,14 @@ int sac_dev_save_end(sac_handle h, double* w) {
   Dev& d = *(Dev*)h;
   if (!d.save_pending) return fail(SAC_E_ARG, "no save in progress");
   d.save_pending = false;
+  const auto bg = std::move(d.save_bg);
   HIPCHK(hipEventSynchronize(d.save_done));
   const size_t n = (size_t)d.ne * (size_t)d.ncell_grid;
   if (d.esz == sizeof(double))
     sac::xfer::host_copy(w, (const double*)d.save_host, n);
   else
     sac::xfer::host_copy(w, (const float*)d.save_host, n);
-  sac::xfer::host_copy(w + n, d.bg_host.data(), d.bg_host.size());
+  sac::xfer::host_copy(w + n, bg->data(), bg->size());
   return 0;
 }
 
@@ -810,7 +816,7 @@ int sac_dev_getboundary(sac_handle h) {
     ghost_fill_sequential(d, SAC_SLOT_W, !d.initialized || d.bg_ghosts_stale);
     d.initialized = true;  // no stored values in this path
     d.bg_ghosts_stale = false;
-    d.bg_host.clear();
+    d.bg_host.reset();
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(d.stream));
     return 0;
@@ -829,7 +835,7 @@ int sac_dev_getboundary(sac_handle h) {
     a.general = d.cont1_b || (d.ext1_b && !a.keep_fixed);
     sac::launch_ghost(a, d.stream);
     d.bg_ghosts_stale = false;
-    d.bg_host.clear();  // background ghosts filled: the cached copy is stale
+    d.bg_host.reset();  // background ghosts filled: the cached copy is stale
   }
   if (!d.initialized) {
     // first call: then store 'fixed' values
