@@ -769,8 +769,7 @@ int sac_dev_save_begin(sac_handle h) {
   }
   // the snapshot in the host's layout, so that one plain copy takes it over
   const sac::xfer::Fields f = {d.reg[SAC_SLOT_W], (int)d.esz, d.ne, nullptr};
-  sac::xfer::launch_pack(d.g, f, d.save_dev, d.stream);
-  HIPCHK(hipGetLastError());
+  HIPCHK(sac::xfer::launch_pack(d.g, f, d.save_dev, d.stream));
   HIPCHK(hipEventRecord(d.save_taken, d.stream));
   HIPCHK(hipStreamWaitEvent(d.save_stream, d.save_taken, 0));
   HIPCHK(hipMemcpyAsync(d.save_host, d.save_dev, bytes, hipMemcpyDeviceToHost, d.save_stream));

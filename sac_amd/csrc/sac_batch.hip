@@ -1050,9 +1050,9 @@ int sac_batch_download(sac_batch_handle h, double* w) {
       b.device, (long long)first.size() - 1, sizeof(double) * (size_t)most,
       [&](long long c, void* pin, hipEvent_t ev, std::string& e) -> int {
         const int m0 = first[c], m1 = first[c + 1];
-        hipLaunchKernelGGL(kb_pack, dim3((unsigned)(m1 - m0) * (NE + NBG)), dim3(256), 0, b.stream,
-                           b.a, b.d_hoff, m0, (double*)pin);
-        hipError_t s = hipEventRecord(ev, b.stream);
+        hipError_t s = sac::xfer::launch(kb_pack, dim3((unsigned)(m1 - m0) * (NE + NBG)), dim3(256),
+                                         b.stream, b.a, b.d_hoff, m0, (double*)pin);
+        if (s == hipSuccess) s = hipEventRecord(ev, b.stream);
         if (s == hipSuccess) s = hipEventSynchronize(ev);
         if (s != hipSuccess) {
           e = std::string("download: ") + hipGetErrorString(s);

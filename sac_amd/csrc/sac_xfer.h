@@ -2,8 +2,10 @@
 // downloads, saves): kernels that pack padded device rows to the host's
 // layout, pinned buffers, and host threads that copy.
 #pragma once
+#include <algorithm>
 #include <functional>
 #include <string>
+#include <tuple>
 
 #include "sac_common.h"
 
@@ -29,8 +31,24 @@ constexpr size_t kSmall = size_t(1) << 19;
 int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n, bool to_host,
          void** small, std::string& err);
 
+// Launch a kernel and return this launch's own error.  The last error that the
+// runtime keeps is one per thread, so that of a worker is not seen by the
+// caller, and it may be one that another call left there.
+template <typename... P, typename... A>
+hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_t st, A... a) {
+  std::tuple<P...> p(a...);
+  void* args[sizeof...(P)];
+  std::apply([&](P&... x) {
+    void* v[] = {&x...};
+    std::copy(v, v + sizeof...(P), args);
+  }, p);
+  const hipError_t e = hipLaunchKernel((const void*)kernel, grid, block, args, 0, st);
+  if (e != hipSuccess) (void)hipGetLastError();  // the caller gets it
+  return e;
+}
+
 // pack the fields of f (f.host unused) into contiguous device memory at `out`
-void launch_pack(const GridDesc& g, const Fields& f, void* out, hipStream_t stream);
+hipError_t launch_pack(const GridDesc& g, const Fields& f, void* out, hipStream_t stream);
 
 // memcpy / FP32 to FP64 by several host threads
 void host_copy(double* dst, const double* src, size_t n);

@@ -48,17 +48,16 @@ __global__ void __launch_bounds__(256) k_rows(T* dev, T* flat, unsigned n, unsig
 }
 
 template <bool OUT>
-void launch_rows(const GridDesc& g, const Fields& f, long long first, unsigned n, void* flat,
+hipError_t launch_rows(const GridDesc& g, const Fields& f, long long first, unsigned n, void* flat,
                  hipStream_t st) {
   const unsigned G0 = (unsigned)g.G[0], rows = (unsigned)g.G[1] * (unsigned)g.G[2];
   const unsigned R0 = (unsigned)(first / G0), x0 = (unsigned)(first % G0);
   const dim3 nb((n + 255) / 256), bs(256);
   if (f.esz == 8)
-    hipLaunchKernelGGL((k_rows<uint64_t, OUT>), nb, bs, 0, st, (uint64_t*)f.dev, (uint64_t*)flat, n,
-                       x0, R0, G0, rows, g.st[1], g.fs);
-  else
-    hipLaunchKernelGGL((k_rows<uint32_t, OUT>), nb, bs, 0, st, (uint32_t*)f.dev, (uint32_t*)flat, n,
-                       x0, R0, G0, rows, g.st[1], g.fs);
+    return launch(k_rows<uint64_t, OUT>, nb, bs, st, (uint64_t*)f.dev, (uint64_t*)flat, n, x0, R0,
+                  G0, rows, g.st[1], g.fs);
+  return launch(k_rows<uint32_t, OUT>, nb, bs, st, (uint32_t*)f.dev, (uint32_t*)flat, n, x0, R0, G0,
+                rows, g.st[1], g.fs);
 }
 
 // fn(begin, end) on slices of [0, n), on several threads where it pays
@@ -176,25 +175,25 @@ static int copy_small(const GridDesc& g, hipStream_t stream, const Fields* f, in
     return SAC_E_NOMEM;
   }
   size_t at = 0;
-  for (int k = 0; k < n; k++) {
+  int rc = 0;
+  for (int k = 0; k < n && !rc; k++) {
     const size_t m = ncell * f[k].nfield;
     char* p = (char*)*small + at;
-    if (to_host) {
-      launch_rows<true>(g, f[k], 0, (unsigned)m, p, stream);
-    } else {
-      to_pinned(p, f[k].host, f[k].esz, m);
-      launch_rows<false>(g, f[k], 0, (unsigned)m, p, stream);
-    }
+    if (!to_host) to_pinned(p, f[k].host, f[k].esz, m);
+    rc = hip_err(to_host ? launch_rows<true>(g, f[k], 0, (unsigned)m, p, stream)
+                         : launch_rows<false>(g, f[k], 0, (unsigned)m, p, stream),
+                 "copy kernel", err);
     at += (m * f[k].esz + 15) / 16 * 16;
   }
-  if (int rc = hip_err(hipStreamSynchronize(stream), "copy", err)) return rc;
+  const int e = hip_err(hipStreamSynchronize(stream), "copy", err);
+  if (rc || e) return rc ? rc : e;
   at = 0;
   for (int k = 0; k < n && to_host; k++) {
     const size_t m = ncell * f[k].nfield;
     from_pinned(f[k].host, (char*)*small + at, f[k].esz, m);
     at += (m * f[k].esz + 15) / 16 * 16;
   }
-  return hip_err(hipGetLastError(), "copy kernels", err);
+  return 0;
 }
 
 int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n, bool to_host,
@@ -218,7 +217,7 @@ int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int
     const unsigned m = (unsigned)std::min(per, ncell * s.nfield - lo);
     double* h = s.host + lo;
     if (to_host) {
-      launch_rows<true>(g, s, lo, m, pin, stream);
+      if (int rc = hip_err(launch_rows<true>(g, s, lo, m, pin, stream), "copy kernel", e)) return rc;
       if (int rc = hip_err(hipEventRecord(ev, stream), "hipEventRecord", e)) return rc;
       if (int rc = hip_err(hipEventSynchronize(ev), "download", e)) return rc;
       from_pinned(h, pin, s.esz, m);
@@ -227,18 +226,20 @@ int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int
     // the buffer is free once its previous chunk has been read
     if (int rc = hip_err(hipEventSynchronize(ev), "upload", e)) return rc;
     to_pinned(pin, h, s.esz, m);
-    launch_rows<false>(g, s, lo, m, pin, stream);
+    if (int rc = hip_err(launch_rows<false>(g, s, lo, m, pin, stream), "copy kernel", e)) return rc;
     return hip_err(hipEventRecord(ev, stream), "hipEventRecord", e);
   };
-  if (int rc = for_chunks(device, first[n], bytes, fn, err)) return rc;
-  return hip_err(hipGetLastError(), "copy kernels", err);
+  return for_chunks(device, first[n], bytes, fn, err);
 }
 
-void launch_pack(const GridDesc& g, const Fields& f, void* out, hipStream_t stream) {
+hipError_t launch_pack(const GridDesc& g, const Fields& f, void* out, hipStream_t stream) {
   const long long ncell = (long long)g.G[0] * g.G[1] * g.G[2], total = ncell * f.nfield;
   const long long per = 1LL << 30;  // elements of a launch (32-bit thread numbers)
-  for (long long lo = 0; lo < total; lo += per)
-    launch_rows<true>(g, f, lo, (unsigned)std::min(per, total - lo), (char*)out + lo * f.esz, stream);
+  hipError_t e = hipSuccess;
+  for (long long lo = 0; lo < total && e == hipSuccess; lo += per)
+    e = launch_rows<true>(g, f, lo, (unsigned)std::min(per, total - lo), (char*)out + lo * f.esz,
+                          stream);
+  return e;
 }
 
 }  // namespace xfer

@@ -9,6 +9,7 @@
 #include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 
 typedef int hipError_t;
 typedef struct { uint32_t x, y, z; } dim3;
@@ -172,6 +173,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t sh
     pthread_mutex_unlock(&lock);
   }
   if (hip_host_fail_launch && hip_host_fail_launch == (other() ? 1 : 2)) return err(LAUNCH);
+  if (hip_host_fail_launch) usleep(20000); /* the failing threads get chunks too */
   for (int k = 0; k < nkernels; k++)
     if (kernels[k].host == f) {
       const char *t = strstr(kernels[k].name, "k_rowsI");

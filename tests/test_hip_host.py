@@ -34,3 +34,59 @@ def test_save_keeps_its_background(stub, precision):
         dev.save_begin()
         np.testing.assert_array_equal(dev.save_end(), -want)
     """)
+
+
+@pytest.mark.parametrize("n", [(70, 61, 64), (300001,)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("where", [1, 2])
+def test_copy_reports_a_failed_launch(stub, n, precision, where):
+    """A copy kernel that cannot be launched fails the call, whichever thread
+    launched it (a state of several chunks)."""
+    hip_host.run(stub, f"""
+        p = state_problem({n!r})
+        dev = device.Device(p, precision={precision!r})
+        dev.upload(p.w)
+        assert knob("threads").value > 0  # chunks went over other threads
+        knob("fail_launch").value = {where}
+        for call in (lambda: dev.upload(p.w), dev.download,
+                     lambda: dev.upload_slot(1, p.w), lambda: dev.download_slot(1)):
+            try:
+                call()
+            except device.SacError as e:
+                assert "failed" in str(e), e
+            else:
+                raise AssertionError("reported as done")
+        knob("fail_launch").value = 0
+        dev.upload(p.w)
+        np.testing.assert_array_equal(dev.download()[8:], p.w[8:])
+    """)
+
+
+@pytest.mark.parametrize("n", [(800,), (300001,)])
+def test_copy_is_not_failed_by_an_earlier_error(stub, n):
+    """An error that some other call of the program left behind is not a
+    copy's, and the copy leaves it where it is."""
+    hip_host.run(stub, f"""
+        p = state_problem({n!r})
+        dev = device.Device(p)
+        for call in (lambda: dev.upload(p.w), dev.download, lambda: dev.upload_slot(1, p.w)):
+            assert hip.hipMemcpy(None, None, 0, 0) == 1
+            call()
+            assert hip.hipGetLastError() == 1
+    """)
+
+
+@pytest.mark.parametrize("where", [1, 2])
+def test_ensemble_download_reports_a_failed_launch(stub, where):
+    hip_host.run(stub, f"""
+        ens = batch.Ensemble([state_problem((n,)) for n in (20000, 30000, 40000, 50000, 9000)] * 3)
+        ens.download()
+        assert knob("threads").value > 0
+        knob("fail_launch").value = {where}
+        try:
+            ens.download()
+        except device.SacError as e:
+            assert "failed" in str(e), e
+        else:
+            raise AssertionError("reported as done")
+    """)
