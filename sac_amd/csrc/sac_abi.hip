@@ -148,11 +148,17 @@ long long fieldsz(const Dev& d) { return d.g.fs; }
 
 int balloc(Dev& d, void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess) return fail(SAC_E_NOMEM, "hipMalloc of %zu bytes failed: %s", bytes,
-                                   hipGetErrorString(e));
-  d.bytes += (long long)bytes;
+  if (e != hipSuccess) {
+    *p = nullptr;
+    return fail(SAC_E_NOMEM, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+  }
   e = hipMemset(*p, 0, bytes);
-  if (e != hipSuccess) return fail(SAC_E_HIP, "hipMemset: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    hipFree(*p);
+    *p = nullptr;
+    return fail(SAC_E_HIP, "hipMemset: %s", hipGetErrorString(e));
+  }
+  d.bytes += (long long)bytes;
   return 0;
 }
 int dalloc(Dev& d, double** p, long long nelem) {
@@ -750,18 +756,24 @@ int sac_dev_download_slot(sac_handle h, int slot, double* w) {
 // host memory on the save stream after an event; sac_dev_save_end waits for
 // that copy and writes the caller's array.
 
+// What saves keep, each made if it is not there: a call that fails half way
+// leaves the rest to the next one.
+static int save_resources(Dev& d, size_t bytes) {
+  if (!d.save_stream) HIPCHK(hipStreamCreateWithFlags(&d.save_stream, hipStreamNonBlocking));
+  if (!d.save_taken) HIPCHK(hipEventCreateWithFlags(&d.save_taken, hipEventDisableTiming));
+  if (!d.save_done) HIPCHK(hipEventCreateWithFlags(&d.save_done, hipEventDisableTiming));
+  if (!d.save_dev)
+    if (int rc = balloc(d, &d.save_dev, bytes)) return rc;
+  if (!d.save_host) HIPCHK(hipHostMalloc(&d.save_host, bytes, hipHostMallocDefault));
+  return 0;
+}
+
 int sac_dev_save_begin(sac_handle h) {
   if (int rc = check_handle(h)) return rc;
   Dev& d = *(Dev*)h;
   if (d.save_pending) return fail(SAC_E_ARG, "a save is already in progress");
   const size_t bytes = d.esz * (size_t)d.ncell_grid * (size_t)d.ne;
-  if (!d.save_stream) {
-    HIPCHK(hipStreamCreateWithFlags(&d.save_stream, hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&d.save_taken, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&d.save_done, hipEventDisableTiming));
-    if (int rc = balloc(d, &d.save_dev, bytes)) return rc;
-    HIPCHK(hipHostMalloc(&d.save_host, bytes, hipHostMallocDefault));
-  }
+  if (int rc = save_resources(d, bytes)) return rc;
   if (!d.bg_host) {  // the background is static: one synchronous copy
     auto bg = std::make_shared<std::vector<double>>((size_t)d.nbg * (size_t)d.ncell_grid);
     if (int rc = copy_bg_out(d, bg->data())) return rc;

@@ -90,3 +90,39 @@ def test_ensemble_download_reports_a_failed_launch(stub, where):
         else:
             raise AssertionError("reported as done")
     """)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("what,n", [("fail_malloc", 1), ("fail_event", 1), ("fail_event", 2),
+                                    ("fail_pinned", 1)])
+def test_save_after_a_failed_allocation(stub, precision, what, n):
+    """A save that cannot get its buffers returns an error; one that can,
+    later, is a save like any other."""
+    hip_host.run(stub, f"""
+        p = state_problem((16, 9, 8))
+        want = p.w.copy()
+        if {precision!r} == "mixed":
+            want[:8] = want[:8].astype(np.float32)
+        dev = device.Device(p, precision={precision!r})
+        dev.upload(p.w)
+        dev.download()
+        before = dev.memory()
+        knob({what!r}).value = {n}
+        for _ in range({3 if what == "fail_pinned" else 1}):
+            try:
+                dev.save_begin()
+            except device.SacError:
+                pass
+            else:
+                raise AssertionError("no error")
+        knob({what!r}).value = 0
+        dev.save_begin()
+        assert dev.save_ready()
+        np.testing.assert_array_equal(dev.save_end(), want)
+        assert knob("null_stores").value == 0
+        dev.save_begin()
+        np.testing.assert_array_equal(dev.save_end(), want)
+        assert dev.memory() == before + 20 * 13 * 12 * 8 * {4 if precision == "mixed" else 8}
+        dev.close()
+        assert knob("pinned_now", ctypes.c_size_t).value == 0
+    """)
