@@ -22,7 +22,14 @@ namespace {
 
 thread_local std::string g_err;
 
+// The runtime's last error, if this is one of its errors, ends here: it has
+// been reported, and the next call would take it for its own.
+void reported(int code) {
+  if (code == SAC_E_HIP || code == SAC_E_NOMEM) (void)hipGetLastError();
+}
+
 int fail(int code, const char* fmt, ...) {
+  reported(code);
   char buf[512];
   va_list ap;
   va_start(ap, fmt);
@@ -464,6 +471,7 @@ int red_host(Dev& d, const unsigned long long* p, int at, int n, double* x) {
 namespace sac {
 // the message of sac_dev_last_error() for entry points in other files
 int set_error(int code, const char* fmt, ...) {
+  reported(code);
   char buf[512];
   va_list ap;
   va_start(ap, fmt);

@@ -411,6 +411,8 @@ using namespace sac::batch;
 thread_local std::string g_berr;
 
 int bfail(int code, const char* fmt, ...) {
+  // reported here: not the next call's
+  if (code == SAC_E_HIP || code == SAC_E_NOMEM) (void)hipGetLastError();
   char buf[512];
   va_list ap;
   va_start(ap, fmt);

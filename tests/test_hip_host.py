@@ -126,3 +126,54 @@ def test_save_after_a_failed_allocation(stub, precision, what, n):
         dev.close()
         assert knob("pinned_now", ctypes.c_size_t).value == 0
     """)
+
+
+def test_reported_errors_are_not_reported_again(stub):
+    """An allocation that failed is an error of the call that made it, not of
+    the next call of this library or of the program."""
+    hip_host.run(stub, """
+        p = state_problem((16, 9, 8))
+        knob("fail_malloc").value = 3
+        try:
+            device.Device(p)
+        except device.SacError as e:
+            assert "hipMalloc" in str(e)
+        else:
+            raise AssertionError("no error")
+        assert hip.hipGetLastError() == 0
+        dev = device.Device(p)
+        dev.upload(p.w)
+        for what in ("fail_malloc", "fail_event", "fail_pinned"):
+            knob(what).value = 1
+            try:
+                dev.save_begin()
+            except device.SacError:
+                pass
+            else:
+                raise AssertionError("no error")
+            knob(what).value = 0
+            dev.getboundary()
+            dev.synchronize()
+            dev.save_begin()
+            dev.save_end()
+            dev.close()
+            dev = device.Device(p)
+            dev.upload(p.w)
+        # a small copy without pinned memory
+        t = state_problem((50,))
+        small = device.Device(t)
+        knob("fail_pinned").value = 1
+        try:
+            small.upload(t.w)
+        except device.SacError:
+            pass
+        assert hip.hipGetLastError() == 0
+        knob("fail_pinned").value = 0
+        tubes = [state_problem((n,)) for n in (20, 30)]
+        knob("fail_malloc").value = 2
+        try:
+            batch.Ensemble(tubes)
+        except device.SacError:
+            pass
+        assert hip.hipGetLastError() == 0
+    """)
