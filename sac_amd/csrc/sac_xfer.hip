@@ -154,7 +154,11 @@ int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::st
     for (int t = 1; t < nt; t++) th.emplace_back(worker, t);
   } catch (const std::system_error&) {  // the threads there are take the chunks
   }
+  // this thread is the caller's: its current device comes back
+  int current = device;
+  const bool known = hipGetDevice(&current) == hipSuccess;
   worker(0);
+  if (known && current != device) (void)hipSetDevice(current);
   for (auto& x : th) x.join();
   for (int t = 0; t < nt; t++)
     if (rcs[t]) {

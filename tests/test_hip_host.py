@@ -177,3 +177,21 @@ def test_reported_errors_are_not_reported_again(stub):
             pass
         assert hip.hipGetLastError() == 0
     """)
+
+
+def test_copies_leave_the_current_device(stub):
+    """A thread whose current device is not the handle's keeps it through the
+    copies, as through those of one buffer."""
+    hip_host.run(stub, """
+        cur = ctypes.c_int()
+        p = state_problem((70, 61, 64))
+        dev = device.Device(p)
+        ens = batch.Ensemble([state_problem((n,)) for n in (20000, 30000, 40000, 50000)])
+        assert hip.hipSetDevice(1) == 0
+        for call in (lambda: dev.upload(p.w), dev.download, lambda: dev.upload_slot(1, p.w),
+                     lambda: dev.download_slot(1), ens.download):
+            call()
+            hip.hipGetDevice(ctypes.byref(cur))
+            assert cur.value == 1, cur.value
+        np.testing.assert_array_equal(dev.download(), p.w)
+    """)
