@@ -197,7 +197,7 @@ sac::RedCombine stage_combine(Dev& d, int out) {
   c.visc_keep = d.visc_taken ? 0 : 1;
   d.visc_taken = false;
   c.host = (out == SAC_SLOT_W) ? d.red_host : nullptr;
-  d.posted = out == SAC_SLOT_W;
+  d.posted = c.host != nullptr;
   return c;
 }
 
@@ -666,10 +666,13 @@ int sac_dev_init(int ndim, int ndir, const int* nx, int nw, const int* iws, int 
         d->ext1_b |= x1;
       }
     }
-  if (hipMalloc((void**)&d->red, kRedBytes) != hipSuccess ||
-      hipHostMalloc((void**)&d->red_host, sizeof(unsigned long long) * sac::kRedSlots,
-                    hipHostMallocDefault) != hipSuccess)
+  if (hipMalloc((void**)&d->red, kRedBytes) != hipSuccess)
     return bail(fail(SAC_E_NOMEM, "reduction buffer"));
+  if (hipHostMalloc((void**)&d->red_host, sizeof(unsigned long long) * sac::kRedSlots,
+                    hipHostMallocDefault) != hipSuccess) {
+    d->red_host = nullptr;  // no pinned memory: nothing is posted
+    (void)hipGetLastError();
+  }
   hipMemset(d->red, 0, kRedBytes);
   // getdt_grav (src/vacusr.gravity.t:114-121): computed once, at it==itmin
   d->dtgrav = kBigDouble;

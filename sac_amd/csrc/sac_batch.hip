@@ -1064,7 +1064,21 @@ int sac_batch_download(sac_batch_handle h, double* w) {
         return 0;
       },
       err);
-  return rc ? bfail(rc, "%s", err.c_str()) : 0;
+  if (rc != sac::xfer::kNoPinned) return rc ? bfail(rc, "%s", err.c_str()) : 0;
+  // no pinned memory: field by field through ordinary memory
+  BCHK(hipStreamSynchronize(b.stream));
+  std::vector<double> f((size_t)b.fs);
+  for (int v = 0; v < NE + NBG; v++) {
+    const double* src = v < NE ? b.d_reg[SAC_SLOT_W] + v * b.fs : b.d_bg + (v - NE) * b.fs;
+    BCHK(hipMemcpy(f.data(), src, sizeof(double) * f.size(), hipMemcpyDeviceToHost));
+    for (int i = 0; i < b.ntubes; i++) {
+      const int G0 = b.gx(i), G1 = b.gy(i);
+      for (int r = 0; r < G1; r++)
+        memcpy(w + b.hoff[i] + ((size_t)v * G1 + r) * G0,
+               &f[(size_t)b.start[i] + (size_t)r * b.pitch[i]], sizeof(double) * G0);
+    }
+  }
+  return 0;
 }
 
 int sac_batch_memory(sac_batch_handle h, long long* bytes) {

@@ -26,7 +26,8 @@ struct Fields {
 // `stream`; returns when the copy is done.  0, or a SAC_E_* code with the
 // message in err.  small: a pinned buffer of kSmall bytes for copies that fit
 // in it, of one caller at a time, or null (allocated on first use; the caller
-// frees it with hipHostFree).
+// frees it with hipHostFree).  Where there is no pinned memory the rows are
+// copied from and to ordinary memory.
 constexpr size_t kSmall = size_t(1) << 19;
 int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n, bool to_host,
          void** small, std::string& err);
@@ -57,6 +58,8 @@ void host_copy(double* dst, const float* src, size_t n);
 // Work in `n` chunks of at most `bytes` each: on up to kWorkers host threads,
 // each with a pinned buffer of its own, fn(chunk, buffer, event) for every
 // chunk; fn returns 0 or a SAC_E_* code (message in the string it is given).
+// kNoPinned, and nothing done, if no thread could get a buffer.
+constexpr int kNoPinned = -1;
 using ChunkFn = std::function<int(long long chunk, void* pinned, hipEvent_t ev, std::string& err)>;
 int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::string& err);
 

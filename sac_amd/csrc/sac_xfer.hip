@@ -129,9 +129,7 @@ int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::st
     int rc = hip_err(hipSetDevice(device), "hipSetDevice", errs[t]);
     if (!rc && hipHostMalloc(&pin, bytes, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
-      if (t > 0) return;  // the other threads take the chunks
-      errs[t] = "no pinned memory";
-      rc = SAC_E_NOMEM;
+      return;  // the other threads take the chunks
     }
     if (!rc) rc = hip_err(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate", errs[t]);
     while (!rc && !stop) {
@@ -165,6 +163,30 @@ int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::st
       err = errs[t];
       return rcs[t];
     }
+  return next ? 0 : kNoPinned;  // a thread with a buffer takes chunks until there are none
+}
+
+// Without pinned memory: field by field with the runtime's own copies of rows,
+// FP32 elements by way of a buffer
+static int copy_plain(const GridDesc& g, hipStream_t stream, const Fields* f, int n, bool to_host,
+                      std::string& err) {
+  const size_t ncell = (size_t)g.G[0] * g.G[1] * g.G[2], rows = (size_t)g.G[1] * g.G[2];
+  std::vector<float> tmp;
+  for (int k = 0; k < n; k++) {
+    const size_t esz = (size_t)f[k].esz, w = esz * g.G[0], pitch = esz * (size_t)g.st[1];
+    for (int v = 0; v < f[k].nfield; v++) {
+      double* h = f[k].host + v * ncell;
+      char* dev = (char*)f[k].dev + esz * (size_t)v * g.fs;
+      if (esz == 4) tmp.resize(ncell);
+      void* flat = esz == 4 ? (void*)tmp.data() : (void*)h;
+      if (!to_host && esz == 4) to_pinned(flat, h, 4, ncell);
+      hipError_t e = to_host ? hipMemcpy2DAsync(flat, w, dev, pitch, w, rows, hipMemcpyDeviceToHost, stream)
+                             : hipMemcpy2DAsync(dev, pitch, flat, w, w, rows, hipMemcpyHostToDevice, stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      if (int rc = hip_err(e, "copy", err)) return rc;
+      if (to_host && esz == 4) from_pinned(h, flat, 4, ncell);
+    }
+  }
   return 0;
 }
 
@@ -175,8 +197,8 @@ static int copy_small(const GridDesc& g, hipStream_t stream, const Fields* f, in
   const size_t ncell = (size_t)g.G[0] * g.G[1] * g.G[2];
   if (!*small && hipHostMalloc(small, kSmall, hipHostMallocDefault) != hipSuccess) {
     *small = nullptr;
-    err = "no pinned memory";
-    return SAC_E_NOMEM;
+    (void)hipGetLastError();
+    return copy_plain(g, stream, f, n, to_host, err);
   }
   size_t at = 0;
   int rc = 0;
@@ -233,7 +255,8 @@ int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int
     if (int rc = hip_err(launch_rows<false>(g, s, lo, m, pin, stream), "copy kernel", e)) return rc;
     return hip_err(hipEventRecord(ev, stream), "hipEventRecord", e);
   };
-  return for_chunks(device, first[n], bytes, fn, err);
+  const int rc = for_chunks(device, first[n], bytes, fn, err);
+  return rc == kNoPinned ? copy_plain(g, stream, f, n, to_host, err) : rc;
 }
 
 hipError_t launch_pack(const GridDesc& g, const Fields& f, void* out, hipStream_t stream) {

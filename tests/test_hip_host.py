@@ -195,3 +195,41 @@ def test_copies_leave_the_current_device(stub):
             assert cur.value == 1, cur.value
         np.testing.assert_array_equal(dev.download(), p.w)
     """)
+
+
+@pytest.mark.parametrize("n", [(800,), (300001,), (61, 47), (70, 61, 64)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("where", [1, 2])
+def test_copies_without_pinned_memory(stub, n, precision, where):
+    """Pinned memory makes copies fast and is no condition for them: with none
+    at all (1), or none for the worker threads (2), states go up and down."""
+    hip_host.run(stub, f"""
+        knob("fail_pinned").value = {where}
+        p = state_problem({n!r})
+        want = p.w.copy()
+        if {precision!r} == "mixed":
+            want[:8] = want[:8].astype(np.float32)
+        dev = device.Device(p, precision={precision!r})
+        dev.upload(p.w)
+        np.testing.assert_array_equal(dev.download(), want)
+        other = state_problem({n!r}, seed=6).w
+        dev.upload_slot(1, other)
+        want[:8] = other[:8].astype(np.float32) if {precision!r} == "mixed" else other[:8]
+        np.testing.assert_array_equal(dev.download_slot(1), want)
+        dev.getboundary()
+        dev.getdt_special(1.0)
+        assert dev.maxviscoef == 0.0
+        assert hip.hipGetLastError() == 0
+    """)
+
+
+@pytest.mark.parametrize("ndim", [1, 2])
+def test_ensemble_download_without_pinned_memory(stub, ndim):
+    hip_host.run(stub, f"""
+        knob("fail_pinned").value = 1
+        probs = [state_problem((n,) if {ndim} == 1 else (n, 60 - n // 2)) for n in (6, 33, 90)]
+        ens = batch.Ensemble(probs)
+        for got, p in zip(ens.download(), probs):
+            np.testing.assert_array_equal(got, p.w)
+        assert hip.hipGetLastError() == 0
+    """)
