@@ -385,19 +385,21 @@ __global__ void kb_tick(Args a) {
 
 __global__ void kb_zero_u32(unsigned int* p) { *p = 0u; }
 
-// The state of tubes m0.. in the host's layout (per tube the NE + NBG fields,
-// unpadded, from element off[tube] of the whole) to `out`, which holds it from
-// element off[m0] on: one block per tube and field.
-__global__ void __launch_bounds__(256) kb_pack(Args a, const long long* off, int m0, double* out) {
+// Elements lo..hi-1 of the host's layout of the states (per tube the NE + NBG
+// fields, unpadded, tube t from element off[t] on) to `out`; lo lies in tube
+// m0.  One block per tube and field for the part of it in the range, or
+// gridDim.y of them.
+__global__ void __launch_bounds__(256) kb_pack(Args a, const long long* off, int m0, long long lo,
+                                               long long hi, double* out) {
   const int tube = m0 + (int)blockIdx.x / (NE + NBG), v = (int)blockIdx.x % (NE + NBG);
   const unsigned G0 = (unsigned)a.nxy[2 * tube] + 4;
   const unsigned G1 = a.ndim == 2 ? (unsigned)a.nxy[2 * tube + 1] + 4 : 1;
-  const long long p = a.pitch[tube], n = (long long)G0 * G1;
+  const long long p = a.pitch[tube], n = (long long)G0 * G1, at = off[tube] + v * n;
   const double* f = (v < NE ? a.reg[SAC_SLOT_W] + v * a.fs : a.bg + (v - NE) * a.fs) + a.start[tube];
-  double* o = out + (off[tube] - off[m0]) + v * n;
-  for (long long i = threadIdx.x; i < n; i += 256) {
+  const long long b = lo > at ? lo - at : 0, e = hi - at < n ? hi - at : n;
+  for (long long i = b + blockIdx.y * 256u + threadIdx.x; i < e; i += 256 * gridDim.y) {
     const long long r = (n >> 32) ? i / G0 : (long long)((unsigned)i / G0);
-    o[i] = f[r * p + (i - r * G0)];
+    out[at + i - lo] = f[r * p + (i - r * G0)];
   }
 }
 
@@ -1028,8 +1030,7 @@ int sac_batch_status(sac_batch_handle h, double* t, int* it, int* state) {
 int sac_batch_download(sac_batch_handle h, double* w) {
   if (!h || !w) return bfail(SAC_E_ARG, "null argument");
   Batch& b = *(Batch*)h;
-  // Chunks of consecutive members through pinned buffers (sac_xfer.h); a
-  // member larger than a buffer gets one of its size.
+  // Chunks of the host's layout through pinned buffers (sac_xfer.h)
   if (!b.d_hoff) {
     b.hoff.assign((size_t)b.ntubes + 1, 0);
     for (int i = 0; i < b.ntubes; i++)
@@ -1039,28 +1040,31 @@ int sac_batch_download(sac_batch_handle h, double* w) {
                    hipMemcpyHostToDevice));
   }
   constexpr long long kMost = (4LL << 20) / sizeof(double);
-  std::vector<int> first(1, 0);
-  long long most = 0;
-  for (int i = 0; i < b.ntubes;) {
-    int j = i + 1;
-    while (j < b.ntubes && b.hoff[j + 1] - b.hoff[i] <= kMost) j++;
-    most = std::max(most, b.hoff[j] - b.hoff[i]);
-    first.push_back(i = j);
-  }
+  const long long total = b.hoff.back();
+  // the tube that holds element k
+  auto tube_of = [&](long long k) {
+    return (int)(std::upper_bound(b.hoff.begin(), b.hoff.end(), k) - b.hoff.begin()) - 1;
+  };
   std::string err;
   const int rc = sac::xfer::for_chunks(
-      b.device, (long long)first.size() - 1, sizeof(double) * (size_t)most,
+      b.device, (total + kMost - 1) / kMost, sizeof(double) * (size_t)std::min(total, kMost),
       [&](long long c, void* pin, hipEvent_t ev, std::string& e) -> int {
-        const int m0 = first[c], m1 = first[c + 1];
-        hipError_t s = sac::xfer::launch(kb_pack, dim3((unsigned)(m1 - m0) * (NE + NBG)), dim3(256),
-                                         b.stream, b.a, b.d_hoff, m0, (double*)pin);
+        const long long lo = c * kMost, hi = std::min(total, lo + kMost);
+        const int m0 = tube_of(lo), m1 = tube_of(hi - 1) + 1;
+        // a block walks up to 4096 elements, or more than 64 blocks would share a field
+        long long most = 1;
+        for (int i = m0; i < m1; i++) most = std::max(most, (long long)b.gx(i) * b.gy(i));
+        const unsigned ny = (unsigned)std::min((std::min(most, kMost) + 4095) / 4096, 64LL);
+        hipError_t s = sac::xfer::launch(kb_pack, dim3((unsigned)(m1 - m0) * (NE + NBG), ny),
+                                         dim3(256), b.stream, b.a, b.d_hoff, m0, lo, hi,
+                                         (double*)pin);
         if (s == hipSuccess) s = hipEventRecord(ev, b.stream);
         if (s == hipSuccess) s = hipEventSynchronize(ev);
         if (s != hipSuccess) {
           e = std::string("download: ") + hipGetErrorString(s);
           return SAC_E_HIP;
         }
-        memcpy(w + b.hoff[m0], pin, sizeof(double) * (size_t)(b.hoff[m1] - b.hoff[m0]));
+        memcpy(w + lo, pin, sizeof(double) * (size_t)(hi - lo));
         return 0;
       },
       err);

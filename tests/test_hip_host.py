@@ -233,3 +233,16 @@ def test_ensemble_download_without_pinned_memory(stub, ndim):
             np.testing.assert_array_equal(got, p.w)
         assert hip.hipGetLastError() == 0
     """)
+
+
+def test_ensemble_download_pins_no_more_than_its_buffers(stub):
+    """However large the members are: eight buffers of 4 MB."""
+    hip_host.run(stub, """
+        ens = batch.Ensemble([state_problem((n,)) for n in (200000, 300, 150000, 90000)])
+        knob("pinned_peak", ctypes.c_size_t).value = 0
+        knob("pinned_most", ctypes.c_size_t).value = 0
+        ens.download()
+        assert 0 < knob("pinned_most", ctypes.c_size_t).value <= 4 << 20
+        assert knob("pinned_peak", ctypes.c_size_t).value <= 8 * (4 << 20)
+        assert knob("pinned_now", ctypes.c_size_t).value == 0
+    """)
