@@ -746,12 +746,14 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   b->start.resize(ntubes);
   b->pitch.resize(ntubes);
   b->dxo.resize(ntubes);
+  b->hoff.assign((size_t)ntubes + 1, 0);
   long long off = 0, doff = 0;
   for (int i = 0; i < ntubes; i++) {
     const int G0 = b->gx(i), G1 = b->gy(i);
     b->start[i] = off + sac::kFieldPad;  // each mesh row starts on a 128-byte line
     b->pitch[i] = (ndim == 1) ? G0 : (G0 + 15) / 16 * 16;
     off += ((long long)b->pitch[i] * G1 + sac::kFieldPad + sac::kFieldPadEnd + 15) / 16 * 16;
+    b->hoff[i + 1] = b->hoff[i] + (long long)G0 * G1 * (NE + NBG);
     b->dxo[i] = doff;
     doff += G0 + (ndim == 2 ? G1 : 0);
     b->max_frame = std::max(b->max_frame, 4 * G0 + 4 * (G1 - 4));
@@ -777,6 +779,7 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   if ((rc = balloc(*b, (void**)&b->d_it, sizeof(int) * ntubes))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_state, sizeof(int) * ntubes))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_dxmin, sizeof(double) * 2 * ntubes))) return bail(rc);
+  if ((rc = balloc(*b, (void**)&b->d_hoff, sizeof(long long) * b->hoff.size()))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_running, sizeof(unsigned int)))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_active, sizeof(int) * ntubes))) return bail(rc);
   b->active.resize(ntubes);
@@ -787,9 +790,9 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   std::vector<double> dxmin(2 * (size_t)ntubes, 1.0);
   std::vector<double> dxt((size_t)doff * sac::kDxTables);
   sac::fill_dx_tables(dxt.data(), doff, dx, doff);
-  long long hoff = 0;
   for (int i = 0; i < ntubes; i++) {
     const int G0 = b->gx(i), G1 = b->gy(i);
+    const long long hoff = b->hoff[i];
     for (int v = 0; v < NE + NBG; v++)
       for (int r = 0; r < G1; r++)
         memcpy(&pk[(size_t)v * b->fs + b->start[i] + (size_t)r * b->pitch[i]],
@@ -804,7 +807,6 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
       }
       dxmin[2 * i + d] = mn;
     }
-    hoff += (long long)G0 * G1 * (NE + NBG);
   }
   if (hipMemcpy(b->d_reg[SAC_SLOT_W], pk.data(), fb * NE, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(b->d_bg, pk.data() + (size_t)b->fs * NE, fb * NBG, hipMemcpyHostToDevice) !=
@@ -820,7 +822,9 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
       hipMemcpy(b->d_dxo, b->dxo.data(), sizeof(long long) * ntubes, hipMemcpyHostToDevice) !=
           hipSuccess ||
       hipMemcpy(b->d_dxmin, dxmin.data(), sizeof(double) * 2 * ntubes, hipMemcpyHostToDevice) !=
-          hipSuccess)
+          hipSuccess ||
+      hipMemcpy(b->d_hoff, b->hoff.data(), sizeof(long long) * b->hoff.size(),
+                hipMemcpyHostToDevice) != hipSuccess)
     return bail(bfail(SAC_E_HIP, "upload failed"));
   Args& a = b->a;
   a.ndim = ndim;
@@ -1031,14 +1035,6 @@ int sac_batch_download(sac_batch_handle h, double* w) {
   if (!h || !w) return bfail(SAC_E_ARG, "null argument");
   Batch& b = *(Batch*)h;
   // Chunks of the host's layout through pinned buffers (sac_xfer.h)
-  if (!b.d_hoff) {
-    b.hoff.assign((size_t)b.ntubes + 1, 0);
-    for (int i = 0; i < b.ntubes; i++)
-      b.hoff[i + 1] = b.hoff[i] + (long long)b.gx(i) * b.gy(i) * (NE + NBG);
-    if (int rc = balloc(b, (void**)&b.d_hoff, sizeof(long long) * b.hoff.size())) return rc;
-    BCHK(hipMemcpy(b.d_hoff, b.hoff.data(), sizeof(long long) * b.hoff.size(),
-                   hipMemcpyHostToDevice));
-  }
   constexpr long long kMost = (4LL << 20) / sizeof(double);
   const long long total = b.hoff.back();
   // the tube that holds element k

@@ -246,3 +246,14 @@ def test_ensemble_download_pins_no_more_than_its_buffers(stub):
         assert knob("pinned_peak", ctypes.c_size_t).value <= 8 * (4 << 20)
         assert knob("pinned_now", ctypes.c_size_t).value == 0
     """)
+
+
+def test_ensemble_download_allocates_nothing_on_the_device(stub):
+    hip_host.run(stub, """
+        probs = [state_problem((n,)) for n in (20000, 300)]
+        ens = batch.Ensemble(probs)
+        before = ens.memory()
+        knob("fail_malloc").value = 1
+        ens.download()
+        assert ens.memory() == before and knob("fail_malloc").value == 1
+    """)
