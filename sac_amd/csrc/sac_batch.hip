@@ -505,7 +505,45 @@ int balloc(Batch& b, void** p, size_t bytes) {
   return 0;
 }
 
-int set_shape(Batch& b, Shape s) {
+// Make shape s and the running members `active` the ones in use.  The new
+// tables are on the device before the old ones are freed, so that a call that
+// fails leaves everything as it was.
+int set_shape(Batch& b, Shape s, std::vector<int> active) {
+  std::vector<Tile> tiles, st;
+  bool rows_fit = true;
+  if (b.ndim == 1) {
+    const int span = s.ck * s.tb;
+    for (int i : active)
+      for (int c = 0; c < b.nxy[2 * i]; c += span) tiles.push_back({i, 2 + c, 0});
+  } else {
+    const int tby = s.tb / s.tbx;
+    for (int i : active)
+      for (int c1 = 0; c1 < b.nxy[2 * i + 1]; c1 += tby)
+        for (int c0 = 0; c0 < b.nxy[2 * i]; c0 += s.tbx) tiles.push_back({i, 2 + c0, 2 + c1});
+    // stage tiles of each running patch
+    for (int i : active) rows_fit = rows_fit && sac::tile::rows_fit(b.pitch[i]);
+    for (int i : active)
+      for (int c1 = 2; c1 < 2 + b.nxy[2 * i + 1]; c1 += sac::tile::TY)
+        for (int c0 = 2; c0 < 2 + b.nxy[2 * i]; c0 += sac::tile::TX) st.push_back({i, c0, c1});
+  }
+  const Tile none = {active.empty() ? 0 : active[0], 2, 2};
+  if (tiles.empty()) tiles.push_back(none);
+  if (st.empty()) st.push_back(none);
+  Tile* dt[2] = {nullptr, nullptr};  // tiles, stiles
+  const std::vector<Tile>* ht[2] = {&tiles, &st};
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < b.ndim && e == hipSuccess; k++) {
+    const size_t bytes = sizeof(Tile) * ht[k]->size();
+    e = hipMalloc((void**)&dt[k], bytes);
+    if (e == hipSuccess) e = hipMemcpy(dt[k], ht[k]->data(), bytes, hipMemcpyHostToDevice);
+  }
+  if (e == hipSuccess)
+    e = hipMemcpy(b.d_active, active.data(), sizeof(int) * active.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    for (Tile* t : dt)
+      if (t) hipFree(t);
+    return bfail(SAC_E_HIP, "tile tables: %s", hipGetErrorString(e));
+  }
   // the graph's kernel nodes hold the tile tables freed below: destroy the
   // executable graph first (the stream is idle here), so no graph ever
   // refers to freed memory
@@ -514,45 +552,19 @@ int set_shape(Batch& b, Shape s) {
     b.graph = nullptr;
   }
   b.graph_steps = 0;
-  std::vector<Tile> tiles;
-  if (b.ndim == 1) {
-    const int span = s.ck * s.tb;
-    for (int i : b.active)
-      for (int c = 0; c < b.nxy[2 * i]; c += span) tiles.push_back({i, 2 + c, 0});
-  } else {
-    const int tby = s.tb / s.tbx;
-    for (int i : b.active)
-      for (int c1 = 0; c1 < b.nxy[2 * i + 1]; c1 += tby)
-        for (int c0 = 0; c0 < b.nxy[2 * i]; c0 += s.tbx) tiles.push_back({i, 2 + c0, 2 + c1});
-  }
-  if (tiles.empty()) tiles.push_back({b.active.empty() ? 0 : b.active[0], 2, 2});
-  if (b.ndim == 2) {
-    // stage tiles of each running patch
-    std::vector<Tile> st;
-    b.rows_fit = true;
-    for (int i : b.active) b.rows_fit = b.rows_fit && sac::tile::rows_fit(b.pitch[i]);
-    for (int i : b.active)
-      for (int c1 = 2; c1 < 2 + b.nxy[2 * i + 1]; c1 += sac::tile::TY)
-        for (int c0 = 2; c0 < 2 + b.nxy[2 * i]; c0 += sac::tile::TX) st.push_back({i, c0, c1});
-    if (st.empty()) st.push_back({b.active.empty() ? 0 : b.active[0], 2, 2});
-    b.a.nstiles = (int)st.size();
-    if (b.d_stiles) hipFree(b.d_stiles);
-    b.d_stiles = nullptr;
-    BCHK(hipMalloc((void**)&b.d_stiles, sizeof(Tile) * st.size()));
-    BCHK(hipMemcpy(b.d_stiles, st.data(), sizeof(Tile) * st.size(), hipMemcpyHostToDevice));
-    b.a.stiles = b.d_stiles;
-  }
   if (b.d_tiles) hipFree(b.d_tiles);
-  b.d_tiles = nullptr;
-  BCHK(hipMalloc((void**)&b.d_tiles, sizeof(Tile) * tiles.size()));
-  BCHK(hipMemcpy(b.d_tiles, tiles.data(), sizeof(Tile) * tiles.size(), hipMemcpyHostToDevice));
+  if (b.d_stiles) hipFree(b.d_stiles);
+  b.d_tiles = dt[0];
+  b.d_stiles = dt[1];
   b.ntiles = (int)tiles.size();
   b.shape = s;
+  b.rows_fit = rows_fit;
+  b.active = std::move(active);
   b.a.tiles = b.d_tiles;
   b.a.ntiles = b.ntiles;
   b.a.tbx = s.tbx;
-  BCHK(hipMemcpy(b.d_active, b.active.data(), sizeof(int) * b.active.size(),
-                 hipMemcpyHostToDevice));
+  b.a.stiles = b.d_stiles;
+  b.a.nstiles = (int)st.size();
   b.a.active = b.d_active;
   b.a.nactive = (int)b.active.size();
   return 0;
@@ -695,8 +707,7 @@ int compact(Batch& b, int steps_per_graph) {
   for (int i : b.active)
     if (st[i] == RUNNING) act.push_back(i);
   if (act.empty() || act.size() == b.active.size()) return 0;
-  b.active.swap(act);
-  if (int rc = set_shape(b, b.shape)) return rc;
+  if (int rc = set_shape(b, b.shape, std::move(act))) return rc;
   b.compactions += 1;
   // graph runs recapture; direct-launch runs (steps_per_graph <= 0) never capture
   return steps_per_graph > 0 ? build_graph(b, steps_per_graph) : 0;
@@ -782,8 +793,8 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   if ((rc = balloc(*b, (void**)&b->d_hoff, sizeof(long long) * b->hoff.size()))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_running, sizeof(unsigned int)))) return bail(rc);
   if ((rc = balloc(*b, (void**)&b->d_active, sizeof(int) * ntubes))) return bail(rc);
-  b->active.resize(ntubes);
-  for (int i = 0; i < ntubes; i++) b->active[i] = i;
+  std::vector<int> all(ntubes);
+  for (int i = 0; i < ntubes; i++) all[i] = i;
   // host layout per tube: w(G0[,G1], nw) column-major, tubes one after
   // another; dx: G0 values (then G1 values) per tube
   std::vector<double> pk((size_t)b->fs * (NE + NBG), 0.0);
@@ -853,7 +864,7 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   a.dtmin = 1.0e-99;
   a.itmax = itmax;
   a.running = b->d_running;
-  if ((rc = set_shape(*b, ndim == 1 ? Shape{1, 128, 0} : Shape{1, 256, 64}))) return bail(rc);
+  if ((rc = set_shape(*b, ndim == 1 ? Shape{1, 128, 0} : Shape{1, 256, 64}, all))) return bail(rc);
   // initial getboundary (background and state) and cmax of W
   enqueue_ghost(*b, b->d_bg, NBG);
   enqueue_ghost(*b, b->d_reg[SAC_SLOT_W], NE);
@@ -923,7 +934,7 @@ int sac_batch_tune(sac_batch_handle h, int trial_steps, int* ck, int* tb, double
   const int nshape = (b.ndim == 1) ? (int)(sizeof(kShapes1) / sizeof(Shape)) : 1;
   for (int k = 0; k < nshape; k++) {
     const Shape s = shapes[k];
-    if (int rc = set_shape(b, s)) return rc;
+    if (int rc = set_shape(b, s, b.active)) return rc;
     if (int rc = build_graph(b, trial_steps)) return rc;
     BCHK(hipGraphLaunch(b.graph, b.stream));  // warm-up replay
     BCHK(hipStreamSynchronize(b.stream));
@@ -949,7 +960,7 @@ int sac_batch_tune(sac_batch_handle h, int trial_steps, int* ck, int* tb, double
                    hipMemcpyHostToDevice));
     if (int rc = restore_state(b, r0)) return rc;
   }
-  if (int rc = set_shape(b, bs)) return rc;
+  if (int rc = set_shape(b, bs, b.active)) return rc;
   if (ck) *ck = bs.ck;
   if (tb) *tb = bs.tb;
   if (ms_per_step) *ms_per_step = best;
@@ -964,7 +975,7 @@ int sac_batch_set_shape(sac_batch_handle h, int index) {
                                    : (int)(sizeof(kShapes2) / sizeof(Shape));
   if (index < 0 || index >= nshape)
     return bfail(SAC_E_ARG, "shape index %d outside 0..%d", index, nshape - 1);
-  return set_shape(b, shapes[index]);
+  return set_shape(b, shapes[index], b.active);
 }
 
 int sac_batch_shape(sac_batch_handle h, int* ck, int* tbx, int* tby) {

@@ -20,9 +20,9 @@ int hip_host_fail_malloc = 0;       /* the n-th hipMalloc from now on fails, onc
 int hip_host_fail_event = 0;        /* the n-th event creation from now on fails, once */
 int hip_host_fail_pinned = 0;       /* 1: every hipHostMalloc fails; 2: on other threads only */
 int hip_host_fail_launch = 0;       /* launches fail: 1 on other threads, 2 on the first thread */
-int hip_host_fail_new = 0;          /* the n-th operator new from now on fails, once */
 /* what happened */
 int hip_host_null_stores = 0;       /* kernels that would have used a null pointer */
+int hip_host_freed_used = 0;        /* ensemble kernels given memory that was freed */
 size_t hip_host_pinned_most = 0;    /* largest pinned allocation */
 size_t hip_host_pinned_now = 0;     /* pinned bytes, now and at most */
 size_t hip_host_pinned_peak = 0;
@@ -64,7 +64,15 @@ hipError_t hipMalloc(void **p, size_t n) {
   if (counted(&hip_host_fail_malloc)) return *p = NULL, err(NOMEM);
   return *p = calloc(1, n ? n : 1), OK;
 }
-hipError_t hipFree(void *p) { return free(p), OK; }
+static void *freed[4096]; /* kept, so that no allocation gets the address again */
+static int nfreed = 0;
+hipError_t hipFree(void *p) {
+  pthread_mutex_lock(&lock);
+  if (p && nfreed < 4096) freed[nfreed++] = p;
+  else free(p);
+  pthread_mutex_unlock(&lock);
+  return OK;
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) {
   (void)flags;
   if (hip_host_fail_pinned == 1 || (hip_host_fail_pinned == 2 && other())) return *p = NULL, err(NOMEM);
@@ -178,6 +186,11 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t sh
     if (kernels[k].host == f) {
       const char *t = strstr(kernels[k].name, "k_rowsI");
       if (t) rows(args, t[7] == 'm' ? 8 : 4, strncmp(t + 8, "Lb1", 3) == 0);
+      /* the pointers of sac::batch::Args, which is longer than this */
+      if (strstr(kernels[k].name, "sac5batch") && strstr(kernels[k].name, "NS0_4ArgsE"))
+        for (int w = 0; w < 25; w++)
+          for (int j = 0; j < nfreed; j++)
+            hip_host_freed_used += ((void **)args[0])[w] == freed[j];
       return OK;
     }
   return err(INVALID);

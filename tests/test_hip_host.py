@@ -257,3 +257,28 @@ def test_ensemble_download_allocates_nothing_on_the_device(stub):
         ens.download()
         assert ens.memory() == before and knob("fail_malloc").value == 1
     """)
+
+
+@pytest.mark.parametrize("ndim,n", [(1, 1), (2, 1), (2, 2)])
+def test_shape_whose_tables_cannot_be_allocated(stub, ndim, n):
+    """The ensemble goes on with the tables it has."""
+    hip_host.run(stub, f"""
+        probs = [state_problem((n,) if {ndim} == 1 else (n, 60 - n // 2)) for n in (6, 33, 90)]
+        ens = batch.Ensemble(probs)
+        ens.run(steps_per_graph=-1, max_steps=1)
+        assert knob("freed_used").value == 0
+        was = ens.shape()
+        knob("fail_malloc").value = {n}
+        try:
+            ens.set_shape(0)
+        except device.SacError:
+            assert ens.shape() == was
+        else:
+            assert knob("fail_malloc").value > 0  # it takes fewer allocations
+        knob("fail_malloc").value = 0
+        ens.run(steps_per_graph=-1, max_steps=1)
+        assert knob("freed_used").value == 0
+        ens.set_shape(0)
+        ens.run(steps_per_graph=-1, max_steps=1)
+        assert knob("freed_used").value == 0
+    """)
