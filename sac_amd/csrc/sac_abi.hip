@@ -432,6 +432,20 @@ void stage(Dev& d, int wct, int base, int out, double qa, bool rk4_last = false)
   }
 }
 
+void closure_free(Closure* c) {
+  if (!c) return;
+  hipFree(c->P32);
+  hipFree(c->P16);
+  hipFree(c->m1);
+  hipFree(c->m2);
+  hipFree(c->partial);
+  hipFree(c->loss);
+  for (int k = 0; k < 3; k++) hipFree(c->RF[k]);
+  hipFree(c->feat);
+  hipFree(c->targ);
+  delete c;
+}
+
 int check_handle(sac_handle h) {
   if (!h) return fail(SAC_E_ARG, "null handle");
   return 0;
@@ -704,19 +718,7 @@ int sac_dev_free(sac_handle h) {
   hipFree(d->red);
   if (d->red_host) hipHostFree(d->red_host);
   if (d->pin) hipHostFree(d->pin);
-  if (d->cl) {
-    Closure* c = d->cl;
-    hipFree(c->P32);
-    hipFree(c->P16);
-    hipFree(c->m1);
-    hipFree(c->m2);
-    hipFree(c->partial);
-    hipFree(c->loss);
-    for (int k = 0; k < 3; k++) hipFree(c->RF[k]);
-    hipFree(c->feat);
-    hipFree(c->targ);
-    delete c;
-  }
+  closure_free(d->cl);
   if (d->save_stream) hipStreamSynchronize(d->save_stream);
   hipFree(d->save_dev);
   if (d->save_host) hipHostFree(d->save_host);
@@ -1121,7 +1123,12 @@ int sac_closure_init(sac_handle h, long long capacity, int max_blocks, unsigned 
   if (d.prec != SAC_PREC_FP64) return fail(SAC_E_UNSUPPORTED, "the learned closure runs in FP64 storage");
   if (capacity < 0 || max_blocks < 1) return fail(SAC_E_ARG, "capacity/max_blocks");
   Closure* c = new Closure();
-  d.cl = c;
+  const long long bytes = d.bytes;
+  auto bail = [&](int code) {
+    closure_free(c);
+    d.bytes = bytes;
+    return code;
+  };
   const int NP = sac::mlp::NPARAM;
   int rc = 0;
   if ((rc = balloc(d, (void**)&c->P32, sizeof(float) * NP)) ||
@@ -1130,15 +1137,15 @@ int sac_closure_init(sac_handle h, long long capacity, int max_blocks, unsigned 
       (rc = balloc(d, (void**)&c->m2, sizeof(float) * NP)) ||
       (rc = balloc(d, (void**)&c->partial, sizeof(float) * (size_t)NP * max_blocks)) ||
       (rc = balloc(d, (void**)&c->loss, sizeof(float) * max_blocks)))
-    return rc;
+    return bail(rc);
   c->max_blocks = max_blocks;
   const int np_var = 2 * d.ndim + 1;
   for (int k = 0; k < d.ndim; k++)
-    if ((rc = balloc(d, (void**)&c->RF[k], sizeof(float) * (size_t)np_var * d.g.fs))) return rc;
+    if ((rc = balloc(d, (void**)&c->RF[k], sizeof(float) * (size_t)np_var * d.g.fs))) return bail(rc);
   if (capacity > 0) {
     if ((rc = balloc(d, (void**)&c->feat, sizeof(uint16_t) * sac::closure::kFeat * (size_t)capacity)) ||
         (rc = balloc(d, (void**)&c->targ, sizeof(float) * sac::closure::kTarg * (size_t)capacity)))
-      return rc;
+      return bail(rc);
   }
   c->cap = capacity;
   // He-normal initial weights (fan-in), zero biases, from a seeded
@@ -1163,9 +1170,13 @@ int sac_closure_init(sac_handle h, long long capacity, int max_blocks, unsigned 
   fill(OFF_W2, H, H);
   fill(OFF_W3, H, H);
   fill(OFF_W4, OUT, H);
-  HIPCHK(hipMemcpy(c->P32, p.data(), sizeof(float) * NP, hipMemcpyHostToDevice));
-  sac::closure::launch_to_bf16(c->P32, c->P16, d.stream);
-  HIPCHK(hipStreamSynchronize(d.stream));
+  hipError_t e = hipMemcpy(c->P32, p.data(), sizeof(float) * NP, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    sac::closure::launch_to_bf16(c->P32, c->P16, d.stream);
+    e = hipStreamSynchronize(d.stream);
+  }
+  if (e != hipSuccess) return bail(fail(SAC_E_HIP, "parameters: %s", hipGetErrorString(e)));
+  d.cl = c;
   return 0;
 }
 

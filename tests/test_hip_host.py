@@ -282,3 +282,28 @@ def test_shape_whose_tables_cannot_be_allocated(stub, ndim, n):
         ens.run(steps_per_graph=-1, max_steps=1)
         assert knob("freed_used").value == 0
     """)
+
+
+@pytest.mark.parametrize("n", [1, 3, 7, 9])
+def test_closure_that_cannot_be_allocated(stub, n):
+    """It is not there, its memory is given back, and it can be asked for
+    again."""
+    hip_host.run(stub, f"""
+        from sac_amd import closure
+        p = state_problem((16, 9, 8))
+        dev = device.Device(p)
+        before = dev.memory()
+        knob("fail_malloc").value = {n}
+        try:
+            closure.Closure(dev, capacity=1000)
+        except device.SacError as e:
+            assert "hipMalloc" in str(e), e
+        else:
+            raise AssertionError("no error")
+        assert dev.memory() == before
+        L = closure._lib()
+        assert L.sac_closure_enable(dev.handle, 1, 0.1) == 1  # not initialised
+        closure.Closure(dev, capacity=1000)
+        assert dev.memory() > before
+        assert L.sac_closure_enable(dev.handle, 1, 0.1) == 0
+    """)
