@@ -788,7 +788,13 @@ int sac_dev_save_begin(sac_handle h) {
   const size_t bytes = d.esz * (size_t)d.ncell_grid * (size_t)d.ne;
   if (int rc = save_resources(d, bytes)) return rc;
   if (!d.bg_host) {  // the background is static: one synchronous copy
-    auto bg = std::make_shared<std::vector<double>>((size_t)d.nbg * (size_t)d.ncell_grid);
+    std::shared_ptr<std::vector<double>> bg;
+    std::string err;
+    if (int rc = sac::xfer::guarded(err, [&] {
+          bg = std::make_shared<std::vector<double>>((size_t)d.nbg * (size_t)d.ncell_grid);
+          return 0;
+        }))
+      return fail(rc, "%s", err.c_str());
     if (int rc = copy_bg_out(d, bg->data())) return rc;
     d.bg_host = bg;
   }

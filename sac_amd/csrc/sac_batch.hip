@@ -1042,9 +1042,7 @@ int sac_batch_status(sac_batch_handle h, double* t, int* it, int* state) {
   return 0;
 }
 
-int sac_batch_download(sac_batch_handle h, double* w) {
-  if (!h || !w) return bfail(SAC_E_ARG, "null argument");
-  Batch& b = *(Batch*)h;
+static int download(Batch& b, double* w, std::string& err) {
   // Chunks of the host's layout through pinned buffers (sac_xfer.h)
   constexpr long long kMost = (4LL << 20) / sizeof(double);
   const long long total = b.hoff.back();
@@ -1052,7 +1050,6 @@ int sac_batch_download(sac_batch_handle h, double* w) {
   auto tube_of = [&](long long k) {
     return (int)(std::upper_bound(b.hoff.begin(), b.hoff.end(), k) - b.hoff.begin()) - 1;
   };
-  std::string err;
   const int rc = sac::xfer::for_chunks(
       b.device, (total + kMost - 1) / kMost, sizeof(double) * (size_t)std::min(total, kMost),
       [&](long long c, void* pin, hipEvent_t ev, std::string& e) -> int {
@@ -1075,13 +1072,17 @@ int sac_batch_download(sac_batch_handle h, double* w) {
         return 0;
       },
       err);
-  if (rc != sac::xfer::kNoPinned) return rc ? bfail(rc, "%s", err.c_str()) : 0;
+  if (rc != sac::xfer::kNoPinned) return rc;
   // no pinned memory: field by field through ordinary memory
-  BCHK(hipStreamSynchronize(b.stream));
   std::vector<double> f((size_t)b.fs);
+  hipError_t s = hipStreamSynchronize(b.stream);
   for (int v = 0; v < NE + NBG; v++) {
     const double* src = v < NE ? b.d_reg[SAC_SLOT_W] + v * b.fs : b.d_bg + (v - NE) * b.fs;
-    BCHK(hipMemcpy(f.data(), src, sizeof(double) * f.size(), hipMemcpyDeviceToHost));
+    if (s == hipSuccess) s = hipMemcpy(f.data(), src, sizeof(double) * f.size(), hipMemcpyDeviceToHost);
+    if (s != hipSuccess) {
+      err = std::string("download: ") + hipGetErrorString(s);
+      return SAC_E_HIP;
+    }
     for (int i = 0; i < b.ntubes; i++) {
       const int G0 = b.gx(i), G1 = b.gy(i);
       for (int r = 0; r < G1; r++)
@@ -1090,6 +1091,13 @@ int sac_batch_download(sac_batch_handle h, double* w) {
     }
   }
   return 0;
+}
+
+int sac_batch_download(sac_batch_handle h, double* w) {
+  if (!h || !w) return bfail(SAC_E_ARG, "null argument");
+  std::string err;
+  const int rc = sac::xfer::guarded(err, [&] { return download(*(Batch*)h, w, err); });
+  return rc ? bfail(rc, "%s", err.c_str()) : 0;
 }
 
 int sac_batch_memory(sac_batch_handle h, long long* bytes) {

@@ -3,10 +3,12 @@
 // layout, pinned buffers, and host threads that copy.
 #pragma once
 #include <algorithm>
+#include <exception>
 #include <functional>
 #include <string>
 #include <tuple>
 
+#include "../../include/sac_amd.h"
 #include "sac_common.h"
 
 namespace sac {
@@ -31,6 +33,17 @@ struct Fields {
 constexpr size_t kSmall = size_t(1) << 19;
 int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n, bool to_host,
          void** small, std::string& err);
+
+// f() with what it throws made an error: nothing may leave a C entry point
+template <typename F>
+int guarded(std::string& err, const F& f) {
+  try {
+    return f();
+  } catch (const std::exception&) {
+    err = "no host memory";  // short enough for a string without memory of its own
+    return SAC_E_NOMEM;
+  }
+}
 
 // Launch a kernel and return this launch's own error.  The last error that the
 // runtime keeps is one per thread, so that of a worker is not seen by the

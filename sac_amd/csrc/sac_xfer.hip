@@ -16,11 +16,8 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
-#include <system_error>
 #include <thread>
 #include <vector>
-
-#include "../../include/sac_amd.h"
 
 namespace sac {
 namespace xfer {
@@ -69,8 +66,9 @@ void parallel_slices(size_t n, size_t per_thread, const F& fn) {
   auto slice = [&](size_t t) { fn(n * t / nt, n * (t + 1) / nt); };
   size_t t = 1;
   try {
+    th.reserve(nt);
     for (; t < nt; t++) th.emplace_back(slice, t);
-  } catch (const std::system_error&) {  // no more threads: the rest here
+  } catch (const std::exception&) {  // no more threads, or memory for them: the rest here
   }
   slice(0);
   for (; t < nt; t++) slice(t);
@@ -115,15 +113,15 @@ void host_copy(double* dst, const float* src, size_t n) {
   });
 }
 
-int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::string& err) {
-  if (n <= 0) return 0;
+static int run_chunks(int device, long long n, size_t bytes, const ChunkFn& fn,
+                      std::string& err) {
   const long long hw = std::max(1u, std::thread::hardware_concurrency());
   const int nt = (int)std::min<long long>({(long long)kWorkers, hw, n});
   std::vector<std::string> errs((size_t)nt);
   std::vector<int> rcs((size_t)nt, 0);
   std::atomic<long long> next{0};
   std::atomic<bool> stop{false};
-  auto worker = [&](int t) {
+  auto work = [&](int t) {
     void* pin = nullptr;
     hipEvent_t ev = nullptr;
     int rc = hip_err(hipSetDevice(device), "hipSetDevice", errs[t]);
@@ -135,7 +133,7 @@ int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::st
     while (!rc && !stop) {
       const long long c = next.fetch_add(1);
       if (c >= n) break;
-      rc = fn(c, pin, ev, errs[t]);
+      rc = guarded(errs[t], [&] { return fn(c, pin, ev, errs[t]); });
     }
     // the buffer's last chunk may still be on its way to the device
     if (ev) {
@@ -147,10 +145,17 @@ int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::st
     if (rc) stop = true;
     rcs[t] = rc;
   };
+  auto worker = [&](int t) {
+    if (int rc = guarded(errs[t], [&] { return work(t), 0; })) {
+      rcs[t] = rc;
+      stop = true;
+    }
+  };
   std::vector<std::thread> th;
   try {
+    th.reserve((size_t)nt);
     for (int t = 1; t < nt; t++) th.emplace_back(worker, t);
-  } catch (const std::system_error&) {  // the threads there are take the chunks
+  } catch (const std::exception&) {  // the threads there are take the chunks
   }
   // this thread is the caller's: its current device comes back
   int current = device;
@@ -164,6 +169,11 @@ int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::st
       return rcs[t];
     }
   return next ? 0 : kNoPinned;  // a thread with a buffer takes chunks until there are none
+}
+
+int for_chunks(int device, long long n, size_t bytes, const ChunkFn& fn, std::string& err) {
+  if (n <= 0) return 0;
+  return guarded(err, [&] { return run_chunks(device, n, bytes, fn, err); });
 }
 
 // Without pinned memory: field by field with the runtime's own copies of rows,
@@ -222,8 +232,8 @@ static int copy_small(const GridDesc& g, hipStream_t stream, const Fields* f, in
   return 0;
 }
 
-int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n, bool to_host,
-         void** small, std::string& err) {
+static int copy_any(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n,
+                    bool to_host, void** small, std::string& err) {
   const long long ncell = (long long)g.G[0] * g.G[1] * g.G[2];
   size_t all = 0;
   for (int k = 0; k < n; k++) all += (size_t)ncell * f[k].nfield * f[k].esz + 16;
@@ -257,6 +267,11 @@ int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int
   };
   const int rc = for_chunks(device, first[n], bytes, fn, err);
   return rc == kNoPinned ? copy_plain(g, stream, f, n, to_host, err) : rc;
+}
+
+int copy(const GridDesc& g, int device, hipStream_t stream, const Fields* f, int n, bool to_host,
+         void** small, std::string& err) {
+  return guarded(err, [&] { return copy_any(g, device, stream, f, n, to_host, small, err); });
 }
 
 hipError_t launch_pack(const GridDesc& g, const Fields& f, void* out, hipStream_t stream) {

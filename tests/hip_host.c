@@ -5,6 +5,7 @@
  * its failure paths can be run without a GPU.  Each hip_host_* variable sets a
  * failure or counts what happened. */
 #define _GNU_SOURCE
+#include <dlfcn.h>
 #include <pthread.h>
 #include <stdint.h>
 #include <stdlib.h>
@@ -20,6 +21,7 @@ int hip_host_fail_malloc = 0;       /* the n-th hipMalloc from now on fails, onc
 int hip_host_fail_event = 0;        /* the n-th event creation from now on fails, once */
 int hip_host_fail_pinned = 0;       /* 1: every hipHostMalloc fails; 2: on other threads only */
 int hip_host_fail_launch = 0;       /* launches fail: 1 on other threads, 2 on the first thread */
+int hip_host_fail_new = 0;          /* the n-th operator new from now on throws, once */
 /* what happened */
 int hip_host_null_stores = 0;       /* kernels that would have used a null pointer */
 int hip_host_freed_used = 0;        /* ensemble kernels given memory that was freed */
@@ -43,6 +45,16 @@ static int counted(int *n) { /* the call that brings *n to 0 */
   const int hit = *n > 0 && --*n == 0;
   pthread_mutex_unlock(&lock);
   return hit;
+}
+
+/* ---- operator new of the library ---- */
+void *_Znwm(size_t n) {
+  if (counted(&hip_host_fail_new)) {
+    void (*bad)(void) = (void (*)(void))dlsym(RTLD_DEFAULT, "_ZSt17__throw_bad_allocv");
+    if (bad) bad();
+    abort();
+  }
+  return malloc(n ? n : 1);
 }
 
 /* ---- errors and devices ---- */
@@ -181,7 +193,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t sh
     pthread_mutex_unlock(&lock);
   }
   if (hip_host_fail_launch && hip_host_fail_launch == (other() ? 1 : 2)) return err(LAUNCH);
-  if (hip_host_fail_launch) usleep(20000); /* the failing threads get chunks too */
+  if (hip_host_fail_launch) usleep(5000); /* the failing threads get chunks too */
   for (int k = 0; k < nkernels; k++)
     if (kernels[k].host == f) {
       const char *t = strstr(kernels[k].name, "k_rowsI");

@@ -13,6 +13,7 @@ import ctypes, sys
 import numpy as np
 sys.path.insert(0, {root!r})
 hip = ctypes.CDLL({stub!r}, mode=ctypes.RTLD_GLOBAL)
+ctypes.CDLL("libstdc++.so.6", mode=ctypes.RTLD_GLOBAL)  # what operator new throws
 
 def knob(name, kind=ctypes.c_int):
     return kind.in_dll(hip, "hip_host_" + name)
@@ -39,7 +40,7 @@ def state_problem(n, seed=5):
 
 def build(folder):
     out = os.path.join(str(folder), "hip_host.so")
-    subprocess.run(["gcc", "-O2", "-Wall", "-shared", "-fPIC", "-pthread",
+    subprocess.run(["gcc", "-O2", "-Wall", "-fexceptions", "-shared", "-fPIC", "-pthread",
                     os.path.join(HERE, "hip_host.c"), "-o", out], check=True)
     return out
 

@@ -307,3 +307,46 @@ def test_closure_that_cannot_be_allocated(stub, n):
         assert dev.memory() > before
         assert L.sac_closure_enable(dev.handle, 1, 0.1) == 0
     """)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_copies_without_host_memory(stub, precision):
+    """Where the host has no memory left for a thread or a list, a copy is
+    slower or an error, never an exception out of a C entry point."""
+    hip_host.run(stub, f"""
+        p = state_problem((70, 61, 64))
+        dev = device.Device(p, precision={precision!r})
+        dev.upload(p.w)
+        want = dev.download()
+        dev.save_begin()
+        dev.save_end()
+        ens = batch.Ensemble([state_problem((n,)) for n in (20000, 30000, 40000, 50000)])
+        ens.download()
+
+        def save():
+            dev.save_begin()
+            return dev.save_end()
+
+        def first_save():  # copies the background too
+            dev.upload(want)
+            knob("fail_new").value = n
+            return save()
+
+        lost = done = 0
+        for call in (lambda: dev.upload(p.w), dev.download, ens.download, save, first_save):
+            for n in range(1, 20):
+                knob("fail_new").value = n
+                try:
+                    got = call()
+                    if knob("fail_new").value == 0:
+                        done += 1
+                    if call not in (ens.download,) and got is not None:
+                        np.testing.assert_array_equal(got, want)
+                except device.SacError as e:
+                    assert "host memory" in str(e), e
+                    lost += 1
+                knob("fail_new").value = 0
+        assert lost > 0 and done > 0
+        dev.upload(p.w)
+        np.testing.assert_array_equal(dev.download(), want)
+    """)
