@@ -295,15 +295,14 @@ int sac_batch_free(sac_batch_handle h);
 /* Autotuner: times trial_steps steps for every launch shape from the
  * current state, restores the state, keeps the fastest shape.  Tubes: LDS
  * line tiles of tb in {64,128,256} cells, one per thread (ck = 1).
- * Patches: a stage has one tile (16 x 16 cells), so one shape is timed; the
- * shapes, tiles of tbx x tb/tbx cells for tb in {64,128,256} and tbx in
- * {16,...,tb} (12 of them), are those of the first cmax sweep. */
+ * Patches: a stage has one tile, 16 x 16 cells, which is timed. */
 int sac_batch_tune(sac_batch_handle h, int trial_steps, int *ck, int *tb, double *ms_per_step);
-/* Use launch shape `index` of the autotuner's list (tubes 0..2, patches
- * 0..11) without timing. */
+/* Use launch shape `index` without timing: tubes 0..2 (64, 128, 256 cells);
+ * patches 0..11, tiles of tbx x tb/tbx cells for tb in {64,128,256} and tbx
+ * in {16,...,tb}, which are kept for sac_batch_shape and change nothing. */
 int sac_batch_set_shape(sac_batch_handle h, int index);
-/* The current tile: cells per thread (ck) and the tile's extent along x and
- * y in cells (tubes: tbx = threads*ck, tby = 1; patches: ck = 1). */
+/* The shape in use: cells per thread (ck = 1) and the extent along x and y in
+ * cells (tubes: the tile, tby = 1; patches: as set, see above). */
 int sac_batch_shape(sac_batch_handle h, int *ck, int *tbx, int *tby);
 /* Advance every tube to its end, replaying a graph of steps_per_graph steps
  * at most max_steps steps in total; returns the steps issued.

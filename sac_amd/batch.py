@@ -114,14 +114,15 @@ class Ensemble:
         return ck.value, tb.value, ms.value
 
     def shape(self):
-        """Current tile: (cells per thread, extent along x, extent along y)."""
+        """Shape in use: (cells per thread, extent along x, extent along y); a
+        patch stage's tile is 16 x 16 whatever was set."""
         ck, tx, ty = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         _check(_lib().sac_batch_shape(self._h, ctypes.byref(ck), ctypes.byref(tx),
                                       ctypes.byref(ty)))
         return ck.value, tx.value, ty.value
 
     def set_shape(self, index):
-        """Use launch shape `index` of the autotuner's list without timing."""
+        """Use launch shape `index` without timing (patches: no effect)."""
         _check(_lib().sac_batch_set_shape(self._h, index))
 
     def run(self, steps_per_graph=32, max_steps=10 ** 7):
@@ -175,9 +176,8 @@ def _main():
                         ("patches", patch_ensemble(count=args.patches))):
         e = Ensemble(probs, courantpar=0.3, tmax=0.1)
         n = e.run(steps_per_graph=-1, max_steps=args.steps)
-        ck, tx, ty = e.shape()
         e.close()
-        print(f"{name}: {len(probs)} problems, {n} steps, tile {tx}x{ty}", flush=True)
+        print(f"{name}: {len(probs)} problems, {n} steps", flush=True)
 
 
 if __name__ == "__main__":

@@ -64,11 +64,8 @@ struct Args {
   const long long* dxo;      // offset of each tube's cell widths in dx (x, then y)
   const Tile* tiles;         // tiles of the tubes in `active`
   int ntiles;
-  int tbx;                   // tile width along x in cells (2-D)
   const int* active;         // tubes still running when the tiles were built
   int nactive;
-  const Tile* stiles;        // patches: stage tiles (first cell at column c0 and row c1)
-  int nstiles;
   double* reg[kSlots];
   const double* bg;
   const double* dx;          // cell widths per tube: G_x values, then G_y values
@@ -111,23 +108,6 @@ __device__ __forceinline__ GridDesc tube_grid(const Args& a, int tube) {
 
 __device__ __forceinline__ unsigned long long* red_of(const Args& a, int tube, int slot) {
   return a.red + ((size_t)tube * kSlots + slot) * kRed;
-}
-
-// cell of thread `tid`: cell j of its group of CK along x (tubes), or its
-// position in the tile (patches, CK = 1); false outside the mesh
-template <int NDIM, int CK>
-__device__ __forceinline__ bool tile_cell(const Args& a, const Tile& tl, const GridDesc& g, int j,
-                                          int (&c)[3]) {
-  const int tid = (int)threadIdx.x;
-  if (NDIM == 1) {
-    c[0] = tl.c0 + tid * CK + j;
-    c[1] = c[2] = 0;
-    return c[0] <= g.Mhi[0];
-  }
-  c[0] = tl.c0 + tid % a.tbx;
-  c[1] = tl.c1 + tid / a.tbx;
-  c[2] = 0;
-  return c[0] <= g.Mhi[0] && c[1] <= g.Mhi[1];
 }
 
 // 'cont' ghost cells (getboundary, src/vacgrid.t:366-370) whose value is
@@ -185,8 +165,8 @@ __global__ void __launch_bounds__(tile::NT, 4) kb_patch_stage(Args a, int wct, i
   __shared__ tile::Smem<2, NDIR, double, false> sm;
   // each XCD takes one contiguous range of tiles (shared halos in one L2)
   const unsigned b = xcd_block8();
-  if (b >= (unsigned)a.nstiles) return;
-  const Tile tl = a.stiles[b];
+  if (b >= (unsigned)a.ntiles) return;
+  const Tile tl = a.tiles[b];
   if (a.state[tl.tube] != RUNNING) return;  // uniform over the block
   const GridDesc g = tube_grid<2>(a, tl.tube);
   clear_red_w(a, tl.tube, tl.c0 == g.Mlo[0] && tl.c1 == g.Mlo[1], out);
@@ -253,8 +233,8 @@ __global__ void __launch_bounds__(LT) kb_tube_stage(Args a, int wct, int base, i
   block_max_atomic<3>(r, red_of(a, tl.tube, out), a.visc + tl.tube);
 }
 
-// cmax reductions of register `slot` of every running tube
-template <int NDIM, int CK>
+// cmax reductions of register `slot` of every running tube, one cell per thread
+template <int NDIM>
 __global__ void __launch_bounds__(256) kb_cmax(Args a, int slot) {
   const Tile tl = a.tiles[blockIdx.x];
   if (a.state[tl.tube] != RUNNING) return;
@@ -264,20 +244,18 @@ __global__ void __launch_bounds__(256) kb_cmax(Args a, int slot) {
   double redv[2 * NDIM];
 #pragma unroll
   for (int k = 0; k < 2 * NDIM; k++) redv[k] = 0.0;
+  const int t = (int)threadIdx.x;
+  const int c[2] = {tl.c0 + (NDIM == 1 ? t : t % tile::TX), NDIM == 1 ? 0 : tl.c1 + t / tile::TX};
+  if (c[0] <= g.Mhi[0] && (NDIM == 1 || c[1] <= g.Mhi[1])) {
+    Pt<NDIR, double> p;
+    load_pt<NDIR, double, double>(a.reg[slot] + o, a.bg + o, a.fs, lin(g, c[0], c[1], 0), p);
+    double cm[NDIM];
+    cmax_all<NDIM, NDIR>(p, a.gamma, cm);
 #pragma unroll
-  for (int j = 0; j < CK; j++) {
-    int c[3];
-    if (tile_cell<NDIM, CK>(a, tl, g, j, c)) {
-      Pt<NDIR, double> p;
-      load_pt<NDIR, double, double>(a.reg[slot] + o, a.bg + o, a.fs, lin(g, c[0], c[1], c[2]), p);
-      double cm[NDIM];
-      cmax_all<NDIM, NDIR>(p, a.gamma, cm);
-#pragma unroll
-      for (int d = 0; d < NDIM; d++) {
-        const double dxd = (d == 0) ? dx0[c[0]] : dx0[g.G[0] + c[1]];
-        redv[d] = fmax(redv[d], cm[d]);
-        redv[NDIM + d] = fmax(redv[NDIM + d], cm[d] / dxd);
-      }
+    for (int d = 0; d < NDIM; d++) {
+      const double dxd = (d == 0) ? dx0[c[0]] : dx0[g.G[0] + c[1]];
+      redv[d] = cm[d];
+      redv[NDIM + d] = cm[d] / dxd;
     }
   }
   block_max_atomic<2 * NDIM>(redv, red_of(a, tl.tube, slot));
@@ -430,22 +408,22 @@ int bfail(int code, const char* fmt, ...) {
     if (e_ != hipSuccess) return bfail(SAC_E_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
   } while (0)
 
-// launch shapes the autotuner chooses from.  Tubes: tiles of tb consecutive
-// cells of one tube, one cell per thread (kb_tube_stage<tb>).  Patches: a
-// stage has one tile, 16 x 16 cells; the shapes, tbx x (tb/tbx) cells, are
-// those of the first cmax sweep, and the autotuner times the steps only.
-// Every shape gives the same result bit for bit.
+// Launch shapes.  Tubes: tiles of tb consecutive cells of one tube, one cell
+// per thread (kb_tube_stage<tb>), which the autotuner chooses from; every one
+// gives the same result bit for bit.  Patches: a stage has one tile, 16 x 16
+// cells.  The shapes that callers can set and read there, tbx x (tb/tbx)
+// cells, are those of earlier patch kernels and reach no kernel.
 struct Shape {
-  int ck, tb, tbx;
+  int tb, tbx;
 };
 // Tubes start with 128: of tubes of 200 to 2000 cells the last tile leaves 5 %
 // of the threads idle instead of 10 (stage 0.283 ms against 0.312; 64 cells
 // 0.281 but 0.366 against 0.363 in RK4's last); on one tube of 10^6 cells, where
 // no tile is idle, the two lengths differ by 1 % (61.0 and 60.2 us).
-const Shape kShapes1[] = {{1, 64, 0}, {1, 128, 0}, {1, 256, 0}};
-const Shape kShapes2[] = {{1, 64, 16},  {1, 64, 32},  {1, 64, 64},   {1, 128, 16},
-                          {1, 128, 32}, {1, 128, 64}, {1, 128, 128}, {1, 256, 16},
-                          {1, 256, 32}, {1, 256, 64}, {1, 256, 128}, {1, 256, 256}};
+const Shape kShapes1[] = {{64, 0}, {128, 0}, {256, 0}};
+const Shape kShapes2[] = {{64, 16},  {64, 32},  {64, 64},   {128, 16},
+                          {128, 32}, {128, 64}, {128, 128}, {256, 16},
+                          {256, 32}, {256, 64}, {256, 128}, {256, 256}};
 
 struct Batch {
   int device = 0;
@@ -466,7 +444,6 @@ struct Batch {
   int* d_pitch = nullptr;
   long long* d_dxo = nullptr;
   Tile* d_tiles = nullptr;
-  Tile* d_stiles = nullptr;
   bool rows_fit = true;          // 32-bit offsets in the stage tiles
   int* d_active = nullptr;
   double* d_reg[kSlots] = {nullptr, nullptr, nullptr, nullptr};
@@ -483,7 +460,7 @@ struct Batch {
   std::vector<long long> hoff;   // element of each tube in the host's layout, and the end
   long long* d_hoff = nullptr;
   unsigned int* d_running = nullptr;
-  Shape shape{2, 128, 0};
+  Shape shape{128, 0};
   int ntiles = 0;
   hipGraphExec_t graph = nullptr;
   int graph_steps = 0;
@@ -506,43 +483,30 @@ int balloc(Batch& b, void** p, size_t bytes) {
 }
 
 // Make shape s and the running members `active` the ones in use.  The new
-// tables are on the device before the old ones are freed, so that a call that
-// fails leaves everything as it was.
+// table is on the device before the old one is freed, so that a call that fails
+// leaves everything as it was.
 int set_shape(Batch& b, Shape s, std::vector<int> active) {
-  std::vector<Tile> tiles, st;
+  std::vector<Tile> tiles;
   bool rows_fit = true;
-  if (b.ndim == 1) {
-    const int span = s.ck * s.tb;
-    for (int i : active)
-      for (int c = 0; c < b.nxy[2 * i]; c += span) tiles.push_back({i, 2 + c, 0});
-  } else {
-    const int tby = s.tb / s.tbx;
-    for (int i : active)
-      for (int c1 = 0; c1 < b.nxy[2 * i + 1]; c1 += tby)
-        for (int c0 = 0; c0 < b.nxy[2 * i]; c0 += s.tbx) tiles.push_back({i, 2 + c0, 2 + c1});
-    // stage tiles of each running patch
-    for (int i : active) rows_fit = rows_fit && sac::tile::rows_fit(b.pitch[i]);
-    for (int i : active)
+  for (int i : active) {
+    rows_fit = rows_fit && sac::tile::rows_fit(b.pitch[i]);
+    if (b.ndim == 1) {
+      for (int c = 2; c < 2 + b.nxy[2 * i]; c += s.tb) tiles.push_back({i, c, 0});
+    } else {
       for (int c1 = 2; c1 < 2 + b.nxy[2 * i + 1]; c1 += sac::tile::TY)
-        for (int c0 = 2; c0 < 2 + b.nxy[2 * i]; c0 += sac::tile::TX) st.push_back({i, c0, c1});
+        for (int c0 = 2; c0 < 2 + b.nxy[2 * i]; c0 += sac::tile::TX) tiles.push_back({i, c0, c1});
+    }
   }
-  const Tile none = {active.empty() ? 0 : active[0], 2, 2};
-  if (tiles.empty()) tiles.push_back(none);
-  if (st.empty()) st.push_back(none);
-  Tile* dt[2] = {nullptr, nullptr};  // tiles, stiles
-  const std::vector<Tile>* ht[2] = {&tiles, &st};
-  hipError_t e = hipSuccess;
-  for (int k = 0; k < b.ndim && e == hipSuccess; k++) {
-    const size_t bytes = sizeof(Tile) * ht[k]->size();
-    e = hipMalloc((void**)&dt[k], bytes);
-    if (e == hipSuccess) e = hipMemcpy(dt[k], ht[k]->data(), bytes, hipMemcpyHostToDevice);
-  }
+  if (tiles.empty()) tiles.push_back({active.empty() ? 0 : active[0], 2, 2});
+  Tile* dt = nullptr;
+  hipError_t e = hipMalloc((void**)&dt, sizeof(Tile) * tiles.size());
+  if (e == hipSuccess)
+    e = hipMemcpy(dt, tiles.data(), sizeof(Tile) * tiles.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(b.d_active, active.data(), sizeof(int) * active.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
-    for (Tile* t : dt)
-      if (t) hipFree(t);
-    return bfail(SAC_E_HIP, "tile tables: %s", hipGetErrorString(e));
+    if (dt) hipFree(dt);
+    return bfail(SAC_E_HIP, "tile table: %s", hipGetErrorString(e));
   }
   // the graph's kernel nodes hold the tile tables freed below: destroy the
   // executable graph first (the stream is idle here), so no graph ever
@@ -553,18 +517,13 @@ int set_shape(Batch& b, Shape s, std::vector<int> active) {
   }
   b.graph_steps = 0;
   if (b.d_tiles) hipFree(b.d_tiles);
-  if (b.d_stiles) hipFree(b.d_stiles);
-  b.d_tiles = dt[0];
-  b.d_stiles = dt[1];
+  b.d_tiles = dt;
   b.ntiles = (int)tiles.size();
   b.shape = s;
   b.rows_fit = rows_fit;
   b.active = std::move(active);
   b.a.tiles = b.d_tiles;
   b.a.ntiles = b.ntiles;
-  b.a.tbx = s.tbx;
-  b.a.stiles = b.d_stiles;
-  b.a.nstiles = (int)st.size();
   b.a.active = b.d_active;
   b.a.nactive = (int)b.active.size();
   return 0;
@@ -595,7 +554,7 @@ void launch_tube_stage(Batch& b, dim3 gt, dim3 bt, int wct, int base, int out, d
 
 template <typename Off>
 void launch_patch_stage(Batch& b, int wct, int base, int out, double da, int last) {
-  const dim3 gs((unsigned)((b.a.nstiles + 7) / 8 * 8)), bs(sac::tile::NT);  // for xcd_block8
+  const dim3 gs((unsigned)((b.a.ntiles + 7) / 8 * 8)), bs(sac::tile::NT);  // for xcd_block8
   if (last)
     hipLaunchKernelGGL((kb_patch_stage<true, Off>), gs, bs, 0, b.stream, b.a, wct, base, out, da);
   else
@@ -637,11 +596,11 @@ void enqueue_step(Batch& b) {
 void enqueue_cmax(Batch& b, int slot) {
   const dim3 gn((b.ntubes + 255) / 256), bn(256);
   hipLaunchKernelGGL(kb_zero_red, gn, bn, 0, b.stream, b.a, slot);
-  const dim3 gt(b.ntiles), bt(b.shape.tb);
+  const dim3 gt(b.ntiles);
   if (b.ndim == 2)
-    hipLaunchKernelGGL((kb_cmax<2, 1>), gt, bt, 0, b.stream, b.a, slot);
+    hipLaunchKernelGGL(kb_cmax<2>, gt, dim3(sac::tile::NC), 0, b.stream, b.a, slot);
   else
-    hipLaunchKernelGGL((kb_cmax<1, 1>), gt, bt, 0, b.stream, b.a, slot);
+    hipLaunchKernelGGL(kb_cmax<1>, gt, dim3(b.shape.tb), 0, b.stream, b.a, slot);
 }
 
 // capture `steps` time steps (and the running-tube counter reset) in one graph
@@ -864,7 +823,7 @@ int sac_batch_init_nd(int ndim, int ntubes, const int* ncell, int nw, const doub
   a.dtmin = 1.0e-99;
   a.itmax = itmax;
   a.running = b->d_running;
-  if ((rc = set_shape(*b, ndim == 1 ? Shape{1, 128, 0} : Shape{1, 256, 64}, all))) return bail(rc);
+  if ((rc = set_shape(*b, ndim == 1 ? Shape{128, 0} : Shape{256, 64}, all))) return bail(rc);
   // initial getboundary (background and state) and cmax of W
   enqueue_ghost(*b, b->d_bg, NBG);
   enqueue_ghost(*b, b->d_reg[SAC_SLOT_W], NE);
@@ -896,7 +855,6 @@ int sac_batch_free(sac_batch_handle h) {
   hipFree(b->d_pitch);
   hipFree(b->d_dxo);
   hipFree(b->d_tiles);
-  hipFree(b->d_stiles);
   hipFree(b->d_active);
   hipFree(b->d_red);
   hipFree(b->d_visc);
@@ -961,7 +919,7 @@ int sac_batch_tune(sac_batch_handle h, int trial_steps, int* ck, int* tb, double
     if (int rc = restore_state(b, r0)) return rc;
   }
   if (int rc = set_shape(b, bs, b.active)) return rc;
-  if (ck) *ck = bs.ck;
+  if (ck) *ck = 1;  // cells per thread
   if (tb) *tb = bs.tb;
   if (ms_per_step) *ms_per_step = best;
   return 0;
@@ -981,8 +939,8 @@ int sac_batch_set_shape(sac_batch_handle h, int index) {
 int sac_batch_shape(sac_batch_handle h, int* ck, int* tbx, int* tby) {
   if (!h) return bfail(SAC_E_ARG, "null handle");
   const Batch& b = *(const Batch*)h;
-  if (ck) *ck = b.shape.ck;
-  if (tbx) *tbx = (b.ndim == 1) ? b.shape.tb * b.shape.ck : b.shape.tbx;
+  if (ck) *ck = 1;  // cells per thread
+  if (tbx) *tbx = (b.ndim == 1) ? b.shape.tb : b.shape.tbx;
   if (tby) *tby = (b.ndim == 1) ? 1 : b.shape.tb / b.shape.tbx;
   return 0;
 }

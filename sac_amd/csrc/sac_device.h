@@ -1129,14 +1129,6 @@ __device__ __forceinline__ void final_cells(const FinalArgs& a, const GridDesc& 
   update_cells<NDIM, NDIR, S, C, V, RK4L>(a, g, c, ic0, nv, R, redv);
 }
 
-// One mesh cell c of the grid g; the cmax values of the result go to redv.
-// RK4L: RK4's last stage (a.w1, a.w2 set; w3 is the stage input a.wct).
-template <int NDIM, int NDIR, typename S, typename C, bool RK4L>
-__device__ __forceinline__ void final_cell(const FinalArgs& a, const GridDesc& g, const int (&c)[3],
-                                           double (&redv)[2 * NDIM]) {
-  final_cells<NDIM, NDIR, S, C, 1, RK4L>(a, g, c, 1, redv);
-}
-
 // 1-D grids in FP64: a whole RK stage of the tile of LT cells from c0 on: the
 // x work (line1_tile), then gravity and the update of the thread's cell from
 // the rate in registers (1-D has no cross terms, so nothing waits for other

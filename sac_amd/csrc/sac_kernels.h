@@ -140,7 +140,5 @@ void launch_zero_u64(unsigned long long* p, int n, hipStream_t st);
 void launch_axpy4(int prec, long long n, void* out, const void* a0, double c0, const void* a1,
                   double c1, const void* a2, double c2, const void* a3, double c3,
                   hipStream_t st);
-void launch_to_float(long long n, float* out, const double* in, hipStream_t st);
-void launch_to_double(long long n, double* out, const float* in, hipStream_t st);
 
 }  // namespace sac

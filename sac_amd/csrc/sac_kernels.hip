@@ -486,13 +486,6 @@ __global__ void k_axpy4(long long n, S* __restrict__ out, const S* a0, double c0
   out[i] = (S)s;
 }
 
-// type conversion of n elements (FP64 staging <-> FP32 registers)
-template <typename D, typename S>
-__global__ void k_convert(long long n, D* __restrict__ out, const S* __restrict__ in) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (D)in[i];
-}
-
 // ---------------------------------------------------------------------
 // launchers
 
@@ -784,18 +777,6 @@ void launch_axpy4(int prec, long long n, void* out, const void* a0, double c0, c
     hipLaunchKernelGGL(k_axpy4<double>, grid, dim3(bs), 0, st, n, (double*)out,
                        (const double*)a0, c0, (const double*)a1, c1, (const double*)a2, c2,
                        (const double*)a3, c3);
-}
-
-void launch_to_float(long long n, float* out, const double* in, hipStream_t st) {
-  const int bs = 256;
-  hipLaunchKernelGGL((k_convert<float, double>), dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0,
-                     st, n, out, in);
-}
-
-void launch_to_double(long long n, double* out, const float* in, hipStream_t st) {
-  const int bs = 256;
-  hipLaunchKernelGGL((k_convert<double, float>), dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0,
-                     st, n, out, in);
 }
 
 }  // namespace sac
