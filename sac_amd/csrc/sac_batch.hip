@@ -157,7 +157,7 @@ __device__ __forceinline__ void clear_red_w(const Args& a, int tube, bool first,
 
 // Patches: a whole RK stage of one 16 x 16 tile (stage_tile, also used by 2-D
 // grids), with the 'cont' ghosts of its cells.  512 patches
-// of 32-160 cells (4.8 M): 0.706 ms a stage, RK4's last 0.769; the two line
+// of 32-160 cells (4.8 M): 0.65 ms a stage, RK4's last 0.72; the two line
 // kernels and the update before took 0.996 and 1.155.
 template <bool RK4L, typename Off>
 __global__ void __launch_bounds__(tile::NT, 4) kb_patch_stage(Args a, int wct, int base, int out,

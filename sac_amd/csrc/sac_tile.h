@@ -27,7 +27,7 @@
 // wavefronts halve the chain and give four wavefronts per SIMD instead of
 // two.  A 2-D stage of 501 x 299 cells was an x and a y line kernel and an
 // update, 19.8 + 16.3 + 15.5 us; here 21.3.  512 patches (4.8 M cells): 0.996
-// ms before, 0.677 now.  Reading the cell's background, c_tot and dx before
+// ms before, 0.65 now.  Reading the cell's background, c_tot and dx before
 // the points, and the base register while the axes are handed over, is 15 %
 // of that.  In 3-D a tile is bound by both its VALU issue (2350 instructions
 // per 64 cells, 60 % of the time at the 2.07 GHz the card runs FP64 work at)

@@ -1,6 +1,7 @@
 """One RK4 step of 1-D grids at sizes around the tiles of the one-launch
-stage (64 cells up to 4096 cells, 256 above), against the oracle: a step's
-rounding differences stay at a few 1e-16 per variable, the bar is 1e-12."""
+stage (64 cells up to 32768 cells; test_stage1_long.py has the grids on tiles
+of 256), against the oracle: a step's rounding differences stay at a few 1e-16
+per variable, the bar is 1e-12."""
 import pytest
 
 from sac_amd import problems
