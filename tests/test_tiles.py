@@ -1,8 +1,9 @@
 """Stages on 16 x 16 tiles (2-D grids in one launch): one RK4 step at extents
 around the tile edges (tiles start at the first mesh cell along both axes;
 test_tile_edges.py has the extents that end one along x), every boundary type,
-with Powell's sources and resistivity, against the oracle in FP64 at 1e-12 per variable and at FP32 resolution (1e-5, as in the other tests of the
-mixed form), and against the schedule of one line pass per axis."""
+with Powell's sources and resistivity, against the oracle in FP64 at 1e-12 per
+variable and at FP32 resolution (1e-5, as in the other tests of the mixed
+form), and against the schedule of one line pass per axis."""
 import numpy as np
 import pytest
 
